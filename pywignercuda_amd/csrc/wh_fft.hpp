@@ -349,6 +349,8 @@ struct WaveSync {
 // the first pass are multiples of R, so padr(i + R m) = padr(i) + (R+1) m, and
 // the first pass (radix R, span 1) writes the R consecutive indices of one
 // aligned group of R, so padr(R b + q) = padr(R b) + q.
+template <int BIT, typename T>
+__device__ __forceinline__ void lane_swap(cplx<T>& a, cplx<T>& b);
 template <typename T, int N, int R, int P>
 struct PassIO {
   static constexpr int NP = num_passes(N, R);
@@ -412,12 +414,90 @@ struct PassIO {
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = o[j];
   }
+  // the last pass with its inputs exchanged between lanes instead of through LDS (swaps_lanes):
+  // register q = r mm + j then holds input j of butterfly t + mm TT
+  template <int DIR, class Tw>
+  __device__ __forceinline__ static void swap(cplx<T> (&v)[R], int tl, const Tw& tw) {
+    constexpr int r = pass_radix(N, R, P), nb = R / r;
+    constexpr int top = ilog2(TT) - 1;  // lane bit of the highest bit of j
+    static_for<0, ilog2(r)>([&](auto B) {
+      constexpr int bit = decltype(B)::value;  // bit of j
+      static_for<0, R>([&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+        if constexpr (!((q >> bit) & 1)) lane_swap<top - (ilog2(r) - 1 - bit)>(v[q], v[q | (1 << bit)]);
+      });
+    });
+    cplx<T> o[R];
+    static_for<0, nb>([&](auto MM) {
+      constexpr int mm = decltype(MM)::value;
+      cplx<T> x[r];
+#pragma unroll
+      for (int j = 0; j < r; ++j) x[j] = v[mm * r + j];
+      static_for<1, r>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        x[j] = tw.template mul<DIR>(x[j], TwSlots<N, R>::off(P) + j - 1, (j * tl) & (N - 1));
+        x[j] = rot<DIR, (j * mm) % R, R>(x[j]);
+      });
+      dft<DIR, r>(x);
+#pragma unroll
+      for (int q = 0; q < r; ++q) o[mm + q * nb] = x[q];
+    });
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = o[j];
+  }
 };
+
+// Exchange of a lane-index bit with a register-index bit: lane halves (BIT 5) or odd and even
+// rows of 16 lanes (BIT 4) of the registers a (bit clear) and b (bit set).  Afterwards a holds
+// what was in the lanes with the bit clear (of a, then of b), b what was in the others.
+template <int BIT>
+__device__ __forceinline__ void lane_swap(unsigned& a, unsigned& b) {
+  static_assert(BIT == 4 || BIT == 5, "v_permlane16_swap_b32, v_permlane32_swap_b32");
+  if constexpr (BIT == 5) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  }
+}
+template <int BIT, typename T>
+__device__ __forceinline__ void lane_swap(cplx<T>& a, cplx<T>& b) {
+  constexpr int W = sizeof(cplx<T>) / 4;
+  struct Words {
+    unsigned w[W];
+  };
+  Words x = __builtin_bit_cast(Words, a), y = __builtin_bit_cast(Words, b);
+#pragma unroll
+  for (int i = 0; i < W; ++i) lane_swap<BIT>(x.w[i], y.w[i]);
+  a = __builtin_bit_cast(cplx<T>, x);
+  b = __builtin_bit_cast(cplx<T>, y);
+}
+
+// The exchange before the last pass can stay in registers: lane t of a team holds the outputs q
+// of butterfly t, whose top log2(r) index bits are the inputs j of the last pass, and the last
+// pass needs lane bits and the low bits of q exchanged -- one swap instruction per register pair
+// and bit where those are lane bits 4 and 5 (r = 4 on 64 lanes, r = 2 on 64 or 32 lanes).
+// The LDS pipe of a CU serves its four SIMDs: an exchange of four radix-16 FP64 teams at N = 1024
+// keeps it for about 1000 cycles while the FP64 units wait; the 64 swaps of a lane run on each
+// SIMD by itself.  Measured (1024^2): damped FP64 step 52.7 -> 51.0 us, 32 FP64 grids 586 -> 565 us
+// per step, 64 uneven complex64-state grids 275 -> 267 us.  Other lane bits have no swap
+// instruction (moves through DPP need two to four per pair): those passes stay in LDS.
+template <int N, int R, int P, class Sync>
+constexpr bool swaps_lanes() {
+  constexpr int r = pass_radix(N, R, P), TT = N / R;
+  return std::is_same_v<Sync, WaveSync> && P == num_passes(N, R) - 1 && P >= 2 && r <= R && TT / r >= 16 &&
+         (TT == 64 || TT == 32);
+}
 
 template <typename T, int N, int R, int DIR, int P, class Sync, class Lds, class Tw>
 struct TeamPass {
   __device__ __forceinline__ static void run(cplx<T> (&v)[R], int t, Lds lds, const Tw& tw) {
-    if constexpr (P < num_passes(N, R)) {
+    if constexpr (P < num_passes(N, R) && swaps_lanes<N, R, P, Sync>()) {
+      PassIO<T, N, R, P>::template swap<DIR>(v, opaque_v(t), tw);
+    } else if constexpr (P < num_passes(N, R)) {
       const int tl = opaque_v(t);
       Sync::sync();  // every lane has read the previous pass's inputs
       PassIO<T, N, R, P>::write(v, tl, lds);
