@@ -19,7 +19,7 @@
 namespace wh {
 
 template <typename T, int N, int R, int BLOCK>
-__device__ __forceinline__ void adj_psweep_body(const SweepArgs& a, const Member& m, int tile, cplx<T>* lds) {
+__device__ __forceinline__ void adj_psweep_body(const SweepArgs& a, CMember& m, int tile, cplx<T>* lds) {
   constexpr int TT = N / R, C = BLOCK / TT;
   const int tid = threadIdx.x;
   const int c = tid % C, t = tid / C;
@@ -102,8 +102,8 @@ __device__ __forceinline__ void adj_psweep_body(const SweepArgs& a, const Member
 template <typename T, int R, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) adj_psweep_kernel(SweepArgs a) {
   __shared__ cplx<T> lds[lds_elems<BLOCK, R>()];
-  const unsigned w = a.work[blockIdx.x];
-  const Member& m = a.members[w >> 16];
+  const unsigned w = cmem(a.work)[blockIdx.x];
+  CMember& m = member_at(a.members, w >> 16);
   const int tile = int(w & 0xffffu);
 #define BODY(n) adj_psweep_body<T, n, R, BLOCK>(a, m, tile, lds)
   WH_DISPATCH(m.P, BODY)
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(BLOCK) adj_psweep_kernel(SweepArgs a) {
 // grad[k] = scale * sum_x gcols[x][k]   (one block per member; member 0 for single plans)
 __global__ void __launch_bounds__(256) grad_reduce_kernel(const Member* members, double* grad, double scale) {
   __shared__ double red[kMaxDeg + 1][256];
-  const Member& m = members[blockIdx.x];
+  CMember& m = member_at(members, blockIdx.x);
   double acc[kMaxDeg + 1];
 #pragma unroll
   for (int k = 0; k <= kMaxDeg; ++k) acc[k] = 0.0;

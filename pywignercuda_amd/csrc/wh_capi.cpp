@@ -568,6 +568,9 @@ int build_work_lists(wh_ensemble* e) {
   for (const auto& v : {&wx, &wp, &wpcl, &wc, &ws, &wg})
     for (unsigned w : *v)
       if ((w & 0xffffu) == 0xffffu) return fail(WH_INVALID_SIZE, "a member has more than 65535 tiles");
+  // the members' record items end the x list: the row tiles keep their XCDs (block q runs on XCD
+  // q % 8; a list shifted by one cost the ODM step 3%, whose row sweeps follow each other)
+  for (int i = 0; i < e->n; ++i) wx.push_back((unsigned(i) << 16) | unsigned(wh::kRecordTile));
   WH_TRY(e->work_x.upload(wx));
   WH_TRY(e->work_p.upload(wp));
   if (e->cl()) WH_TRY(e->work_pcl.upload(wpcl));
@@ -622,7 +625,12 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
     } else {
       WH_TRY(b->pot.upload(md.pot_coef, size_t(md.pot_rows) * (WH_MAX_DEG + 1) * sizeof(double)));
     }
-    WH_TRY(upload_opt(b->theta_decay, md.theta_decay, P));
+    if (desc->damping == 1 && !md.theta_decay) {  // the friction sweep reads the table unconditionally
+      const std::vector<double> ones(P, 1.0);
+      WH_TRY(b->theta_decay.upload(ones.data(), P * sizeof(double)));
+    } else {
+      WH_TRY(upload_opt(b->theta_decay, md.theta_decay, P));
+    }
     WH_TRY(upload_opt(b->lambda_decay, md.lambda_decay, X));
     WH_TRY(upload_opt(b->x_mask, md.x_mask, X));
     WH_TRY(upload_opt(b->sigma_p, md.sigma_p, P));
@@ -781,6 +789,7 @@ int xsweep(wh_ensemble* e, int flags, hipStream_t s) {
     return fail(WH_INTERNAL_ERROR, "x work list cut for another variant");
   wh::SweepArgs a = sweep_args(e, flags, 1.0, 0);
   a.work = e->work_x.buf.as<unsigned>();
+  a.ntiles = e->n == 1 ? e->work_x.n - 1 : 0;  // the record item is the last
   WH_LAUNCH(e->d.precision == WH_C128      ? wh::launch_xsweep_f64(e->xvar, a, e->work_x.n, s)
             : e->d.precision == WH_C64_WIDE ? wh::launch_xsweep_f32w(e->xvar, a, e->work_x.n, s)
                                       : wh::launch_xsweep_f32(e->xvar, a, e->work_x.n, s),
@@ -800,6 +809,7 @@ int psweep(wh_ensemble* e, int flags, double frac, int step_add, hipStream_t s) 
   if (!same_variant(launched, cl ? e->built_pcl : e->built_p))
     return fail(WH_INTERNAL_ERROR, "p work list cut for another variant");
   a.work = wl.buf.as<unsigned>();
+  a.ntiles = e->n == 1 ? wl.n : 0;
   if (e->expr) {
     // expression-program members: their [P][X] tables at the time index this sweep reads
     // (and the next one for the merged Strang half step)

@@ -46,6 +46,7 @@ enum SweepFlags {
 };
 
 constexpr int kTileObs = 12;  // observable partials per tile
+constexpr int kRecordTile = 0xffff;  // x work item that forms a member's record (kTileScale), no row tile
 
 // One ensemble member, resident in device memory.
 struct Member {
@@ -95,9 +96,21 @@ struct Member {
   int pad1, pad2;
 };
 
+// The member table as kernels read it: constant memory for the whole kernel (the bind kernels and
+// uploads that write it are launches of their own), so that every field is a scalar load that the
+// compiler may place anywhere.  Through a generic reference the fields read behind the first
+// branch became vector loads, one full memory latency each: four of them in front of a p sweep's
+// loads at 512^2.
+using CMember = const __attribute__((address_space(4))) Member;
+__device__ __forceinline__ CMember& member_at(const Member* members, unsigned i) {
+  return ((CMember*)members)[i];
+}
+
 struct SweepArgs {
   const Member* members;
   const unsigned* work;  // (member << 16) | tile, one per block
+  int ntiles;            // > 0: a plan of one member with that many tiles, the work item follows
+                         // from the block index (one dependent load less in front of the sweep)
   int* step;             // device step counter (time index)
   int step_add;
   int flags;

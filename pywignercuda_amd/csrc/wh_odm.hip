@@ -43,7 +43,7 @@ __device__ __forceinline__ cplx<U> nar(cplx<double> v) {
 // weight, sgn: the channel's weight and sign (GPU_Wigner2D_ODM2 runs two channels,
 // (weightLindbland1, +1) then (weightLindbland2, -1), GPU_Wigner2D_FFT.py:2173-2181)
 template <typename S, typename T, int N, int R, int BLOCK>
-__device__ __forceinline__ void odm_x_body(const Member& m, int tile, cplx<T>* lds, double weight, double sgn) {
+__device__ __forceinline__ void odm_x_body(CMember& m, int tile, cplx<T>* lds, double weight, double sgn) {
   constexpr int TT = N / R, ROWS = BLOCK / TT;
   constexpr int LSZ = Padded<N, R>::size;
   const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
@@ -109,7 +109,7 @@ __device__ __forceinline__ void odm_x_body(const Member& m, int tile, cplx<T>* l
 }
 
 template <typename S, typename T, int N, int R, int BLOCK>
-__device__ __forceinline__ void odm_p_body(const Member& m, int tile, cplx<T>* lds, double weight, double sgn) {
+__device__ __forceinline__ void odm_p_body(CMember& m, int tile, cplx<T>* lds, double weight, double sgn) {
   constexpr int TT = N / R;
   constexpr int C = BLOCK / TT;
   const int tid = threadIdx.x;
@@ -146,7 +146,7 @@ __device__ __forceinline__ void odm_p_body(const Member& m, int tile, cplx<T>* l
 }
 
 template <typename S, typename T, int N, int R, int BLOCK>
-__device__ __forceinline__ void odm_back_body(const Member& m, int tile, cplx<T>* lds) {
+__device__ __forceinline__ void odm_back_body(CMember& m, int tile, cplx<T>* lds) {
   constexpr int TT = N / R, ROWS = BLOCK / TT;
   constexpr int LSZ = Padded<N, R>::size;
   const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
@@ -171,8 +171,8 @@ template <typename S, typename T, int KIND>
 __global__ void __launch_bounds__(kOdmBlock) odm_kernel(const Member* members, const unsigned* work, double weight,
                                                         double sgn) {
   __shared__ cplx<T> lds[lds_elems<kOdmBlock, kOdmR>()];
-  const unsigned w = work[blockIdx.x];
-  const Member& m = members[w >> 16];
+  const unsigned w = cmem(work)[blockIdx.x];
+  CMember& m = member_at(members, w >> 16);
   const int tile = int(w & 0xffffu);
   constexpr int R = kOdmR, BLOCK = kOdmBlock;
   if constexpr (KIND == 0) {

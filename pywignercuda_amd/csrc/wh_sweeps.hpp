@@ -49,9 +49,11 @@ struct BoppOdd {
 template <class CP>
 __device__ __forceinline__ BoppOdd bopp_odd(CP c, int deg, double x, double f) {
   static_assert(kMaxDeg == 8, "odd Taylor terms u, u^3, u^5, u^7");
-  double d[kMaxDeg + 1];
+  double d[kMaxDeg + 1];  // (every row has kMaxDeg + 1 entries: loaded unconditionally, in one go)
 #pragma unroll
-  for (int n = 0; n <= kMaxDeg; ++n) d[n] = n <= deg ? c[n] : 0.0;
+  for (int n = 0; n <= kMaxDeg; ++n) d[n] = c[n];
+#pragma unroll
+  for (int n = 0; n <= kMaxDeg; ++n) d[n] = n <= deg ? d[n] : 0.0;
 #pragma unroll
   for (int i = 0; i < kMaxDeg; ++i) {
 #pragma unroll
@@ -142,6 +144,20 @@ constexpr bool size_ok() {
   return N >= R * 4 && N / R <= BLOCK && BLOCK / (N / R) <= 64;
 }
 
+// The (member << 16) | tile item of this block.  A plan of one member computes it: x tiles in
+// block order and the record item last; p tiles with consecutive tiles on one XCD (as the work
+// lists are cut on the host).
+__device__ __forceinline__ unsigned x_item(const SweepArgs& a) {
+  if (a.ntiles <= 0) return cmem(a.work)[blockIdx.x];
+  return int(blockIdx.x) < a.ntiles ? blockIdx.x : unsigned(kRecordTile);
+}
+__device__ __forceinline__ unsigned p_item(const SweepArgs& a) {
+  if (a.ntiles <= 0) return cmem(a.work)[blockIdx.x];
+  const unsigned q = blockIdx.x, nt = unsigned(a.ntiles);
+  return nt % 8 == 0 ? (q % 8) * (nt / 8) + q / 8 : q;
+}
+__device__ __forceinline__ bool first_member(const SweepArgs& a, CMember& m) { return &m == &member_at(a.members, 0); }
+
 // ------------------------------------------------------------------ observables
 // Sum over the 64 lanes of a wave (fixed xor tree: deterministic).
 __device__ __forceinline__ double wave_sum(double v) {
@@ -158,17 +174,17 @@ __device__ __forceinline__ double dpp_f64(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, int(unsigned(b >> 32)), CTRL, ROWMASK, 0xF, false);
   return __longlong_as_double((static_cast<unsigned long long>(unsigned(hi)) << 32) | unsigned(lo));
 }
-// Sum over aligned groups of G lanes (G = 8, 16, 32 or 64) by VALU lane moves (no LDS
+// Sum over aligned groups of G lanes (G = 1, 2, 4 .. 64) by VALU lane moves (no LDS
 // traffic, fixed order: deterministic); the last lane of each group holds the sum.
 //   quad_perm [1,0,3,2], [2,3,0,1]: quad sums;  row_half_mirror: sums of 8;  row_mirror:
 //   sums of 16;  row_bcast15 into rows 1, 3: sums of 32 there;  row_bcast31 into rows 2,
 //   3: the sum of 64 in row 3.
 template <int G>
 __device__ __forceinline__ double group_sum(double v) {
-  static_assert(G == 8 || G == 16 || G == 32 || G == 64, "group of 8..64 lanes");
-  v += dpp_f64<0xB1>(v);
-  v += dpp_f64<0x4E>(v);
-  v += dpp_f64<0x141>(v);
+  static_assert(G >= 1 && G <= 64 && (G & (G - 1)) == 0, "group of 1..64 lanes");
+  if constexpr (G >= 2) v += dpp_f64<0xB1>(v);
+  if constexpr (G >= 4) v += dpp_f64<0x4E>(v);
+  if constexpr (G >= 8) v += dpp_f64<0x141>(v);
   if constexpr (G >= 16) v += dpp_f64<0x140>(v);
   if constexpr (G >= 32) v += dpp_f64<0x142, 0xA>(v);
   if constexpr (G >= 64) v += dpp_f64<0x143, 0xC>(v);
@@ -178,9 +194,15 @@ __device__ __forceinline__ double group_sum(double v) {
 // Observable terms of one column from its sums s = (Re S0, Im S0, sum p W, sum p^2 W,
 // sum min(W, 0)): the integrands of <x>, <x^2>, <p>, <p^2>, <xp>, <dV/dx>, <p dV/dx>,
 // <x dV/dx>, energy, negative area (the per-step record of GPU_Wigner2D_FFT.py:1856-1876).
-__device__ __forceinline__ void column_terms(const Member& m, int col, const double (&s)[kNCol],
+struct ColumnHost {
+  double x, dv, v0;
+};
+__device__ __forceinline__ ColumnHost column_host(CMember& m, int col) {
+  return {gmem(m.x_host)[col], gmem(m.dv_host)[col], gmem(m.v0_host)[col]};
+}
+__device__ __forceinline__ void column_terms(CMember& m, ColumnHost h, const double (&s)[kNCol],
                                              double (&o)[12]) {
-  const double x = gmem(m.x_host)[col], dv = gmem(m.dv_host)[col], v0 = gmem(m.v0_host)[col];
+  const double x = h.x, dv = h.dv, v0 = h.v0;
   o[0] = s[0];
   o[1] = s[1];
   o[2] = x * s[0];
@@ -197,7 +219,7 @@ __device__ __forceinline__ void column_terms(const Member& m, int col, const dou
 
 // Record row, pending factor and step counter from the 12 observable sums of a member
 // (the normalised state is W / n, n = dXdP sum W; observables Re(dXdP sum W A / n)).
-__device__ __forceinline__ void write_record(const Member& m, const double (&r)[12], int renorm, int record,
+__device__ __forceinline__ void write_record(CMember& m, const double (&r)[12], int renorm, int record,
                                              int step) {
   const double nr = m.dxdp * r[0], ni = m.dxdp * r[1];
   double f = 1.0, sr = 1.0, si = 0.0;
@@ -229,82 +251,115 @@ __device__ __forceinline__ void write_record(const Member& m, const double (&r)[
 }
 
 // kTilePart epilogue of a p-sweep tile: csum holds the kNCol sums of each of the tile's
-// C columns (LDS, visible to every thread: written before a barrier); thread k < 12 forms
-// observable term k of each column and sums them in column order into
-// m.tilepart[k * X + tile].  Tile 0 of member 0 copies the step index to rec_step.
-template <int BLOCK, int C>
-__device__ __forceinline__ void write_tile_partial(const SweepArgs& a, const Member& m, int tile,
-                                                   const double* csum, int step) {
+// C columns (LDS, visible to every thread: written before a barrier); lane c < C forms the 12
+// observable terms of column c (host values h, loaded at the kernel's start) and the lanes' sum
+// goes to m.tilepart[k * X + tile].  Tile 0 of member 0 copies the step index to rec_step.
+// (One lane per term, each forming every column's terms with the loads of their host values in
+// the loop, kept a 128-column tile row of 16 columns busy for 5300 cycles of its 34600.)
+template <int C>
+__device__ __forceinline__ void write_tile_partial(const SweepArgs& a, CMember& m, int tile,
+                                                   const double* csum, ColumnHost h, int step) {
+  static_assert(C <= 64, "one wave");
   const int tid = threadIdx.x;
-  if (tid < 12) {
-    double t = 0.0;
-    for (int c = 0; c < C; ++c) {
-      double s[kNCol], o[12];
+  if (tid < 64) {
+    double s[kNCol], o[12];
+    const int c = tid % C;
 #pragma unroll
-      for (int k = 0; k < kNCol; ++k) s[k] = csum[c * kNCol + k];
-      column_terms(m, tile * C + c, s, o);
+    for (int k = 0; k < kNCol; ++k) s[k] = csum[c * kNCol + k];
+    column_terms(m, h, s, o);
 #pragma unroll
-      for (int k = 0; k < 12; ++k)
-        if (k == tid) t += o[k];
+    for (int k = 0; k < 12; ++k) o[k] = group_sum<C>(o[k]);
+    if (tid == C - 1) {
+#pragma unroll
+      for (int k = 0; k < 12; ++k) gmem(m.tilepart)[size_t(k) * m.X + tile] = o[k];
     }
-    gmem(m.tilepart)[size_t(tid) * m.X + tile] = t;
-  } else if (tid == 12 && tile == 0 && &m == a.members) {
-    *gmem(a.rec_step) = step;  // the step index this sweep read at its start
+    if (tid == 0 && tile == 0 && first_member(a, m)) *gmem(a.rec_step) = step;  // the step index this sweep read at its start
   }
 }
 
-// kTileScale prologue of an x-sweep block: sums the tile partials of the member's last
-// p sweep (every block in the same order, so all blocks derive the same factor) and
-// returns the pending factor 1 / norm (or 1).  Tile 0 also forms all 12 sums, writes
-// the record row and the factor; tile 0 of member 0 advances the step index.
-// Contains __syncthreads(); red: kTileRedBytes of LDS outside the transform arrays.
+// kTileScale: the x sweep sums the tile partials of the member's last p sweep (every block in
+// the same order, so all blocks derive the same factor) into the pending factor 1 / norm (or 1).
+// The loads are issued before the state's and the sum is taken when the first transform is done,
+// where the factor is needed; the record row is an item of its own.  With the sum in front of the
+// transform and the record in tile 0 every block waited for the partials' latency, the wave sums
+// and a block barrier (5400 of the 11200 cycles of a 128^2 x sweep): 9.5 -> 4.9 us at 128^2,
+// 16.3 -> 15.9 us at 1024^2.
+// red: kTileRedBytes of LDS outside the transform arrays.
 constexpr int kTileRedBytes = 16 * 12 * 8;
+struct TilePartials {
+  double re, im;
+};
+__device__ __forceinline__ int tile_count(const SweepArgs& a, CMember& m) {
+  return m.X * (m.P / a.pt_R) / a.pt_block;  // X over the columns per p-sweep tile
+}
 template <int BLOCK>
-__device__ __forceinline__ cplx<double> tile_scale(const SweepArgs& a, const Member& m, int tile, double* red) {
+__device__ __forceinline__ TilePartials tile_partials(const SweepArgs& a, CMember& m) {
+  const int ntiles = tile_count(a, m);
+  TilePartials r{0.0, 0.0};
+  for (int i = threadIdx.x; i < ntiles; i += BLOCK) {
+    r.re += gmem(m.tilepart)[i];
+    r.im += gmem(m.tilepart)[size_t(m.X) + i];
+  }
+  return r;
+}
+// Contains __syncthreads().
+template <int BLOCK>
+__device__ __forceinline__ cplx<double> tile_scale(const SweepArgs& a, CMember& m, TilePartials r, double* red) {
+  constexpr int kWaves = BLOCK / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  r.re = group_sum<64>(r.re);
+  r.im = group_sum<64>(r.im);
+  if (lane == 63) {
+    red[wave * 2] = r.re;
+    red[wave * 2 + 1] = r.im;
+  }
+  __syncthreads();
+  r = {0.0, 0.0};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    r.re += red[w * 2];
+    r.im += red[w * 2 + 1];
+  }
+  if (!a.fin_renorm) return {1.0, 0.0};
+  const double nr = m.dxdp * r.re, ni = m.dxdp * r.im;
+  const double m2 = nr * nr + ni * ni;
+  return {nr / m2, -ni / m2};
+}
+
+// The record item of a member (one block of a kTileScale launch, beside the row tiles so that no
+// row waits for it): all 12 sums, the record row and the factor; that of member 0 advances the
+// step index.
+template <int BLOCK>
+__device__ __forceinline__ void record_item(const SweepArgs& a, CMember& m, double* red) {
   constexpr int kWaves = BLOCK / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int pc = a.pt_block / (m.P / a.pt_R);  // columns per p-sweep tile
-  const int ntiles = m.X / pc;
-  const bool rec = tile == 0;
-  const int nk = rec ? 12 : 2;
-  const int rstep = rec ? *gmem(a.rec_step) : 0;  // issued with the partial loads
+  const int ntiles = tile_count(a, m);
+  const int rstep = *cmem(a.rec_step);  // issued with the partial loads
   double r[12];
 #pragma unroll
   for (int k = 0; k < 12; ++k) r[k] = 0.0;
   for (int i = tid; i < ntiles; i += BLOCK) {
 #pragma unroll
-    for (int k = 0; k < 12; ++k)
-      if (k < nk) r[k] += gmem(m.tilepart)[size_t(k) * m.X + i];
+    for (int k = 0; k < 12; ++k) r[k] += gmem(m.tilepart)[size_t(k) * m.X + i];
   }
 #pragma unroll
-  for (int k = 0; k < 12; ++k)
-    if (k < nk) r[k] = group_sum<64>(r[k]);
+  for (int k = 0; k < 12; ++k) r[k] = group_sum<64>(r[k]);
   if (lane == 63) {
 #pragma unroll
-    for (int k = 0; k < 12; ++k)
-      if (k < nk) red[wave * 12 + k] = r[k];
+    for (int k = 0; k < 12; ++k) red[wave * 12 + k] = r[k];
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < 12; ++k) {
-    if (k < nk) {
-      double t = 0.0;
+    double t = 0.0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) t += red[w * 12 + k];
-      r[k] = t;
-    }
+    for (int w = 0; w < kWaves; ++w) t += red[w * 12 + k];
+    r[k] = t;
   }
-  const double nr = m.dxdp * r[0], ni = m.dxdp * r[1];
-  cplx<double> f{1.0, 0.0};
-  if (a.fin_renorm) {
-    const double m2 = nr * nr + ni * ni;
-    f = {nr / m2, -ni / m2};
-  }
-  if (rec && tid == 0) {
+  if (tid == 0) {
     write_record(m, r, a.fin_renorm, a.fin_record, rstep);
-    if (&m == a.members) *gmem(a.step) = rstep + 1;
+    if (first_member(a, m)) *gmem(a.step) = rstep + 1;
   }
-  return f;
 }
 
 // ------------------------------------------------------------------ x sweep
@@ -313,7 +368,7 @@ __device__ __forceinline__ cplx<double> tile_scale(const SweepArgs& a, const Mem
 // js = j (j < R/2) or j - R; computed as E_t * Z^js, E_t = exp(-i a t),
 // Z = exp(-i a TT): two sincos per lane instead of R.
 template <typename S, typename T, int N, int R, int BLOCK, bool TP, typename E>
-__device__ __forceinline__ void xsweep_body(const SweepArgs& a, const Member& m, int tile,
+__device__ __forceinline__ void xsweep_body(const SweepArgs& a, CMember& m, int tile,
                                             cplx<E>* lds) {
   constexpr int TT = N / R, ROWS = BLOCK / TT;
   constexpr int LSZ = Padded<N, R>::size;
@@ -332,6 +387,14 @@ __device__ __forceinline__ void xsweep_body(const SweepArgs& a, const Member& m,
   constexpr bool kWave = TT <= 64;
   using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
 
+  const bool tiles = (a.flags & kTileScale) != 0;
+  TilePartials part{0.0, 0.0};
+  cplx<double> g{1.0 / N, 0.0};
+  if (tiles) {
+    part = tile_partials<BLOCK>(a, m);
+  } else if (a.flags & kScaleOnLoad) {
+    g = {cmem(m.scale)[0] * (1.0 / N), cmem(m.scale)[1] * (1.0 / N)};
+  }
   cplx<T> v[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload(at_off(W, roff + unsigned(j) * kJ)));
@@ -344,23 +407,25 @@ __device__ __forceinline__ void xsweep_body(const SweepArgs& a, const Member& m,
       return TwMem<T>{tw};
     }
   }();
-  // The pending factor and the 1/N of the inverse transform ride on the kinetic
-  // multiplier (the transforms are linear): one complex product per lane instead of 2R.
-  cplx<double> g{1.0 / N, 0.0};
-  if (a.flags & kTileScale) {
-    const cplx<double> f = tile_scale<BLOCK>(a, m, tile, reinterpret_cast<double*>(lds + lds_elems<BLOCK, R>()));
-    g = {f.x * (1.0 / N), f.y * (1.0 / N)};
-  } else if (a.flags & kScaleOnLoad) {
-    g = {cmem(m.scale)[0] * (1.0 / N), cmem(m.scale)[1] * (1.0 / N)};
+  // the two phase factors of the linear form, evaluated while the loads are in flight
+  const double p = m.dp * double(fidx(row, m.P));
+  const double sgn = (a.flags & kConj) ? -1.0 : 1.0;  // adjoint: conj(r e^{-i phi}) = r e^{+i phi}
+  cplx<double> Et{1.0, 0.0}, Z1{1.0, 0.0};
+  if (a.kin_linear) {
+    const double ak = sgn * a.dt * m.dlambda * (a.k_c0 + a.k_c1 * p);
+    Et = expmi(1.0, ak * double(t));
+    Z1 = expmi(1.0, ak * double(TT));
   }
   team_fft<T, N, R, -1, LdsRow<E>, Sync>(v, t, view, twsrc);
 
-  const double p = m.dp * double(fidx(row, m.P));
-  const double sgn = (a.flags & kConj) ? -1.0 : 1.0;  // adjoint: conj(r e^{-i phi}) = r e^{+i phi}
+  // The pending factor and the 1/N of the inverse transform ride on the kinetic
+  // multiplier (the transforms are linear): one complex product per lane instead of 2R.
+  if (tiles) {
+    const cplx<double> f = tile_scale<BLOCK>(a, m, part, reinterpret_cast<double*>(lds + lds_elems<BLOCK, R>()));
+    g = {f.x * (1.0 / N), f.y * (1.0 / N)};
+  }
   if (a.kin_linear) {
-    const double ak = sgn * a.dt * m.dlambda * (a.k_c0 + a.k_c1 * p);
-    const cplx<double> Et = cmul(expmi(1.0, ak * double(t)), g);
-    const cplx<double> Z1 = expmi(1.0, ak * double(TT));
+    Et = cmul(Et, g);
     cplx<double> Zp[R / 2 + 1];  // Z^0 .. Z^(R/2)
     Zp[0] = {1.0, 0.0};
     Zp[1] = Z1;
@@ -421,7 +486,7 @@ struct PSweep {
   // tab: which [P][X] table a member with an expression program reads (0: time index `step`,
   // 1: `step` + 1, the merged Strang half step; expr_table_kernel fills them before the sweep)
   __device__ __forceinline__ static void potential(cplx<T> (&v)[R], const SweepArgs& a,
-                                                   const Member& m, int t_in, int col_in, int step,
+                                                   CMember& m, int t_in, int col_in, int step,
                                                    double scale, int tab) {
     // opaque lane indices: recomputing theta and x -/+ hbar theta/2 per call is cheaper
     // than keeping them live across the transforms between two calls
@@ -478,22 +543,87 @@ struct PSweep {
         v[j] = apply(v[j], expmi(mask, phi));
       }
     }
-    if (m.theta_decay) {
+  }
+
+  // The same multipliers evaluated apart from their use: they do not depend on the state, so the
+  // sweep evaluates them while its loads are in flight (everything but a table and a
+  // Gross-Pitaevskii grid together).  Vector loads return in order, so the values that they are
+  // made of are loaded before the state: the mask and V's table or the grid G.
+  struct MulLoads {
+    double mask, tab[R];
+  };
+  __device__ __forceinline__ static bool early(const SweepArgs& a, CMember& m) {
+    return m.pot_deg >= 0 || !(a.flags & kGP);
+  }
+  __device__ __forceinline__ static void mul_loads(MulLoads& l, const SweepArgs& a, CMember& m, int t, int col,
+                                                   int tab) {
+    l.mask = 1.0;
+    if (m.xmask) l.mask = gmem(m.xmask)[col];
+    if (m.pot_deg < 0 || (a.flags & kGP)) {
+      const size_t toff = (m.pot_deg < 0 && tab && m.pot_expr_len > 0) ? size_t(m.X) * size_t(m.P) : 0;
+      const gptr<const double> src = gmem(m.pot_deg < 0 ? m.pot_dv : const_cast<const double*>(m.G)) + toff;
 #pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.theta_decay)[t + j * TT], 0.0});
+      for (int j = 0; j < R; ++j) l.tab[j] = src[size_t(t + j * TT) * m.X + col];
     }
+  }
+  __device__ __forceinline__ static void multipliers(cplx<double> (&M)[R], const MulLoads& l, const SweepArgs& a,
+                                                     CMember& m, int t, int col, int step, double scale) {
+    const double x = m.dx * double(fidx(col, m.X));
+    const int row = step < m.pot_rows ? step : m.pot_rows - 1;
+    const bool gp = (a.flags & kGP) != 0;
+    const double mask = l.mask * scale;
+    const BoppOdd bopp = bopp_odd(cmem(m.pot) + size_t(row) * (kMaxDeg + 1), m.pot_deg, x, a.vphase);
+    const double hd = a.hbar_half * m.dtheta;
+    auto phase = [&](int i) { return bopp(hd * double(fidx(i, N))); };
+    if (kWave && m.pot_deg >= 0 && !gp) {
+#pragma unroll
+      for (int j = 0; j < R / 2; ++j) M[j] = expmi(mask, phase(t + j * TT));
+      const cplx<double> nyq = expmi(mask, phase(N / 2));
+      const int lane = threadIdx.x & 63;
+      const int src = lane - t + ((TT - t) & (TT - 1));
+      static_for<R / 2, R>([&](auto J) {
+        constexpr int j = decltype(J)::value;
+        cplx<double> q{__shfl(M[R - 1 - j].x, src, 64), __shfl(M[R - 1 - j].y, src, 64)};
+        if constexpr (j == R / 2) {
+          if (t == 0) q = {nyq.x, -nyq.y};
+        } else {
+          if (t == 0) q = M[R - j];
+        }
+        M[j] = {q.x, -q.y};
+      });
+    } else if (m.pot_deg < 0) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) M[j] = expmi(mask, a.vphase * l.tab[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        double phi = phase(t + j * TT);
+        if (gp) phi -= a.gp_phase * l.tab[j];
+        M[j] = expmi(mask, phi);
+      }
+    }
+  }
+  // whether time index step + 1 has the multipliers of step: one row of coefficients, or one
+  // table, for both (the merged half steps, which have no Gross-Pitaevskii phase)
+  __device__ __forceinline__ static bool same_multipliers(CMember& m, int step) {
+    return m.pot_deg >= 0 ? step >= m.pot_rows - 1 : m.pot_expr_len == 0;
+  }
+  __device__ __forceinline__ static void multiply(cplx<T> (&v)[R], const cplx<double> (&M)[R]) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = apply(v[j], M[j]);
   }
 
   // D(Y) = F_p^{-1}[ theta * F_p[ sigma(p) Y ] ]   (Theta_fp_Damping, FFT.py:1135-1143);
-  // the 1/N of the inverse transform is folded into theta (a power of two: exact)
+  // sg, th: sigma and theta / N of this lane's elements (the 1/N of the inverse transform is a
+  // power of two: exact), read once per sweep
   template <class Tw>
-  __device__ __forceinline__ static void cl_operator(cplx<T> (&y)[R], const Member& m, int t,
+  __device__ __forceinline__ static void cl_operator(cplx<T> (&y)[R], const T (&sg)[R], const T (&th)[R], int t,
                                                      View view, const Tw& tw) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], T(gmem(m.sigma_p)[t + j * TT]));
+    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], sg[j]);
     team_fft<T, N, R, -1, View, Sync>(y, t, view, tw);
 #pragma unroll
-    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], T(gmem(m.theta_host)[t + j * TT] * (1.0 / N)));
+    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], th[j]);
     team_fft<T, N, R, +1, View, Sync>(y, t, view, tw);
   }
 };
@@ -508,7 +638,7 @@ constexpr int kPTailBytes = 64 * 12 * 8;
 // TT consecutive lanes (column cc = tid / TT, team index tc = tid % TT) and the store
 // moves it back through LDS; otherwise the load layout is kept throughout.
 template <typename S, typename T, int N, int R, int BLOCK, bool CL, bool TP, typename E>
-__device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m, int tile,
+__device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int tile,
                                             cplx<E>* lds) {
   using PS = PSweep<T, N, R, BLOCK, E>;
   using View = typename PS::View;
@@ -523,13 +653,32 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m,
   const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(m.W));
   const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(m.twP_hi), reinterpret_cast<const cplx<T>*>(m.twP_lo)};
   const View view_c{kWave ? lds + cc * LSZ : lds + cl};
-  const int step = (a.flags & kStepArg) ? a.step_add : *gmem(a.step) + a.step_add;
+  const int step = (a.flags & kStepArg) ? a.step_add : *cmem(a.step) + a.step_add;
 
   // 32-bit byte offsets from the member's base (a state is at most 2048^2 x 16 B); the
   // store recomputes them from an opaque copy of the lane index, so that no address
   // stays live (or is spilled) across the transforms
   const unsigned boff = (unsigned(tl) * unsigned(X) + unsigned(tile * C + cl)) * unsigned(sizeof(cplx<S>));
   const unsigned jstride = unsigned(TT) * unsigned(X) * unsigned(sizeof(cplx<S>));
+  // radix-8 lanes have the registers to keep the multipliers over the first transform (radix-16
+  // lanes spill: -13% on 32 grids of 1024^2)
+  constexpr bool kEarly = R <= 8 && !TP;
+  const bool early = kEarly && PS::early(a, m);
+  typename PS::MulLoads ml;
+  if (early) PS::mul_loads(ml, a, m, tc, col, 0);
+  // the friction tables and the host values of one column per lane: in registers when the state is
+  T sg[CL ? R : 1], th[CL ? R : 1];
+  double decay[CL ? R : 1];  // (a plan with friction always has the table)
+  if constexpr (CL) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if constexpr (kEarly) decay[j] = gmem(m.theta_decay)[tc + j * TT];
+      sg[j] = T(gmem(m.sigma_p)[tc + j * TT]);
+      th[j] = T(gmem(m.theta_host)[tc + j * TT] * (1.0 / N));
+    }
+  }
+  ColumnHost host{0.0, 0.0, 0.0};
+  if (a.flags & kTilePart) host = column_host(m, tile * C + tid % C);
   cplx<T> v[R];
 #pragma unroll
   for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload(at_off(W, boff + unsigned(j) * jstride)));
@@ -542,6 +691,8 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m,
       return TwMem<T>{tw};
     }
   }();
+  cplx<double> M[R];
+  if (early) PS::multipliers(M, ml, a, m, tc, col, step, 1.0 / N);
   if (a.flags & kScaleOnLoad) {
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = scale_load(v[j], m.scale);
@@ -551,27 +702,43 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m,
   } else {
     team_fft<T, N, R, -1, View, Sync>(v, tc, view_c, twsrc);
   }
-  PS::potential(v, a, m, tc, col, step, 1.0 / N, 0);
+  const auto theta_decay = [&]() {
+    if constexpr (CL) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{decay[j], 0.0});
+    } else if (m.theta_decay) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.theta_decay)[tc + j * TT], 0.0});
+    }
+  };
+  if constexpr (CL && !kEarly) {  // in flight while potential() evaluates its multipliers
+    const int t = opaque_v(tc);
+#pragma unroll
+    for (int j = 0; j < R; ++j) decay[j] = gmem(m.theta_decay)[t + j * TT];
+  }
+  if (early)
+    PS::multiply(v, M);
+  else
+    PS::potential(v, a, m, tc, col, step, 1.0 / N, 0);
+  theta_decay();
   team_fft<T, N, R, +1, View, Sync>(v, tc, view_c, twsrc);
 
   if constexpr (CL) {
-    // W + 2aD W + (10/3)a^2 D^2 W + (4/3)a^3 D^3 W, a = i dt gamma, built as
-    // LW = W + (2/3)a D W; LW += a D LW; W += 2a D LW   (FFT.py:1145-1157)
-    cplx<T> lw[R], d[R];
+    // W + 2aD W + (10/3)a^2 D^2 W + (4/3)a^3 D^3 W, a = i dt gamma: the reference's nested
+    // LW = W + (2/3)a D W; LW += a D LW; W += 2a D LW (FFT.py:1145-1157) as the sum of the
+    // powers, which needs two copies of the column in registers instead of three
+    cplx<T> d[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) d[j] = v[j];
-    PS::cl_operator(d, m, tc, view_c, twsrc);
-    const T c1 = T((2.0 / 3.0) * a.cl_a), c2 = T(a.cl_a), c3 = T(2.0 * a.cl_a);
+    const T c1 = T(2.0 * a.cl_a), c2 = T((-10.0 / 3.0) * a.cl_a * a.cl_a),
+            c3 = T((-4.0 / 3.0) * a.cl_a * a.cl_a * a.cl_a);
+    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
 #pragma unroll
-    for (int j = 0; j < R; ++j) lw[j] = cadd(v[j], mul_i(d[j], c1));
+    for (int j = 0; j < R; ++j) v[j] = cadd(v[j], mul_i(d[j], c1));
+    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
 #pragma unroll
-    for (int j = 0; j < R; ++j) d[j] = lw[j];
-    PS::cl_operator(d, m, tc, view_c, twsrc);
-#pragma unroll
-    for (int j = 0; j < R; ++j) lw[j] = cadd(lw[j], mul_i(d[j], c2));
-#pragma unroll
-    for (int j = 0; j < R; ++j) d[j] = lw[j];
-    PS::cl_operator(d, m, tc, view_c, twsrc);
+    for (int j = 0; j < R; ++j) v[j] = cadd(v[j], cscale(d[j], c2));
+    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = cadd(v[j], mul_i(d[j], c3));
   }
@@ -647,8 +814,17 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m,
   }
 
   if (a.flags & kMerge) {
+    if (early && !PS::same_multipliers(m, step)) {
+      const int t = opaque_v(tc), c = opaque_v(col);
+      PS::mul_loads(ml, a, m, t, c, 1);
+      PS::multipliers(M, ml, a, m, t, c, step + 1, 1.0 / N);
+    }
     team_fft<T, N, R, -1, View, Sync>(v, tc, view_c, twsrc);
-    PS::potential(v, a, m, tc, col, step + 1, 1.0 / N, 1);
+    if (early)
+      PS::multiply(v, M);
+    else
+      PS::potential(v, a, m, tc, col, step + 1, 1.0 / N, 1);
+    theta_decay();
     team_fft<T, N, R, +1, View, Sync>(v, tc, view_c, twsrc);
   }
 
@@ -667,12 +843,12 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, const Member& m,
   const unsigned soff = (unsigned(ts / C) * unsigned(X) + unsigned(tile * C + ts % C)) * unsigned(sizeof(cplx<S>));
 #pragma unroll
   for (int j = 0; j < R; ++j) store_cached(at_off(W, soff + unsigned(j) * jstride), to_arith<S>(v[j]));
-  if (a.flags & kTilePart) write_tile_partial<BLOCK, C>(a, m, tile, csum, step - a.step_add);
+  if (a.flags & kTilePart) write_tile_partial<C>(a, m, tile, csum, host, step - a.step_add);
 }
 
 // ------------------------------------------------------------------ Gross-Pitaevskii shift
-template <int N, int R, int BLOCK>
-__device__ __forceinline__ void gpshift_body(const Member& m, int tile, cplx<double>* lds) {
+template <int N, int R, int BLOCK, class M>
+__device__ __forceinline__ void gpshift_body(const M& m, int tile, cplx<double>* lds) {
   constexpr int TT = N / R, ROWS = BLOCK / TT;
   constexpr int LSZ = Padded<N, R>::size;
   const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
@@ -722,9 +898,17 @@ template <typename S, typename T, int R, int BLOCK, bool TP>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TP ? 3 : 2))) xsweep_kernel(SweepArgs a) {
   using E = LdsElem<S, T, TP>;
   __shared__ cplx<E> lds[lds_elems<BLOCK, R>() + kTileRedBytes / sizeof(cplx<E>)];
-  const unsigned w = a.work[blockIdx.x];
-  const Member& m = a.members[w >> 16];
+  const unsigned w = x_item(a);
+  CMember& m = member_at(a.members, w >> 16);
+  // the fields that the sweep's loads wait for, in one round of scalar loads (left to its use, each
+  // came after a wait of its own: 1024^2 x sweep 15.9 -> 14.7 us, p sweep with friction 32.2 -> 30.6)
+  asm volatile("" ::"s"(m.W), "s"(m.X), "s"(m.P), "s"(m.twX_hi), "s"(m.tilepart), "s"(m.dp), "s"(m.dlambda),
+               "s"(m.dxdp), "s"(m.scale), "s"(m.lambda_decay));
   const int tile = int(w & 0xffffu);
+  if (tile == kRecordTile) {
+    if (a.flags & kTileScale) record_item<BLOCK>(a, m, reinterpret_cast<double*>(lds));
+    return;
+  }
 #define BODY(n) xsweep_body<S, T, n, R, BLOCK, TP, E>(a, m, tile, lds)
   WH_DISPATCH_TO(m.X, BODY, TP ? kTpMaxN : 2048)
 #undef BODY
@@ -734,8 +918,12 @@ template <typename S, typename T, int R, int BLOCK, bool CL, bool TP>
 __device__ __forceinline__ void psweep_entry(const SweepArgs& a) {
   using E = LdsElem<S, T, TP>;
   __shared__ cplx<E> lds[lds_elems<BLOCK, R>() + kPTailBytes / sizeof(cplx<E>)];
-  const unsigned w = a.work[blockIdx.x];
-  const Member& m = a.members[w >> 16];
+  const unsigned w = p_item(a);
+  CMember& m = member_at(a.members, w >> 16);
+  // the fields that the sweep's loads wait for, in one round of scalar loads
+  asm volatile("" ::"s"(m.W), "s"(m.X), "s"(m.P), "s"(m.pot), "s"(m.pot_deg), "s"(m.pot_rows), "s"(m.xmask),
+               "s"(m.theta_decay), "s"(m.twP_hi), "s"(m.x_host), "s"(m.dv_host), "s"(m.v0_host), "s"(m.p_host),
+               "s"(m.dx), "s"(m.dtheta), "s"(m.sigma_p), "s"(m.theta_host), "s"(*cmem(a.step)));
   const int tile = int(w & 0xffffu);
 #define BODY(n) psweep_body<S, T, n, R, BLOCK, CL, TP, E>(a, m, tile, lds)
   WH_DISPATCH_TO(m.P, BODY, TP && !CL ? kTpMaxN : 2048)
@@ -750,7 +938,7 @@ template <int R, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) gpshift_kernel(const Member* members, const unsigned* work) {
   __shared__ cplx<double> lds[lds_elems<BLOCK, R>()];
   const unsigned w = work[blockIdx.x];
-  const Member& m = members[w >> 16];
+  CMember& m = member_at(members, w >> 16);
   const int tile = int(w & 0xffffu);
 #define BODY(n) gpshift_body<n, R, BLOCK>(m, tile, lds)
   WH_DISPATCH(m.X, BODY)

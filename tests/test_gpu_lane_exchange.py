@@ -100,3 +100,30 @@ def test_p_sweep(cuda, N, precision):
         assert rel(Y, ref) < bound, (N, v)
         done += 1
     assert done >= 1
+
+
+@pytest.mark.parametrize("X,P", [(128, 128), (256, 512), (128, 1024)])
+def test_friction_without_diffusion(cuda, X, P):
+    """Caldeira-Leggett friction with D_theta = 0 (no decay table from the caller) in every p variant,
+    record rows included, against the oracle: 4 steps, the FP64 bar of the parity tests (1e-10)."""
+    from oracle import wigner2d as ow
+    from pywignercuda_amd.wigner2d import Wigner2D
+
+    args = (X, P, 9.0, 7.0, 0.8, 1.3, 0.01)
+    kw = dict(scheme="lie", gamma=0.1, damping="CaldeiraLeggett", mask=True)
+    p = Wigner2D(*args, potential="0.5*pow(x,2)+0.02*pow(x,4)", dpotential="x+0.08*pow(x,3)", fp_damping="fabs(p)",
+                 device=cuda, variants=(-1, -1, -1), **kw)
+    o = ow.Wigner2DOracle(*args, potential=lambda t, x: 0.5 * x ** 2 + 0.02 * x ** 4,
+                          dpotential=lambda t, x: x + 0.08 * x ** 3, fp_damping=np.abs, **kw)
+    W0 = ow.gaussian_wigner(o.g, x0=1.0, p0=-0.5, s=1.1)
+    ref, obs_ref, _ = o.run(W0, 3)
+    done = 0
+    for v in variants(2):
+        if not try_variant(p, pclvar=v):
+            continue
+        W = p.to_device(W0)
+        obs = p.run(W, 4).cpu().numpy()
+        assert np.linalg.norm(W.cpu().numpy() - ref) < 1e-10 * np.linalg.norm(ref), v
+        assert abs(obs[3, 0] - obs_ref["X"][3]) < 1e-10 and abs(obs[3, 9] - obs_ref["neg"][3]) < 1e-10, v
+        done += 1
+    assert done >= 1
