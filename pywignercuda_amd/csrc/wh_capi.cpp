@@ -32,14 +32,14 @@ hipError_t launch_psweep_f64(int variant, bool cl, const SweepArgs& a, int nwork
 hipError_t launch_psweep_f32(int variant, bool cl, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_expr_table(const Member* members, int member, int cells, int depth, const int* step,
                              int step_add, int use_arg, int ntables, double hbar_half, hipStream_t s);
-hipError_t launch_gpshift(const Member* members, const unsigned* work, int nwork, hipStream_t s);
+hipError_t launch_gpshift(const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_colsum(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s);
 hipError_t launch_observe_noalloc(int prec, Member m, hipStream_t s);
 int noalloc_max_x();
 hipError_t launch_xsweep_f32w(int variant, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_psweep_f32w(int variant, bool cl, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_reduce(const ReduceArgs& a, int nmembers, int* done, hipStream_t s);
-hipError_t launch_colpart_reduce(const Member* members, int nmembers, int xradix, int xblock, const int* step,
+hipError_t launch_colpart_reduce(const Member* members, int nmembers, int max_x, int xradix, int xblock,
                                  hipStream_t s);
 hipError_t launch_scale(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s);
 hipError_t launch_set_int(int* p, int v, hipStream_t s);
@@ -579,6 +579,7 @@ int build_work_lists(wh_ensemble* e) {
   e->built_pcl = wh::kPCLVariants[e->pclvar];
   WH_TRY(e->work_colsum.upload(wc));
   WH_TRY(e->work_scale.upload(ws));
+  for (int i = 0; i < e->n; ++i) wg.push_back((unsigned(i) << 16) | unsigned(wh::kRecordTile));
   if (e->gp()) WH_TRY(e->work_gp.upload(wg));
   if (e->odm()) {
     WH_TRY(e->work_odm_x.upload(wox));
@@ -716,6 +717,15 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
     return fail(WH_INVALID_SIZE, "no kernel variant fits every member's grid");
   };
   WH_TRY(pick(wh::kXVariants, wh::kNumX, true, e->xvar));
+  if (gp) {
+    // fixed for the plan's life (the partial sums are cut by its rows per tile): the radix that is
+    // fastest for a single grid of the widest member's side, measured per x sweep: 4 up to 256,
+    // 8 at 512 (7.4 us at 512^2; radix 16: 9.4) and 2048, 16 at 1024
+    int side = 0;
+    for (const auto& m : e->mem) side = std::max(side, m.X);
+    const int v = side <= 256 ? 3 : side == 1024 ? 0 : 1;
+    if (fits_all(e.get(), wh::kXVariants[v], true)) e->xvar = v;
+  }
   WH_TRY(pick(wh::kPVariants, wh::kNumP, false, e->pvar));
   WH_TRY(pick(wh::kPCLVariants, wh::kNumPCL, false, e->pclvar, true));
   for (int i = 0; i < n; ++i) e->expr = e->expr || e->mem[i].pot_expr_len > 0;
@@ -849,9 +859,20 @@ int reduce(wh_ensemble* e, int renorm, int record, int rho, int update_scale, bo
   return WH_SUCCESS;
 }
 
-int gpshift(wh_ensemble* e, hipStream_t s) {
-  WH_LAUNCH(wh::launch_gpshift(e->mem_dev.as<wh::Member>(), e->work_gp.buf.as<unsigned>(), e->work_gp.n, s),
-            "gpshift");
+int gpshift(wh_ensemble* e, int flags, hipStream_t s) {
+  wh::SweepArgs a = sweep_args(e, flags, 1.0, 0);
+  a.work = e->work_gp.buf.as<unsigned>();
+  a.ntiles = e->n == 1 ? e->work_gp.n - 1 : 0;  // the record item is the last
+  WH_LAUNCH(wh::launch_gpshift(a, e->work_gp.n, s), "gpshift");
+  return WH_SUCCESS;
+}
+// density after the kinetic step from the x sweep's partial sums
+int density(wh_ensemble* e, hipStream_t s) {
+  int max_x = 0;
+  for (const auto& m : e->mem) max_x = std::max(max_x, m.X);
+  WH_LAUNCH(wh::launch_colpart_reduce(e->mem_dev.as<wh::Member>(), e->n, max_x, wh::kXVariants[e->xvar].R,
+                                      wh::kXVariants[e->xvar].block, s),
+            "colpart_reduce");
   return WH_SUCCESS;
 }
 
@@ -861,11 +882,11 @@ int gpshift(wh_ensemble* e, hipStream_t s) {
 //  Strang (GP.py:1898-1999): without GP the second half step of iteration k and the
 //         first of k+1 share one p sweep, the observables taken between them; with GP
 //         V/2, K + partial column sums, density, V/2 + column sums.
-//  Lie and Strang without GP or ODM: no reduce launch; each p sweep writes tile partials
-//  of the observables and the next x sweep turns them into the record row and the
-//  factor (kTileScale).  `first`: the pending factor is the one of the initial reduce.
+//  Without ODM: no reduce launch; each p sweep writes tile partials of the observables and the
+//  next x sweep, or Gross-Pitaevskii shift, turns them into the record row and the factor
+//  (kTileScale).  `first`: the pending factor (and density) is the one of the initial reduce.
 //  After the last iteration tiles_pending(e) asks for one closing reduce.
-bool tiles_pending(const wh_ensemble* e) { return !e->gp() && !e->odm(); }
+bool tiles_pending(const wh_ensemble* e) { return !e->odm(); }
 int renorm_flag(const wh_ensemble* e) { return e->d.renormalize; }
 
 int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
@@ -874,7 +895,7 @@ int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
   const int renorm = d.renormalize;
   if (d.scheme == WH_SCHEME_LIE && e->odm()) {
     // K; V; W += L_ODM(W) (three sweeps); column sums of the result; renormalise
-    if (e->gp()) WH_TRY(gpshift(e, s));
+    if (e->gp()) WH_TRY(gpshift(e, 0, s));
     WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
     WH_TRY(psweep(e, e->gp() ? wh::kGP : 0, 1.0, 0, s));
     // one Lindblad channel (GPU_Wigner2D_FFT, weight 1, sign 1) or two applied in turn
@@ -893,14 +914,12 @@ int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
     // V/2; K; V/2; W += L_ODM(W); column sums; renormalise (GPU_Wigner2D_GPitaevskii.Run,
     // GP.py:1942-1968): the dissipator sits between the two half steps of consecutive
     // iterations, so they are not merged
-    if (e->gp()) WH_TRY(gpshift(e, s));
+    if (e->gp()) WH_TRY(gpshift(e, 0, s));
     WH_TRY(psweep(e, wh::kScaleOnLoad | (e->gp() ? wh::kGP : 0), 0.5, 0, s));
     if (e->gp()) {
       WH_TRY(xsweep(e, wh::kColPart, s));
-      WH_LAUNCH(wh::launch_colpart_reduce(e->mem_dev.as<wh::Member>(), e->n, wh::kXVariants[e->xvar].R,
-                                          wh::kXVariants[e->xvar].block, e->step.as<int>(), s),
-                "colpart_reduce");
-      WH_TRY(gpshift(e, s));
+      WH_TRY(density(e, s));
+      WH_TRY(gpshift(e, wh::kProbSq, s));
     } else {
       WH_TRY(xsweep(e, 0, s));
     }
@@ -915,10 +934,9 @@ int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
               "colsum");
     WH_TRY(reduce(e, renorm, 1, e->gp(), 1, true, s));
   } else if (d.scheme == WH_SCHEME_LIE && e->gp()) {
-    WH_TRY(gpshift(e, s));
+    WH_TRY(gpshift(e, first ? 0 : wh::kTileScale, s));
     WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
-    WH_TRY(psweep(e, wh::kColSums | cl | wh::kGP, 1.0, 0, s));
-    WH_TRY(reduce(e, renorm, 1, 1, 1, true, s));
+    WH_TRY(psweep(e, wh::kColSums | wh::kTilePart | cl | wh::kGP, 1.0, 0, s));
   } else if (d.scheme == WH_SCHEME_LIE) {
     WH_TRY(xsweep(e, first ? wh::kScaleOnLoad : wh::kTileScale, s));
     WH_TRY(psweep(e, wh::kColSums | wh::kTilePart | cl, 1.0, 0, s));
@@ -926,15 +944,12 @@ int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
     WH_TRY(xsweep(e, first ? wh::kScaleOnLoad : wh::kTileScale, s));
     WH_TRY(psweep(e, wh::kColSums | wh::kTilePart | cl | (merge ? wh::kMerge : 0), 0.5, 0, s));
   } else {
-    WH_TRY(gpshift(e, s));
+    WH_TRY(gpshift(e, first ? 0 : wh::kTileScale, s));
     WH_TRY(psweep(e, wh::kScaleOnLoad | wh::kGP, 0.5, 0, s));
     WH_TRY(xsweep(e, wh::kColPart, s));
-    WH_LAUNCH(wh::launch_colpart_reduce(e->mem_dev.as<wh::Member>(), e->n, wh::kXVariants[e->xvar].R,
-                                        wh::kXVariants[e->xvar].block, e->step.as<int>(), s),
-              "colpart_reduce");
-    WH_TRY(gpshift(e, s));
-    WH_TRY(psweep(e, wh::kGP | wh::kColSums | cl, 0.5, 0, s));
-    WH_TRY(reduce(e, renorm, 1, 1, 1, true, s));
+    WH_TRY(density(e, s));
+    WH_TRY(gpshift(e, wh::kProbSq, s));
+    WH_TRY(psweep(e, wh::kGP | wh::kColSums | wh::kTilePart | cl, 0.5, 0, s));
   }
   return WH_SUCCESS;
 }

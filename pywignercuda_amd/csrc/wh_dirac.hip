@@ -1021,7 +1021,10 @@ __global__ void __launch_bounds__(256) dirac_gpshift_kernel(const DiracPlan* __r
   m.X = d.X;
   m.P = d.P;
   constexpr int R = kDiracGpR, BLOCK = 256;
-#define BODY(n) gpshift_body<n, R, BLOCK>(m, int(blockIdx.x), lds)
+#define BODY(n)                                                                                     \
+  cplx<double> v[R];                                                                                \
+  for (int j = 0; j < R; ++j) v[j] = {gmem(m.rho)[int(threadIdx.x) % (n / R) + j * (n / R)], 0.0};  \
+  gpshift_rows<n, R, BLOCK>(v, m, int(blockIdx.x), lds)
   WH_DISPATCH(d.X, BODY)
 #undef BODY
 }

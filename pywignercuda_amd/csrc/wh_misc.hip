@@ -161,26 +161,30 @@ __global__ void __launch_bounds__(256) reduce_kernel(ReduceArgs a, int* done, in
 }
 
 // ------------------------------------------------------------------ density after K
-__global__ void __launch_bounds__(256) colpart_reduce_kernel(const Member* members, int xradix, int xblock,
-                                                             const int* step) {
-  __shared__ double red[256];
-  const Member& m = members[blockIdx.x];
+// rho(x) from the x sweep's partial sums [tiles][X].  One work item = COLS columns of one
+// member, 256 / COLS groups of lanes each summing every (256 / COLS)-th tile.  (One block
+// per member, a column per lane and all tiles in its loop, took 28 us at 512^2.)
+template <int COLS>
+__global__ void __launch_bounds__(256) colpart_reduce_kernel(const Member* members, int xradix, int xblock) {
+  constexpr int G = 256 / COLS;
+  __shared__ double red[G][COLS];
+  CMember& m = member_at(members, blockIdx.y);
   const int nblk = m.P / (xblock / (m.X / xradix));  // x-sweep tiles of this member
-  double ps = 0.0;
-  for (int x = threadIdx.x; x < m.X; x += 256) {
-    double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += m.colpart[size_t(b) * m.X + x];
-    s *= m.rho_factor;
-    m.rho[x] = s;
-    ps += s * s;
-  }
-  red[threadIdx.x] = ps;
+  const int c = threadIdx.x % COLS, g = threadIdx.x / COLS;
+  const int x = blockIdx.x * COLS + c;
+  if (int(blockIdx.x) * COLS >= m.X) return;  // the grid spans the widest member (X is a multiple of COLS)
+  const gptr<const double> part = gmem(const_cast<const double*>(m.colpart));
+  double s = 0.0;
+#pragma unroll 8
+  for (int b = g; b < nblk; b += G) s += part[size_t(b) * m.X + x];
+  red[g][c] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if (threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
+  if (g == 0) {
+    s = 0.0;
+#pragma unroll
+    for (int k = 0; k < G; ++k) s += red[k][c];
+    gmem(m.rho)[x] = s * m.rho_factor;
   }
-  if (threadIdx.x == 0 && m.obs) m.obs[size_t(*step - m.obs_base) * kNObs + kObsProbSq] = m.dx_host * red[0];
 }
 
 // ------------------------------------------------------------------ scale by the pending factor
@@ -360,9 +364,12 @@ hipError_t launch_reduce(const ReduceArgs& a, int nmembers, int* done, hipStream
   hipLaunchKernelGGL(reduce_kernel, dim3(nmembers), dim3(256), 0, s, a, done, nmembers);
   return hipGetLastError();
 }
-hipError_t launch_colpart_reduce(const Member* members, int nmembers, int xradix, int xblock, const int* step,
+hipError_t launch_colpart_reduce(const Member* members, int nmembers, int max_x, int xradix, int xblock,
                                  hipStream_t s) {
-  hipLaunchKernelGGL(colpart_reduce_kernel, dim3(nmembers), dim3(256), 0, s, members, xradix, xblock, step);
+  // 16 columns (one 128-byte line per row of partials) and 16 lane groups
+  constexpr int COLS = 16;
+  hipLaunchKernelGGL(colpart_reduce_kernel<COLS>, dim3(max_x / COLS, nmembers), dim3(256), 0, s, members, xradix,
+                     xblock);
   return hipGetLastError();
 }
 hipError_t launch_scale(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s) {

@@ -10,7 +10,7 @@
 //           (expPotential GPU_Wigner2D_FFT.py:80-126, 795-801, 1891-1913;
 //            expPotential_GrossPitaevskii :479-519; theta_fp + CaldeiraDissipatorOrder3
 //            :399-431, 1135-1157; GPU_Wigner2D_GPitaevskii.py:60-86, 466-496, 1911-1970)
-//   gpshift G(theta, x) = Re iFFT_x[ FFT_x(rho) (-2i sin(lambda theta/2)) ]
+//   gpshift (rows theta)  G(theta, x) = Re iFFT_x[ FFT_x(rho) (-2i sin(lambda theta/2)) ]
 //           (MakeGrossPitaevskiiTerms, GPU_Wigner2D_FFT.py:1687-1705)
 //
 // Each sweep reads and writes the state once.  Phase multipliers are evaluated
@@ -847,29 +847,81 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
 }
 
 // ------------------------------------------------------------------ Gross-Pitaevskii shift
+// One theta row of G per team from the density rho(t + j TT) held in v (real parts).
 template <int N, int R, int BLOCK, class M>
-__device__ __forceinline__ void gpshift_body(const M& m, int tile, cplx<double>* lds) {
+__device__ __forceinline__ void gpshift_rows(cplx<double> (&v)[R], const M& m, int tile, cplx<double>* lds) {
   constexpr int TT = N / R, ROWS = BLOCK / TT;
   constexpr int LSZ = Padded<N, R>::size;
+  using Sync = std::conditional_t<(TT <= 64), WaveSync, BlockSync>;
   const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
   const int row = tile * ROWS + team;
   const Twiddles<double> tw{reinterpret_cast<const cplx<double>*>(m.twX64), nullptr};
   LdsRow<double> view{lds + team * LSZ};
-  cplx<double> v[R];
-#pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = {gmem(m.rho)[t + j * TT], 0.0};
-  team_fft<double, N, R, -1>(v, t, view, tw);
+  // the multiplier does not depend on the density: evaluated while its loads are in flight
+  double f[R];
   const double half_theta = 0.5 * cmem(m.theta_host)[row];
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    double sn, cs;
-    sincos_fp64(gmem(m.lambda_host)[t + j * TT] * half_theta, &sn, &cs);
-    const double f = 2.0 * sn;  // (-2i sin) * (a + ib) = 2 sin b - 2i sin a
-    v[j] = {f * v[j].y, -f * v[j].x};
+    double cs;
+    sincos_fp64(gmem(m.lambda_host)[t + j * TT] * half_theta, &f[j], &cs);
   }
-  team_fft<double, N, R, +1>(v, t, view, tw);
+  const auto twsrc = [&]() {
+    if constexpr (TT <= 64) {
+      TwRegs<double, N, R> r;
+      load_twiddles<double, N, R>(r, t, tw);
+      return r;
+    } else {
+      return TwMem<double>{tw};
+    }
+  }();
+  team_fft<double, N, R, -1, LdsRow<double>, Sync>(v, t, view, twsrc);
+#pragma unroll
+  for (int j = 0; j < R; ++j) v[j] = {2.0 * f[j] * v[j].y, -2.0 * f[j] * v[j].x};  // (-2i sin) (a + ib)
+  team_fft<double, N, R, +1, LdsRow<double>, Sync>(v, t, view, twsrc);
 #pragma unroll
   for (int j = 0; j < R; ++j) gmem(m.G)[size_t(row) * N + t + j * TT] = v[j].x * (1.0 / N);
+}
+
+// kTileScale: the state is that of the p sweep just done: its density is the column sums times the
+// pending factor (from the tile partials, as in the x sweep), and the member's record item forms
+// the record row; without it the density is read from m.rho.  kProbSq: tile 0 records
+// dX sum rho^2 (GP.py:1937-1939).
+template <int N, int R, int BLOCK>
+__device__ __forceinline__ void gpshift_body(const SweepArgs& a, CMember& m, int tile, cplx<double>* lds) {
+  constexpr int TT = N / R;
+  const int t = threadIdx.x % TT;
+  cplx<double> v[R];
+  if (a.flags & kTileScale) {
+    const TilePartials part = tile_partials<BLOCK>(a, m);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const gptr<const double> cs = gmem(const_cast<const double*>(m.colsums)) + size_t(t + j * TT) * kNCol;
+      v[j] = {cs[0], cs[1]};
+    }
+    const cplx<double> f = tile_scale<BLOCK>(a, m, part, reinterpret_cast<double*>(lds + lds_elems<BLOCK, R>()));
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = {(v[j].x * f.x - v[j].y * f.y) * m.rho_factor, 0.0};
+  } else {
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = {gmem(m.rho)[t + j * TT], 0.0};
+  }
+  if ((a.flags & kProbSq) && tile == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < R; ++j) s = fma(v[j].x, v[j].x, s);
+    constexpr int G = TT < 64 ? TT : 64;
+    s = group_sum<G>(s);  // of one team, or of each of a team's waves
+    if constexpr (TT > 64) {
+      double* red = reinterpret_cast<double*>(lds + lds_elems<BLOCK, R>());
+      if (threadIdx.x % 64 == 63) red[threadIdx.x / 64] = s;
+      __syncthreads();
+      s = 0.0;
+#pragma unroll
+      for (int w = 0; w < TT / 64; ++w) s += red[w];
+    }
+    if (threadIdx.x == TT - 1) gmem(m.obs)[size_t(*cmem(a.step) - m.obs_base) * kNObs + kObsProbSq] = m.dx_host * s;
+  }
+  gpshift_rows<N, R, BLOCK>(v, m, tile, lds);
 }
 
 // ------------------------------------------------------------------ kernels
@@ -935,12 +987,18 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(CL ?
 }
 
 template <int R, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) gpshift_kernel(const Member* members, const unsigned* work) {
-  __shared__ cplx<double> lds[lds_elems<BLOCK, R>()];
-  const unsigned w = work[blockIdx.x];
-  CMember& m = member_at(members, w >> 16);
+__global__ void __launch_bounds__(BLOCK) gpshift_kernel(SweepArgs a) {
+  __shared__ cplx<double> lds[lds_elems<BLOCK, R>() + kTileRedBytes / sizeof(cplx<double>)];
+  const unsigned w = x_item(a);
+  CMember& m = member_at(a.members, w >> 16);
   const int tile = int(w & 0xffffu);
-#define BODY(n) gpshift_body<n, R, BLOCK>(m, tile, lds)
+  asm volatile("" ::"s"(m.X), "s"(m.P), "s"(m.rho), "s"(m.colsums), "s"(m.tilepart), "s"(m.G), "s"(m.twX64),
+               "s"(m.lambda_host), "s"(m.theta_host), "s"(m.rho_factor), "s"(m.dxdp));
+  if (tile == kRecordTile) {
+    if (a.flags & kTileScale) record_item<BLOCK>(a, m, reinterpret_cast<double*>(lds));
+    return;
+  }
+#define BODY(n) gpshift_body<n, R, BLOCK>(a, m, tile, lds)
   WH_DISPATCH(m.X, BODY)
 #undef BODY
 }

@@ -5,8 +5,8 @@
 #include "wh_sweeps_inst.inc"
 
 namespace wh {
-hipError_t launch_gpshift(const Member* members, const unsigned* work, int nwork, hipStream_t s) {
-  hipLaunchKernelGGL((gpshift_kernel<16, 256>), dim3(nwork), dim3(256), 0, s, members, work);
+hipError_t launch_gpshift(const SweepArgs& a, int nwork, hipStream_t s) {
+  hipLaunchKernelGGL((gpshift_kernel<16, 256>), dim3(nwork), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 }  // namespace wh
