@@ -55,8 +55,9 @@ hipError_t launch_grad_reduce(const Member* members, int nmembers, double* grad,
 int adj_cols(int P);
 int odm_rows_per_tile(int X);
 int odm_cols_per_tile(int P);
-hipError_t launch_odm(int prec, const Member* members, const unsigned* work_rows, int nrows,
-                      const unsigned* work_cols, int ncols, double weight, double sgn, hipStream_t s);
+int odm_radix();
+int odm_block();
+hipError_t launch_odm(int prec, int kind, const SweepArgs& a, int nwork, double weight, double sgn, hipStream_t s);
 hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s);
 hipError_t launch_dirac_psweep(int prec, int P, bool cl, const DiracPlan* d, int nblocks, hipStream_t s);
 hipError_t launch_dirac_colsum(int prec, const DiracPlan* d, int X, hipStream_t s);
@@ -581,6 +582,7 @@ int build_work_lists(wh_ensemble* e) {
   WH_TRY(e->work_scale.upload(ws));
   for (int i = 0; i < e->n; ++i) wg.push_back((unsigned(i) << 16) | unsigned(wh::kRecordTile));
   if (e->gp()) WH_TRY(e->work_gp.upload(wg));
+  for (int i = 0; i < e->n; ++i) wox.push_back((unsigned(i) << 16) | unsigned(wh::kRecordTile));
   if (e->odm()) {
     WH_TRY(e->work_odm_x.upload(wox));
     WH_TRY(e->work_odm_p.upload(wop));
@@ -768,7 +770,10 @@ wh::SweepArgs sweep_args(const wh_ensemble* e, int flags, double frac, int step_
   a.kdeg = d.kinetic_deg;
   for (int k = 0; k <= wh::kMaxDeg; ++k) a.kcoef[k] = d.kin_coef[k];
   a.rec_step = e->step.as<int>() + 1;
-  const wh::SweepVariant pv = e->cl() ? wh::kPCLVariants[e->pclvar] : wh::kPVariants[e->pvar];
+  // the tiles that wrote the partials: of the last p sweep, or of the ODM join
+  const wh::SweepVariant pv = e->odm() ? wh::SweepVariant{wh::odm_radix(), wh::odm_block(), 0}
+                              : e->cl() ? wh::kPCLVariants[e->pclvar]
+                                        : wh::kPVariants[e->pvar];
   a.pt_R = pv.R;
   a.pt_block = pv.block;
   a.fin_renorm = d.renormalize;
@@ -882,57 +887,78 @@ int density(wh_ensemble* e, hipStream_t s) {
 //  Strang (GP.py:1898-1999): without GP the second half step of iteration k and the
 //         first of k+1 share one p sweep, the observables taken between them; with GP
 //         V/2, K + partial column sums, density, V/2 + column sums.
-//  Without ODM: no reduce launch; each p sweep writes tile partials of the observables and the
-//  next x sweep, or Gross-Pitaevskii shift, turns them into the record row and the factor
-//  (kTileScale).  `first`: the pending factor (and density) is the one of the initial reduce.
+//  No reduce launch (but for ODM with GP, whose density needs column sums): each p sweep, or ODM
+//  join, writes tile partials of the observables and the next x sweep, Gross-Pitaevskii shift or
+//  p sweep turns them into the factor (kTileScale); the record row is an item of that launch.  `first`: the pending factor (and density) is the one of the initial reduce.
 //  After the last iteration tiles_pending(e) asks for one closing reduce.
-bool tiles_pending(const wh_ensemble* e) { return !e->odm(); }
+bool tiles_pending(const wh_ensemble* e) { return !(e->odm() && e->gp()); }
 int renorm_flag(const wh_ensemble* e) { return e->d.renormalize; }
+
+// One sweep of the dissipator; records: an odm_x launch with the members' record items.
+int odm(wh_ensemble* e, int kind, double weight, double sgn, bool records, hipStream_t s) {
+  const bool rows = kind != wh::kOdmP;
+  const int n = rows ? e->work_odm_x.n - (records ? 0 : e->n) : e->work_odm_p.n;  // (record items last)
+  wh::SweepArgs a = sweep_args(e, 0, 1.0, 0);
+  a.work = rows ? e->work_odm_x.buf.as<unsigned>() : e->work_odm_p.buf.as<unsigned>();
+  a.ntiles = e->n == 1 ? n - (records ? 1 : 0) : 0;
+  if (kind == wh::kOdmJoin && e->d.scheme != WH_SCHEME_LIE) a.kin_linear = 0;  // no kinetic step
+  WH_LAUNCH(wh::launch_odm(e->d.precision, kind, a, n, weight, sgn, s), "odm");
+  return WH_SUCCESS;
+}
+// One Lindblad channel (GPU_Wigner2D_FFT, weight 1, sign 1) or two applied in turn
+// (GPU_Wigner2D_ODM2: weightLindbland1 with sign 1, then weightLindbland2 with sign -1);
+// last_back: with the last channel's odm_back.
+int odm_channels(wh_ensemble* e, bool records, bool last_back, hipStream_t s) {
+  const auto& d = e->d;
+  const int nch = d.odm_channels == 2 ? 2 : 1;
+  for (int ch = 0; ch < nch; ++ch) {
+    const double w = ch == 0 ? d.odm_weight1 : d.odm_weight2, sgn = ch == 0 ? 1.0 : -1.0;
+    WH_TRY(odm(e, wh::kOdmX, w, sgn, records && ch == 0, s));
+    WH_TRY(odm(e, wh::kOdmP, w, sgn, false, s));
+    if (last_back || ch < nch - 1) WH_TRY(odm(e, wh::kOdmBack, w, sgn, false, s));
+  }
+  return WH_SUCCESS;
+}
 
 int iteration(wh_ensemble* e, bool merge, bool first, hipStream_t s) {
   const auto& d = e->d;
   const int cl = e->cl() ? wh::kCL : 0;
   const int renorm = d.renormalize;
-  if (d.scheme == WH_SCHEME_LIE && e->odm()) {
-    // K; V; W += L_ODM(W) (three sweeps); column sums of the result; renormalise
-    if (e->gp()) WH_TRY(gpshift(e, 0, s));
-    WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
-    WH_TRY(psweep(e, e->gp() ? wh::kGP : 0, 1.0, 0, s));
-    // one Lindblad channel (GPU_Wigner2D_FFT, weight 1, sign 1) or two applied in turn
-    // (GPU_Wigner2D_ODM2: weightLindbland1 with sign 1, then weightLindbland2 with sign -1)
-    for (int ch = 0; ch < (d.odm_channels == 2 ? 2 : 1); ++ch)
-      WH_LAUNCH(wh::launch_odm(d.precision, e->mem_dev.as<wh::Member>(), e->work_odm_x.buf.as<unsigned>(),
-                               e->work_odm_x.n, e->work_odm_p.buf.as<unsigned>(), e->work_odm_p.n,
-                               ch == 0 ? d.odm_weight1 : d.odm_weight2, ch == 0 ? 1.0 : -1.0, s),
-                "odm");
-    WH_LAUNCH(wh::launch_colsum(storage_code(d.precision), e->mem_dev.as<wh::Member>(),
-                                e->work_colsum.buf.as<unsigned>(),
-                                e->work_colsum.n, s),
-              "colsum");
-    WH_TRY(reduce(e, renorm, 1, e->gp(), 1, true, s));
-  } else if (d.scheme == WH_SCHEME_STRANG && e->odm()) {
-    // V/2; K; V/2; W += L_ODM(W); column sums; renormalise (GPU_Wigner2D_GPitaevskii.Run,
-    // GP.py:1942-1968): the dissipator sits between the two half steps of consecutive
-    // iterations, so they are not merged
-    if (e->gp()) WH_TRY(gpshift(e, 0, s));
-    WH_TRY(psweep(e, wh::kScaleOnLoad | (e->gp() ? wh::kGP : 0), 0.5, 0, s));
-    if (e->gp()) {
+  if (e->odm() && e->gp()) {
+    // Lie K; V, Strang V/2; K; V/2, each with the density terms, then W += L_ODM(W) (three sweeps
+    // per channel); column sums of the result (the density); renormalise.  The dissipator sits
+    // between the two half steps of consecutive iterations, so they are not merged (GP.py:1942-1968).
+    WH_TRY(gpshift(e, 0, s));
+    if (d.scheme == WH_SCHEME_LIE) {
+      WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
+      WH_TRY(psweep(e, wh::kGP, 1.0, 0, s));
+    } else {
+      WH_TRY(psweep(e, wh::kScaleOnLoad | wh::kGP, 0.5, 0, s));
       WH_TRY(xsweep(e, wh::kColPart, s));
       WH_TRY(density(e, s));
       WH_TRY(gpshift(e, wh::kProbSq, s));
-    } else {
-      WH_TRY(xsweep(e, 0, s));
+      WH_TRY(psweep(e, wh::kGP, 0.5, 0, s));
     }
-    WH_TRY(psweep(e, e->gp() ? wh::kGP : 0, 0.5, 0, s));
-    for (int ch = 0; ch < (d.odm_channels == 2 ? 2 : 1); ++ch)
-      WH_LAUNCH(wh::launch_odm(d.precision, e->mem_dev.as<wh::Member>(), e->work_odm_x.buf.as<unsigned>(),
-                               e->work_odm_x.n, e->work_odm_p.buf.as<unsigned>(), e->work_odm_p.n,
-                               ch == 0 ? d.odm_weight1 : d.odm_weight2, ch == 0 ? 1.0 : -1.0, s),
-                "odm");
+    WH_TRY(odm_channels(e, false, true, s));
     WH_LAUNCH(wh::launch_colsum(storage_code(d.precision), e->mem_dev.as<wh::Member>(),
                                 e->work_colsum.buf.as<unsigned>(), e->work_colsum.n, s),
               "colsum");
-    WH_TRY(reduce(e, renorm, 1, e->gp(), 1, true, s));
+    WH_TRY(reduce(e, renorm, 1, 1, 1, true, s));
+  } else if (e->odm()) {
+    // K; V or V/2; K; V/2, then the dissipator without its last sweep, which the next iteration
+    // begins with: odm_join adds it, takes the observables and does the next Lie kinetic step; the
+    // p sweep behind it applies the factor and the record row is an item of the odm_x launch.
+    // 512^2 Lie step: 4 launches instead of 7.
+    const bool lie = d.scheme == WH_SCHEME_LIE;
+    if (!first) WH_TRY(odm(e, wh::kOdmJoin, 1.0, 1.0, false, s));
+    if (lie) {
+      if (first) WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
+    } else {
+      WH_TRY(psweep(e, first ? wh::kScaleOnLoad : wh::kTileScale, 0.5, 0, s));
+      WH_TRY(xsweep(e, 0, s));
+    }
+    WH_TRY(psweep(e, wh::kRecStep | (lie && !first ? wh::kTileScale : 0), lie ? 1.0 : 0.5, 0, s));
+    WH_TRY(odm_channels(e, !first, false, s));
   } else if (d.scheme == WH_SCHEME_LIE && e->gp()) {
     WH_TRY(gpshift(e, first ? 0 : wh::kTileScale, s));
     WH_TRY(xsweep(e, wh::kScaleOnLoad, s));
@@ -1089,6 +1115,11 @@ int ensemble_run(wh_ensemble* e, void* const* states, int first_step, int n_step
     } else {
       WH_TRY(graph_pays(e->graph_chunk, use_graph, n_steps - 1) ? run_graph(e, n_steps - 1, s)
                                                                    : iterations(e, n_steps - 1, false, false, s));
+    }
+    if (e->odm() && !e->gp()) {  // the last iteration's odm_back and observables
+      WH_TRY(odm(e, wh::kOdmBack, 1.0, 1.0, false, s));
+      WH_LAUNCH(wh::launch_colsum(storage_code(prec), md, e->work_colsum.buf.as<unsigned>(), e->work_colsum.n, s),
+                "colsum");
     }
     if (tiles_pending(e)) WH_TRY(reduce(e, renorm_flag(e), 1, 0, 1, true, s));
   }

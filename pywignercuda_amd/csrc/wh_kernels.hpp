@@ -38,13 +38,17 @@ enum SweepFlags {
   kColPart = 32,     // x sweep: partial column sums (Gross-Pitaevskii density after K)
   kConj = 64,        // x sweep: conjugated kinetic multiplier (adjoint step)
   kTilePart = 128,   // p sweep (requires kColSums): each tile writes its 12 observable partial sums
-  kTileScale = 256,  // x sweep, Gross-Pitaevskii shift: the pending factor from the previous p sweep's tile partials;
+  kRecStep = 2048,   // p sweep: copy the time index to rec_step (ODM steps, which write no tile partials)
+  kTileScale = 256,  // x sweep, Gross-Pitaevskii shift, p sweep behind an ODM join: the pending factor from the previous p sweep's tile partials;
                      // the member's record item writes the record row and the factor (no
                      // reduce launch between the sweeps)
   kProbSq = 1024,    // Gross-Pitaevskii shift: tile 0 records dX sum rho^2
   kStepArg = 512,    // p sweep: the time index is step_add itself (single-sweep entry points),
                      // not the device counter
 };
+
+// sweeps of the ODM dissipator (wh_odm.hip)
+enum OdmKind { kOdmX, kOdmP, kOdmBack, kOdmJoin };
 
 constexpr int kTileObs = 12;  // observable partials per tile
 constexpr int kRecordTile = 0xffff;  // x work item that forms a member's record (kTileScale), no row tile

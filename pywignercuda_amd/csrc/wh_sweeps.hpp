@@ -329,12 +329,14 @@ __device__ __forceinline__ cplx<double> tile_scale(const SweepArgs& a, CMember& 
 // The record item of a member (one block of a kTileScale launch, beside the row tiles so that no
 // row waits for it): all 12 sums, the record row and the factor; that of member 0 advances the
 // step index.
-template <int BLOCK>
+// AFTER_P: the iteration's p sweep has run (ODM steps, whose join advances the index): the record
+// is that of the index before the last p sweep's.
+template <int BLOCK, bool AFTER_P = false>
 __device__ __forceinline__ void record_item(const SweepArgs& a, CMember& m, double* red) {
   constexpr int kWaves = BLOCK / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ntiles = tile_count(a, m);
-  const int rstep = *cmem(a.rec_step);  // issued with the partial loads
+  const int rstep = *cmem(a.rec_step) - (AFTER_P ? 1 : 0);  // issued with the partial loads
   double r[12];
 #pragma unroll
   for (int k = 0; k < 12; ++k) r[k] = 0.0;
@@ -358,7 +360,7 @@ __device__ __forceinline__ void record_item(const SweepArgs& a, CMember& m, doub
   }
   if (tid == 0) {
     write_record(m, r, a.fin_renorm, a.fin_record, rstep);
-    if (first_member(a, m)) *gmem(a.step) = rstep + 1;
+    if (!AFTER_P && first_member(a, m)) *gmem(a.step) = rstep + 1;
   }
 }
 
@@ -367,6 +369,20 @@ __device__ __forceinline__ void record_item(const SweepArgs& a, CMember& m, doub
 // exp(-i a m_s), a = dt*dlambda*(k_c0 + k_c1 p), m_s = t + js*TT with
 // js = j (j < R/2) or j - R; computed as E_t * Z^js, E_t = exp(-i a t),
 // Z = exp(-i a TT): two sincos per lane instead of R.
+template <typename T, int R, int TT>
+__device__ __forceinline__ void kinetic_apply(cplx<T> (&v)[R], CMember& m, int t, cplx<double> Et, cplx<double> Z1) {
+  cplx<double> Zp[R / 2 + 1];  // Z^0 .. Z^(R/2)
+  Zp[0] = {1.0, 0.0};
+  Zp[1] = Z1;
+#pragma unroll
+  for (int k = 2; k <= R / 2; ++k) Zp[k] = cmul(Zp[k / 2], Zp[k - k / 2]);
+#pragma unroll
+  for (int j = 0; j < R; ++j) v[j] = apply(v[j], cmul(Et, j < R / 2 ? Zp[j] : cplx<double>{Zp[R - j].x, -Zp[R - j].y}));
+  if (m.lambda_decay) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.lambda_decay)[t + j * TT], 0.0});
+  }
+}
 template <typename S, typename T, int N, int R, int BLOCK, bool TP, typename E>
 __device__ __forceinline__ void xsweep_body(const SweepArgs& a, CMember& m, int tile,
                                             cplx<E>* lds) {
@@ -426,17 +442,7 @@ __device__ __forceinline__ void xsweep_body(const SweepArgs& a, CMember& m, int 
   }
   if (a.kin_linear) {
     Et = cmul(Et, g);
-    cplx<double> Zp[R / 2 + 1];  // Z^0 .. Z^(R/2)
-    Zp[0] = {1.0, 0.0};
-    Zp[1] = Z1;
-#pragma unroll
-    for (int k = 2; k <= R / 2; ++k) Zp[k] = cmul(Zp[k / 2], Zp[k - k / 2]);
-#pragma unroll
-    for (int j = 0; j < R; ++j) v[j] = apply(v[j], cmul(Et, j < R / 2 ? Zp[j] : cplx<double>{Zp[R - j].x, -Zp[R - j].y}));
-    if (m.lambda_decay) {
-#pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.lambda_decay)[t + j * TT], 0.0});
-    }
+    kinetic_apply<T, R, TT>(v, m, t, Et, Z1);
   } else {
     const double hh = a.hbar_half;
 #pragma unroll
@@ -631,6 +637,8 @@ struct PSweep {
 // LDS bytes past the transform arrays of a p-sweep block: per-column sums, then the
 // per-column observable terms (<= 64 columns)
 constexpr int kPTailBytes = 64 * 12 * 8;
+constexpr int kPTailRed = 64 * 11 * 8;  // the last 512 bytes: tile_scale's sums (two per wave)
+static_assert(64 * kNCol * 8 <= kPTailRed, "behind the column sums");
 
 // Lanes: the load layout (column cl = tid % C, team index tl = tid / C) makes every
 // global load and store instruction cover rows of C consecutive columns.  With wave
@@ -677,6 +685,8 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
       th[j] = T(gmem(m.theta_host)[tc + j * TT] * (1.0 / N));
     }
   }
+  TilePartials part{0.0, 0.0};
+  if (a.flags & kTileScale) part = tile_partials<BLOCK>(a, m);
   ColumnHost host{0.0, 0.0, 0.0};
   if (a.flags & kTilePart) host = column_host(m, tile * C + tid % C);
   cplx<T> v[R];
@@ -711,6 +721,12 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
       for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.theta_decay)[tc + j * TT], 0.0});
     }
   };
+  if (a.flags & kTileScale) {  // behind an ODM join: its partials give the pending factor
+    const cplx<double> f = tile_scale<BLOCK>(
+        a, m, part, reinterpret_cast<double*>(reinterpret_cast<char*>(lds + lds_elems<BLOCK, R>()) + kPTailRed));
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = apply(v[j], f);
+  }
   if constexpr (CL && !kEarly) {  // in flight while potential() evaluates its multipliers
     const int t = opaque_v(tc);
 #pragma unroll
@@ -844,6 +860,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
 #pragma unroll
   for (int j = 0; j < R; ++j) store_cached(at_off(W, soff + unsigned(j) * jstride), to_arith<S>(v[j]));
   if (a.flags & kTilePart) write_tile_partial<C>(a, m, tile, csum, host, step - a.step_add);
+  if ((a.flags & kRecStep) && tid == 0 && tile == 0 && first_member(a, m)) *gmem(a.rec_step) = step - a.step_add;
 }
 
 // ------------------------------------------------------------------ Gross-Pitaevskii shift
