@@ -30,8 +30,8 @@ hipError_t launch_xsweep_f64(int variant, const SweepArgs& a, int nwork, hipStre
 hipError_t launch_xsweep_f32(int variant, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_psweep_f64(int variant, bool cl, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_psweep_f32(int variant, bool cl, const SweepArgs& a, int nwork, hipStream_t s);
-hipError_t launch_expr_table(const Member* members, int member, int cells, int depth, const int* step,
-                             int step_add, int use_arg, int ntables, double hbar_half, hipStream_t s);
+hipError_t launch_expr_table(const Member* members, int member, int X, int P, int depth, const int* step,
+                             int step_add, int use_arg, double hbar_half, hipStream_t s);
 hipError_t launch_gpshift(const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_colsum(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s);
 hipError_t launch_observe_noalloc(int prec, Member m, hipStream_t s);
@@ -621,7 +621,7 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
       if (md.pot_deg == WH_POT_TABLE) {
         WH_TRY(b->pot_dv.upload(md.pot_dv, X * P * sizeof(double)));
       } else {
-        // two [P][X] tables, filled on the device before each p sweep (time index, next index)
+        // two [P][X] tables, filled on the device before the p sweeps (even and odd time indices)
         WH_TRY(b->pot_expr.upload(md.pot_expr, size_t(md.pot_expr_len) * 2 * sizeof(double)));
         WH_TRY(b->pot_dv.alloc(2 * X * P * sizeof(double)));
       }
@@ -826,14 +826,14 @@ int psweep(wh_ensemble* e, int flags, double frac, int step_add, hipStream_t s) 
   a.work = wl.buf.as<unsigned>();
   a.ntiles = e->n == 1 ? wl.n : 0;
   if (e->expr) {
-    // expression-program members: their [P][X] tables at the time index this sweep reads
-    // (and the next one for the merged Strang half step)
+    // expression-program members: their [P][X] table at the time index this sweep reads; for the
+    // merged Strang half steps that of the next index (the sweep before left this one's)
     const bool arg = (flags & wh::kStepArg) != 0;
     for (int i = 0; i < e->n; ++i) {
       const wh::Member& m = e->mem[i];
       if (m.pot_expr_len <= 0) continue;
-      WH_LAUNCH(wh::launch_expr_table(e->mem_dev.as<wh::Member>(), i, m.X * m.P, m.pot_expr_depth,
-                                      e->step.as<int>(), step_add, arg ? 1 : 0, (flags & wh::kMerge) ? 2 : 1,
+      WH_LAUNCH(wh::launch_expr_table(e->mem_dev.as<wh::Member>(), i, m.X, m.P, m.pot_expr_depth,
+                                      e->step.as<int>(), step_add + ((flags & wh::kMerge) ? 1 : 0), arg ? 1 : 0,
                                       a.hbar_half, s),
                 "expr_table");
     }

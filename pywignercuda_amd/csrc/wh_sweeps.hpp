@@ -487,13 +487,16 @@ struct PSweep {
   using View = std::conditional_t<kWave, LdsRow<E>, LdsStrided<E, C>>;
   using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
 
+  __device__ __forceinline__ static size_t table_offset(CMember& m, int step) {
+    return (m.pot_expr_len > 0 && (step & 1)) ? size_t(m.X) * size_t(m.P) : 0;
+  }
   // potential step multiplier of time index `step` (expPotential; GP phase optional),
   // times the real factor `scale` (the 1/N of the inverse transform that follows).
-  // tab: which [P][X] table a member with an expression program reads (0: time index `step`,
-  // 1: `step` + 1, the merged Strang half step; expr_table_kernel fills them before the sweep)
+  // A member with an expression program reads slot step % 2 of its two [P][X] tables
+  // (expr_table_kernel fills them before the sweep).
   __device__ __forceinline__ static void potential(cplx<T> (&v)[R], const SweepArgs& a,
                                                    CMember& m, int t_in, int col_in, int step,
-                                                   double scale, int tab) {
+                                                   double scale) {
     // opaque lane indices: recomputing theta and x -/+ hbar theta/2 per call is cheaper
     // than keeping them live across the transforms between two calls
     const int t = opaque_v(t_in), col = opaque_v(col_in);
@@ -542,7 +545,7 @@ struct PSweep {
         if (m.pot_deg >= 0) {
           phi = bopp(hd * double(fidx(i, N)));
         } else {
-          const size_t toff = (tab && m.pot_expr_len > 0) ? size_t(m.X) * size_t(m.P) : 0;
+          const size_t toff = table_offset(m, step);
           phi = a.vphase * gmem(m.pot_dv)[toff + size_t(i) * m.X + col];
         }
         if (gp) phi -= a.gp_phase * gmem(m.G)[size_t(i) * m.X + col];
@@ -562,11 +565,11 @@ struct PSweep {
     return m.pot_deg >= 0 || !(a.flags & kGP);
   }
   __device__ __forceinline__ static void mul_loads(MulLoads& l, const SweepArgs& a, CMember& m, int t, int col,
-                                                   int tab) {
+                                                   int step) {
     l.mask = 1.0;
     if (m.xmask) l.mask = gmem(m.xmask)[col];
     if (m.pot_deg < 0 || (a.flags & kGP)) {
-      const size_t toff = (m.pot_deg < 0 && tab && m.pot_expr_len > 0) ? size_t(m.X) * size_t(m.P) : 0;
+      const size_t toff = m.pot_deg < 0 ? table_offset(m, step) : 0;
       const gptr<const double> src = gmem(m.pot_deg < 0 ? m.pot_dv : const_cast<const double*>(m.G)) + toff;
 #pragma unroll
       for (int j = 0; j < R; ++j) l.tab[j] = src[size_t(t + j * TT) * m.X + col];
@@ -673,7 +676,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   constexpr bool kEarly = R <= 8 && !TP;
   const bool early = kEarly && PS::early(a, m);
   typename PS::MulLoads ml;
-  if (early) PS::mul_loads(ml, a, m, tc, col, 0);
+  if (early) PS::mul_loads(ml, a, m, tc, col, step);
   // the friction tables and the host values of one column per lane: in registers when the state is
   T sg[CL ? R : 1], th[CL ? R : 1];
   double decay[CL ? R : 1];  // (a plan with friction always has the table)
@@ -735,7 +738,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   if (early)
     PS::multiply(v, M);
   else
-    PS::potential(v, a, m, tc, col, step, 1.0 / N, 0);
+    PS::potential(v, a, m, tc, col, step, 1.0 / N);
   theta_decay();
   team_fft<T, N, R, +1, View, Sync>(v, tc, view_c, twsrc);
 
@@ -832,14 +835,14 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   if (a.flags & kMerge) {
     if (early && !PS::same_multipliers(m, step)) {
       const int t = opaque_v(tc), c = opaque_v(col);
-      PS::mul_loads(ml, a, m, t, c, 1);
+      PS::mul_loads(ml, a, m, t, c, step + 1);
       PS::multipliers(M, ml, a, m, t, c, step + 1, 1.0 / N);
     }
     team_fft<T, N, R, -1, View, Sync>(v, tc, view_c, twsrc);
     if (early)
       PS::multiply(v, M);
     else
-      PS::potential(v, a, m, tc, col, step + 1, 1.0 / N, 1);
+      PS::potential(v, a, m, tc, col, step + 1, 1.0 / N);
     theta_decay();
     team_fft<T, N, R, +1, View, Sync>(v, tc, view_c, twsrc);
   }
