@@ -276,6 +276,18 @@ int wh_wigner2d_potential(wh_wigner2d* plan, void* W, int step, int fused, void*
  */
 int wh_wigner2d_adjoint_step(wh_wigner2d* plan, void* Lambda, const void* W_next, int step, double* grad,
                              void* stream);
+
+/* n_steps undamped Lie steps out of W_in into W_out (which may be W_in), time indices first_step..,
+ * without observables or normalisation: two launches per step.  Lie scheme without damping or
+ * Gross-Pitaevskii. */
+int wh_wigner2d_steps(wh_wigner2d* plan, const void* W_in, void* W_out, int first_step, int n_steps, void* stream);
+
+/* Backward pass over n_steps steps from the state W_first before step first_step: recomputes the
+ * states after each step into `states` ([n_steps][P][X], scratch of the caller), then carries
+ * Lambda back through the steps; grads[k][9] (device) <- dL/da(first_step + k).  Restrictions as
+ * wh_wigner2d_adjoint_step. */
+int wh_wigner2d_adjoint_segment(wh_wigner2d* plan, const void* W_first, void* states, void* Lambda, int first_step,
+                                int n_steps, double* grads, void* stream);
 /* Observables of W (FFT.py:1857-1878) into one row of WH_NOBS doubles (device). */
 int wh_wigner2d_observe(wh_wigner2d* plan, const void* W, double* obs_row, void* stream);
 

@@ -226,6 +226,8 @@ def _declare(lib):
         "wh_wigner2d_observe_noalloc": ([POINTER(ObserveDesc), vp, vp, vp], ip),
         "wh_wigner2d_ensemble": ([vp], vp),
         "wh_wigner2d_adjoint_step": ([vp, vp, vp, ip, vp, vp], ip),
+        "wh_wigner2d_steps": ([vp, vp, vp, ip, ip, vp], ip),
+        "wh_wigner2d_adjoint_segment": ([vp, vp, vp, vp, ip, ip, vp, vp], ip),
         "wh_ensemble_create": ([POINTER(EnsembleDesc), POINTER(MemberDesc), ip, POINTER(vp)], ip),
         "wh_ensemble_destroy": ([vp], ip),
         "wh_ensemble_run": ([vp, POINTER(vp), ip, ip, vp, ip, ip, vp], ip),

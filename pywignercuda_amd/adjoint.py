@@ -7,11 +7,11 @@
 the last row for later steps); the result is Re W after n_steps (float64, [P, X]).
 Gradients flow to coef_table (dL/da_k(n)) and to W0.
 
-Forward: the fused run, keeping the state every `checkpoint_every` steps.
+Forward: the sweeps without observables, keeping the state every `checkpoint_every` steps.
 Backward: per segment, last to first, the forward states are recomputed from the
 segment's checkpoint (two single-sweep launches per step) and the adjoint state is carried
-back through the reverse-time step with conjugated phases (wh_wigner2d_adjoint_step), which also
-accumulates dL/da_k(n).  Memory: n_steps/K checkpoints + K states.
+back through the reverse-time steps with conjugated phases, which also give dL/da_k(n)
+(wh_wigner2d_adjoint_segment: one call per segment).  Memory: n_steps/K checkpoints + K states.
 
 The reference has no gradients; there is no reference counterpart to this module.
 """
@@ -42,14 +42,20 @@ def _make_function():
         def forward(ctx, coef_table, W0, prop, n_steps, K):
             prop.set_potential(coef_table.detach())
             W = W0.detach().to(prop.dtype).contiguous().clone()
-            ckpts = [W.clone()]
+            ckpts = [W]
             done = 0
             while done < n_steps:
                 n = min(K, n_steps - done)
-                prop.run(W, n, first_step=done, normalize_initial=False, use_graph=True)
+                if prop.plain:
+                    # out of the checkpoint into the next one, without observables
+                    W = torch.empty_like(W)
+                    prop.steps(ckpts[-1], W, n, first_step=done)
+                else:
+                    W = W.clone()
+                    prop.run(W, n, first_step=done, normalize_initial=False, use_graph=True)
                 done += n
                 if done < n_steps:
-                    ckpts.append(W.clone())
+                    ckpts.append(W)
             ctx.prop, ctx.n_steps, ctx.K = prop, n_steps, K
             ctx.rows = coef_table.shape[0]
             ctx.ckpts = ckpts
@@ -62,20 +68,14 @@ def _make_function():
             Lam = grad_real.to(prop.device).to(prop.dtype).contiguous().clone()
             grads = torch.zeros((n_steps, WH_MAX_DEG + 1), dtype=torch.float64, device=prop.device)
             nseg = len(ctx.ckpts)
+            states = torch.empty((min(K, n_steps), prop.P, prop.X), dtype=prop.dtype, device=prop.device)
             for s in reversed(range(nseg)):
                 n0 = s * K
                 n = min(K, n_steps - n0)
-                W = ctx.ckpts[s].clone()
-                traj = []
-                for k in range(n):
-                    # one Lie step as two single sweeps (bit-identical to run(W, 1) without
-                    # renormalisation, without its observable launches)
-                    prop.kinetic(W)
-                    prop.potential(W, n0 + k, fused=False)
-                    traj.append(W.clone())
-                for k in reversed(range(n)):
-                    prop.adjoint_step(Lam, traj[k], n0 + k, grads[n0 + k])
-                del traj
+                # one call: the segment's states out of its checkpoint (the sweeps of the forward
+                # pass), then the adjoint steps
+                if n > 0:
+                    prop.adjoint_segment(ctx.ckpts[s], states[:n], Lam, n0, grads[n0:n0 + n])
             # coefficient rows: row r receives the steps that read it (row = min(step, rows - 1))
             rows = ctx.rows
             dcoef = torch.zeros((rows, WH_MAX_DEG + 1), dtype=torch.float64, device=prop.device)

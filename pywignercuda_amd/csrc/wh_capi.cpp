@@ -50,9 +50,11 @@ hipError_t launch_set_scale(const Member* members, int nmembers, double re, doub
 hipError_t launch_fft_axis(int prec, int columns, int N, int dir, void* d, int batch, int norm,
                            const void* tw_hi, const void* tw_lo, hipStream_t s);
 int fft_cols_batch_multiple(int prec, int N);
-hipError_t launch_adj_psweep(int prec, const SweepArgs& a, int nwork, hipStream_t s);
-hipError_t launch_grad_reduce(const Member* members, int nmembers, double* grad, double scale, hipStream_t s);
+hipError_t launch_adj_psweep(int prec, const SweepArgs& a, const void* W_next, double* gcols, hipStream_t s);
+hipError_t launch_grad_reduce(const Member* members, const double* gcols, int nsteps, double* grad, double scale,
+                              hipStream_t s);
 int adj_cols(int P);
+size_t adj_moments(int X);
 int odm_rows_per_tile(int X);
 int odm_cols_per_tile(int P);
 int odm_radix();
@@ -402,7 +404,7 @@ struct wh_ensemble {
   // (a tile spans block * R / P columns, which differs between the two variant tables;
   // a CL plan also runs plain p sweeps: the merged Strang first half step, Strang + GP
   // V/2, the unfused single V step)
-  WorkList work_x, work_p, work_pcl, work_colsum, work_scale, work_gp, work_adj, work_odm_x, work_odm_p;
+  WorkList work_x, work_p, work_pcl, work_colsum, work_scale, work_gp, work_odm_x, work_odm_p;
   wh::SweepVariant built_x{}, built_p{}, built_pcl{};  // the variants each list was cut for
   DevBuf step, done, gcols;
   hipStream_t capture_stream = nullptr;
@@ -798,13 +800,16 @@ bool same_variant(const wh::SweepVariant& a, const wh::SweepVariant& b) {
   return a.R == b.R && a.block == b.block && a.tp == b.tp;
 }
 
-int xsweep(wh_ensemble* e, int flags, hipStream_t s) {
+// src, dst: the states read and written (plans of one member; null: the bound state)
+int xsweep(wh_ensemble* e, int flags, hipStream_t s, const void* src = nullptr, void* dst = nullptr) {
   // the work list's tiles are cut for the variant launched over it
   if (!same_variant(wh::kXVariants[e->xvar], e->built_x))
     return fail(WH_INTERNAL_ERROR, "x work list cut for another variant");
   wh::SweepArgs a = sweep_args(e, flags, 1.0, 0);
   a.work = e->work_x.buf.as<unsigned>();
   a.ntiles = e->n == 1 ? e->work_x.n - 1 : 0;  // the record item is the last
+  a.W_src = src;
+  a.W_dst = dst;
   WH_LAUNCH(e->d.precision == WH_C128      ? wh::launch_xsweep_f64(e->xvar, a, e->work_x.n, s)
             : e->d.precision == WH_C64_WIDE ? wh::launch_xsweep_f32w(e->xvar, a, e->work_x.n, s)
                                       : wh::launch_xsweep_f32(e->xvar, a, e->work_x.n, s),
@@ -812,8 +817,9 @@ int xsweep(wh_ensemble* e, int flags, hipStream_t s) {
   return WH_SUCCESS;
 }
 
-int psweep(wh_ensemble* e, int flags, double frac, int step_add, hipStream_t s) {
+int psweep(wh_ensemble* e, int flags, double frac, int step_add, hipStream_t s, void* dst = nullptr) {
   wh::SweepArgs a = sweep_args(e, flags, frac, step_add);
+  a.W_dst = dst;
   const bool cl = (flags & wh::kCL) != 0;
   if (cl && !e->cl()) return fail(WH_INTERNAL_ERROR, "Caldeira-Leggett p sweep on a plan without friction");
   // the plain and the Caldeira-Leggett p variants have their own work lists (their tiles
@@ -1304,6 +1310,71 @@ extern "C" int wh_ensemble_set_potential(wh_ensemble* e, int member, const doubl
   return sync_table(e, changed, s);
 }
 
+namespace {
+// The undamped Lie step as two sweeps out of and into given states, without observables.
+int plain_step(wh_ensemble* e, const void* src, void* dst, int step, hipStream_t s) {
+  WH_TRY(xsweep(e, 0, s, src, dst));
+  return psweep(e, wh::kStepArg, 1.0, step, s, dst);
+}
+int check_plain(const wh_ensemble* e, const char* who) {
+  if (e->d.scheme != WH_SCHEME_LIE || e->cl() || e->odm() || e->gp())
+    return fail(WH_INVALID_VALUE, "%s covers the Lie scheme without damping or Gross-Pitaevskii", who);
+  return WH_SUCCESS;
+}
+int check_adjoint(wh_ensemble* e) {
+  WH_TRY(check_plain(e, "the adjoint step"));
+  if (e->mem[0].pot_deg < 0)
+    return fail(WH_INVALID_VALUE, "the adjoint step needs V as polynomial coefficients (gradients are per coefficient)");
+  if (e->d.precision == WH_C64_WIDE)
+    return fail(WH_INVALID_TYPE, "the adjoint step runs on WH_C128 or WH_C64 states");
+  const wh::Member& m = e->mem[0];
+  const int cols = wh::adj_cols(m.P);
+  if (cols < 1 || cols > 64 || m.X % cols != 0 || m.P < 128)
+    return fail(WH_INVALID_SIZE, "adjoint sweep does not fit a %d x %d grid", m.P, m.X);
+  return WH_SUCCESS;
+}
+// Lambda <- U_step^dagger Lambda; the step's column moments to slot k of the plan's buffer.
+int adjoint_sweeps(wh_ensemble* e, void* Lambda, const void* W_next, int step, int k, hipStream_t s) {
+  const wh::Member& m = e->mem[0];
+  wh::SweepArgs a = sweep_args(e, 0, 1.0, step);
+  a.ntiles = m.X / wh::adj_cols(m.P);
+  a.W_dst = Lambda;
+  WH_LAUNCH(wh::launch_adj_psweep(e->d.precision, a, W_next, e->gcols.as<double>() + size_t(k) * wh::adj_moments(m.X), s),
+            "adj_psweep");
+  return xsweep(e, wh::kConj, s, Lambda, Lambda);
+}
+// The gradient rows of n adjoint steps from their moments.
+int adjoint_reduce(wh_ensemble* e, double* grads, int n, hipStream_t s) {
+  const wh::SweepArgs a = sweep_args(e, 0, 1.0, 0);
+  WH_LAUNCH(wh::launch_grad_reduce(e->mem_dev.as<wh::Member>(), e->gcols.as<double>(), n, grads,
+                                   a.vphase / double(e->mem[0].P), s),
+            "grad_reduce");
+  return WH_SUCCESS;
+}
+// The plan's moment buffer holds n steps (it grows; a growth waits for the stream's work on the
+// old one).
+int adjoint_room(wh_ensemble* e, int n, hipStream_t s) {
+  const size_t bytes = size_t(n) * wh::adj_moments(e->mem[0].X) * sizeof(double);
+  if (e->gcols.bytes >= bytes) return WH_SUCCESS;
+  if (e->gcols.p) WH_HIP(hipStreamSynchronize(s), "sync");
+  return e->gcols.alloc(bytes);
+}
+}  // namespace
+
+extern "C" int wh_wigner2d_steps(wh_wigner2d* p, const void* W_in, void* W_out, int first_step, int n_steps,
+                                 void* stream) {
+  if (!p) return fail(WH_INVALID_PLAN, "wh_wigner2d_steps: plan is NULL");
+  if (!W_in || !W_out || first_step < 0 || n_steps < 1)
+    return fail(WH_INVALID_VALUE, "wh_wigner2d_steps: W_in %p W_out %p first_step %d n_steps %d", W_in, W_out, first_step,
+                n_steps);
+  wh_ensemble* e = p->e;
+  WH_TRY(check_plain(e, "wh_wigner2d_steps"));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (e->table_dirty) WH_TRY(sync_table(e, true, s));
+  for (int k = 0; k < n_steps; ++k) WH_TRY(plain_step(e, k == 0 ? W_in : W_out, W_out, first_step + k, s));
+  return WH_SUCCESS;
+}
+
 extern "C" int wh_wigner2d_adjoint_step(wh_wigner2d* p, void* Lambda, const void* W_next, int step, double* grad,
                                         void* stream) {
   if (!p) return fail(WH_INVALID_PLAN, "wh_wigner2d_adjoint_step: plan is NULL");
@@ -1311,34 +1382,31 @@ extern "C" int wh_wigner2d_adjoint_step(wh_wigner2d* p, void* Lambda, const void
     return fail(WH_INVALID_VALUE, "wh_wigner2d_adjoint_step: Lambda %p W_next %p grad %p step %d", Lambda, W_next,
                 (void*)grad, step);
   wh_ensemble* e = p->e;
-  if (e->d.scheme != WH_SCHEME_LIE || e->cl() || e->odm() || e->gp())
-    return fail(WH_INVALID_VALUE, "the adjoint step covers the Lie scheme without damping or Gross-Pitaevskii");
-  if (e->mem[0].pot_deg < 0)
-    return fail(WH_INVALID_VALUE, "the adjoint step needs V as polynomial coefficients (gradients are per coefficient)");
-  if (e->d.precision == WH_C64_WIDE)
-    return fail(WH_INVALID_TYPE, "the adjoint step runs on WH_C128 or WH_C64 states");
+  WH_TRY(check_adjoint(e));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  wh::Member& m = e->mem[0];
-  if (!e->work_adj.n) {
-    const int cols = wh::adj_cols(m.P);
-    if (cols < 1 || cols > 64 || m.X % cols != 0 || m.P < 128)
-      return fail(WH_INVALID_SIZE, "adjoint sweep does not fit a %d x %d grid", m.P, m.X);
-    std::vector<unsigned> w;
-    for (int t = 0; t < m.X / cols; ++t) w.push_back(unsigned(t));
-    WH_TRY(e->work_adj.upload(w));
-    WH_TRY(e->gcols.alloc(size_t(m.X) * (wh::kMaxDeg + 1) * sizeof(double)));
-  }
-  const bool changed = m.W != Lambda || m.W2 != W_next || m.gcols != e->gcols.as<double>();
-  m.W = Lambda;
-  m.W2 = W_next;
-  m.gcols = e->gcols.as<double>();
-  WH_TRY(sync_table(e, changed, s));
-  WH_LAUNCH(wh::launch_set_int(e->step.as<int>(), step, s), "set_step");
-  wh::SweepArgs a = sweep_args(e, 0, 1.0, 0);
-  a.work = e->work_adj.buf.as<unsigned>();
-  WH_LAUNCH(wh::launch_adj_psweep(e->d.precision, a, e->work_adj.n, s), "adj_psweep");
-  WH_LAUNCH(wh::launch_grad_reduce(e->mem_dev.as<wh::Member>(), 1, grad, a.vphase / double(m.P), s), "grad_reduce");
-  return xsweep(e, wh::kConj, s);
+  if (e->table_dirty) WH_TRY(sync_table(e, true, s));
+  WH_TRY(adjoint_room(e, 1, s));
+  WH_TRY(adjoint_sweeps(e, Lambda, W_next, step, 0, s));
+  return adjoint_reduce(e, grad, 1, s);
+}
+
+extern "C" int wh_wigner2d_adjoint_segment(wh_wigner2d* p, const void* W_first, void* states, void* Lambda,
+                                           int first_step, int n_steps, double* grads, void* stream) {
+  if (!p) return fail(WH_INVALID_PLAN, "wh_wigner2d_adjoint_segment: plan is NULL");
+  if (!W_first || !states || !Lambda || !grads || first_step < 0 || n_steps < 1)
+    return fail(WH_INVALID_VALUE, "wh_wigner2d_adjoint_segment: W_first %p states %p Lambda %p grads %p first_step %d "
+                "n_steps %d", W_first, states, Lambda, (void*)grads, first_step, n_steps);
+  wh_ensemble* e = p->e;
+  WH_TRY(check_adjoint(e));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (e->table_dirty) WH_TRY(sync_table(e, true, s));
+  WH_TRY(adjoint_room(e, n_steps, s));
+  const size_t bytes = size_t(e->mem[0].X) * size_t(e->mem[0].P) * state_bytes(e->d.precision);
+  const auto state = [&](int k) { return static_cast<char*>(states) + size_t(k) * bytes; };
+  for (int k = 0; k < n_steps; ++k)
+    WH_TRY(plain_step(e, k == 0 ? W_first : state(k - 1), state(k), first_step + k, s));
+  for (int k = n_steps - 1; k >= 0; --k) WH_TRY(adjoint_sweeps(e, Lambda, state(k), first_step + k, k, s));
+  return adjoint_reduce(e, grads, n_steps, s);
 }
 
 extern "C" int wh_wigner2d_observe(wh_wigner2d* p, const void* W, double* obs_row, void* stream) {

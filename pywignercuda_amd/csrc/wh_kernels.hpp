@@ -89,9 +89,6 @@ struct Member {
   const double* odm_th;        // [2][P] cos(hbar theta), sin(hbar theta) (host theta)
   void* odm_s;                 // [2][P][X] scratch in the state precision (lambda picture)
   double odm_c, odm_sign;      // 2 gamma dt; +1 damping, -1 pumping
-  // adjoint step (single-grid plans): forward state after the step, gradient column sums
-  const void* W2;              // [P][X] W_{n+1}
-  double* gcols;               // [X][kMaxDeg+1]
   // V(t, x) as an expression program (pot_deg = kPotExpr): (op, value) pairs, t = step * pot_t_step
   const double* pot_expr;
   int pot_expr_len, pot_expr_depth;  // ops; the deepest stack the program reaches
@@ -116,6 +113,10 @@ struct SweepArgs {
   const unsigned* work;  // (member << 16) | tile, one per block
   int ntiles;            // > 0: a plan of one member with that many tiles, the work item follows
                          // from the block index (one dependent load less in front of the sweep)
+  // single-sweep launches of plans of one member: the state that is read and the one that is
+  // written in place of the member's (null: the member's)
+  const void* W_src;
+  void* W_dst;
   int* step;             // device step counter (time index)
   int step_add;
   int flags;

@@ -94,6 +94,10 @@ template <typename T>
 __device__ __forceinline__ gptr<cplx<T>> at_off(gptr<cplx<T>> base, unsigned boff) {
   return reinterpret_cast<gptr<cplx<T>>>(reinterpret_cast<gptr<char>>(base) + boff);
 }
+template <typename T>
+__device__ __forceinline__ gptr<const cplx<T>> at_off(gptr<const cplx<T>> base, unsigned boff) {
+  return reinterpret_cast<gptr<const cplx<T>>>(reinterpret_cast<gptr<const char>>(base) + boff);
+}
 
 template <typename T>
 __device__ __forceinline__ cplx<T> mul_i(cplx<T> a, T s) { return {-s * a.y, s * a.x}; }
@@ -393,7 +397,8 @@ __device__ __forceinline__ void xsweep_body(const SweepArgs& a, CMember& m, int 
   // uniform member base + 32-bit per-lane byte offset (a state is at most 2048^2 x 16 B);
   // the store recomputes the offset from an opaque copy of the lane index, so that no
   // per-row address stays live (or is spilled) across the transforms
-  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(m.W));
+  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(a.W_dst ? a.W_dst : m.W));
+  const gptr<const cplx<S>> src = a.W_src ? gmem(reinterpret_cast<const cplx<S>*>(a.W_src)) : gptr<const cplx<S>>(W);
   const unsigned roff = (unsigned(row) * unsigned(N) + unsigned(t)) * unsigned(sizeof(cplx<S>));
   constexpr unsigned kJ = unsigned(TT * sizeof(cplx<S>));
   const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(m.twX_hi), reinterpret_cast<const cplx<T>*>(m.twX_lo)};
@@ -413,7 +418,7 @@ __device__ __forceinline__ void xsweep_body(const SweepArgs& a, CMember& m, int 
   }
   cplx<T> v[R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload(at_off(W, roff + unsigned(j) * kJ)));
+  for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload<S>(at_off(src, roff + unsigned(j) * kJ)));
   const auto twsrc = [&]() {
     if constexpr (kWave && !TP) {
       TwRegs<T, N, R> r;
@@ -661,7 +666,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   const int cc = kWave ? tid / TT : cl, tc = kWave ? tid % TT : tl;
   const int X = m.X;
   const int col = tile * C + cc;
-  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(m.W));
+  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(a.W_dst ? a.W_dst : m.W));
   const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(m.twP_hi), reinterpret_cast<const cplx<T>*>(m.twP_lo)};
   const View view_c{kWave ? lds + cc * LSZ : lds + cl};
   const int step = (a.flags & kStepArg) ? a.step_add : *cmem(a.step) + a.step_add;
@@ -689,7 +694,8 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
     }
   }
   TilePartials part{0.0, 0.0};
-  if (a.flags & kTileScale) part = tile_partials<BLOCK>(a, m);
+  const bool behind_join = !CL && (a.flags & kTileScale);  // an ODM join's partials give the pending factor
+  if (behind_join) part = tile_partials<BLOCK>(a, m);
   ColumnHost host{0.0, 0.0, 0.0};
   if (a.flags & kTilePart) host = column_host(m, tile * C + tid % C);
   cplx<T> v[R];
@@ -724,7 +730,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
       for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{gmem(m.theta_decay)[tc + j * TT], 0.0});
     }
   };
-  if (a.flags & kTileScale) {  // behind an ODM join: its partials give the pending factor
+  if (behind_join) {
     const cplx<double> f = tile_scale<BLOCK>(
         a, m, part, reinterpret_cast<double*>(reinterpret_cast<char*>(lds + lds_elems<BLOCK, R>()) + kPTailRed));
 #pragma unroll

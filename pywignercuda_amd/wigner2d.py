@@ -343,6 +343,8 @@ class Wigner2D(_PlanBase):
         self.scheme = scheme
         self.cl = damping == "CaldeiraLeggett" and gamma != 0.0
         self.gp = gp_coeff != 0.0
+        # a Lie step of two sweeps and nothing else
+        self.plain = scheme == "lie" and not self.gp and (damping not in ("CaldeiraLeggett", "ODM") or gamma == 0.0)
         t = _Tables(X, P, X_amp, P_amp, hbar, mass, dt, potential=potential, dpotential=dpotential,
                     scheme=scheme, D_theta=D_theta, D_lambda=D_lambda, gamma=gamma, damping=damping,
                     fp_damping=fp_damping, gp_coeff=gp_coeff, gp_rho_factor=gp_rho_factor, mask=mask,
@@ -389,6 +391,11 @@ class Wigner2D(_PlanBase):
         if W.dtype != self.dtype or not W.is_cuda or not W.is_contiguous() or tuple(W.shape) != (self.P, self.X):
             raise ValueError(f"state must be a contiguous {self.dtype} CUDA tensor of shape {(self.P, self.X)}")
 
+    def _check_rows(self, first_step, n_steps):
+        if self.time_table and first_step + n_steps + 1 >= self.pot_table.shape[0]:
+            raise ValueError(f"time-dependent potential table has {self.pot_table.shape[0]} rows; "
+                             f"need {first_step + n_steps + 2} (pass time_rows)")
+
     def set_variants(self, xvar=-1, pvar=-1, pclvar=-1):
         _lib.check(_lib.lib().wh_ensemble_set_variants(self._ens, int(xvar), int(pvar), int(pclvar)),
                    "wh_ensemble_set_variants")
@@ -400,9 +407,7 @@ class Wigner2D(_PlanBase):
         import torch
 
         self._check_state(W)
-        if self.time_table and first_step + n_steps + 1 >= self.pot_table.shape[0]:
-            raise ValueError(f"time-dependent potential table has {self.pot_table.shape[0]} rows; "
-                             f"need {first_step + n_steps + 2} (pass time_rows)")
+        self._check_rows(first_step, n_steps)
         if obs is None:
             obs = torch.zeros((n_steps + 1, WH_NOBS), dtype=torch.float64, device=W.device)
         _lib.check(_lib.lib().wh_wigner2d_run(self._plan, _lib.dptr(W), int(first_step), int(n_steps),
@@ -445,6 +450,31 @@ class Wigner2D(_PlanBase):
         _lib.check(_lib.lib().wh_wigner2d_adjoint_step(self._plan, _lib.dptr(Lam), _lib.dptr(W_next), int(step),
                                                        _lib.dptr(grad_row), _lib.current_stream_handle()),
                    "wh_wigner2d_adjoint_step")
+
+    def steps(self, W_in, W_out, n_steps: int, first_step: int = 0):
+        """n_steps Lie steps out of W_in into W_out (which may be W_in) without observables or
+        normalisation: the state that run(normalize_initial=False) gives without damping."""
+        self._check_state(W_in)
+        self._check_state(W_out)
+        self._check_rows(first_step, n_steps)
+        _lib.check(_lib.lib().wh_wigner2d_steps(self._plan, _lib.dptr(W_in), _lib.dptr(W_out), int(first_step),
+                                                int(n_steps), _lib.current_stream_handle()),
+                   "wh_wigner2d_steps")
+
+    def adjoint_segment(self, W_first, states, Lam, first_step: int, grads):
+        """Backward pass over len(states) steps from W_first (the state before step first_step):
+        states [n, P, X] is scratch for the states after each step, Lam is carried back in place,
+        grads ([n, 9] float64, device) receives dL/da of each step."""
+        n = int(states.shape[0])
+        self._check_state(W_first)
+        self._check_state(Lam)
+        self._check_state(states[0])
+        if not states.is_contiguous() or not grads.is_contiguous() or tuple(grads.shape) != (n, WH_MAX_DEG + 1):
+            raise ValueError(f"states must be contiguous and grads a contiguous [{n}, {WH_MAX_DEG + 1}] tensor")
+        _lib.check(_lib.lib().wh_wigner2d_adjoint_segment(self._plan, _lib.dptr(W_first), _lib.dptr(states),
+                                                          _lib.dptr(Lam), int(first_step), n, _lib.dptr(grads),
+                                                          _lib.current_stream_handle()),
+                   "wh_wigner2d_adjoint_segment")
 
     def observe(self, W):
         import torch
