@@ -70,7 +70,7 @@ hipError_t launch_dirac_mass_table(const DiracPlan* d, int cells, int depth, hip
 hipError_t launch_dirac_a_table(const DiracPlan* d, int cells, int depth, hipStream_t s);
 hipError_t launch_dirac_a_sum(const DiracPlan* d, int X, int depth, int state_add, hipStream_t s);
 hipError_t launch_dirac_finish(int prec, const DiracPlan* d, int P, hipStream_t s);
-int dirac_x_blocks(int prec, int X, int P);
+int dirac_x_blocks(int X, int P);
 int dirac_gp_blocks(int X, int P);
 int dirac_pg_blocks(int X, int P);
 hipError_t launch_dirac_pgeneral(int prec, bool cl, const DiracPlan* d, int nblocks, hipStream_t s);
@@ -1645,7 +1645,7 @@ extern "C" int wh_dirac_create(const wh_dirac_desc* desc, wh_dirac** out) {
   e->d = *desc;
   const auto& d = *desc;
   const size_t X = size_t(d.x_dim), P = size_t(d.p_dim);
-  e->xblocks = wh::dirac_x_blocks(d.precision, d.x_dim, d.p_dim);
+  e->xblocks = wh::dirac_x_blocks(d.x_dim, d.p_dim);
   e->pblocks = wh::dirac_p_blocks(d.x_dim, d.p_dim);
   if (e->xblocks < 1 || e->pblocks < 1) return fail(WH_INVALID_SIZE, "grid %zu x %zu", P, X);
   WH_TRY(make_twiddles(e->twx, d.x_dim, d.precision, d.gp_coeff != 0.0));

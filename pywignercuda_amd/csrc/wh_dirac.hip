@@ -36,39 +36,17 @@ namespace wh {
 
 namespace {
 
-// plane groups closed under the kinetic factor, ordered [r1 c1, r1 c2, r2 c1, r2 c2]
-__constant__ int kDiracGroups[4][4] = {{0, 3, 12, 15}, {1, 2, 13, 14}, {4, 7, 8, 11}, {5, 6, 9, 10}};
-
 __device__ __forceinline__ cplx<double> widen(cplx<double> v) { return v; }
 __device__ __forceinline__ cplx<double> widen(cplx<float> v) { return {double(v.x), double(v.y)}; }
 template <typename T>
 __device__ __forceinline__ cplx<T> narrow(cplx<double> v) { return {T(v.x), T(v.y)}; }
 
-// U(q) = cos(c dt s) - i sin(c dt s) (mh_c beta + q alpha_1) / s on one {r1, r2} block:
-// [[a, b], [b, d]] with a = C - i mh_c S/s, d = C + i mh_c S/s, b = -i q S/s; sgn = -1 gives
-// the dt -> -dt factor of P_minus_Lambda (= U(q)^dagger).
-struct Blk {
-  cplx<double> a, b, d;
-};
-// mass_on = 0: the KvN form (GPU_WignerDiracKvN2D_4x4.py:183-189), whose diagonal is cos(c dt s)
-// alone (s keeps the mass).
-__device__ __forceinline__ Blk kinetic_block(double q, double mh_c, double c_dt, double sgn, double mass_on = 1.0) {
-  const double s = sqrt(mh_c * mh_c + q * q);
-  double sn, cs;
-  sincos_fp64(c_dt * s, &sn, &cs);
-  sn *= sgn;
-  const double f = sn / s;
-  const double m = mass_on * mh_c * f;
-  return {{cs, -m}, {0.0, -q * f}, {cs, m}};
-}
-
-// Positive-energy projector Lambda_+(q) = 1/2 (1 + (m c^2 beta + c q alpha_1) / E) on one
-// {r1, r2} block (DiracElectronProjector / Filter_Kernel with sign +1, :674-760).
-__device__ __forceinline__ Blk projector_block(double q, double mc2, double c) {
-  const double e2 = 2.0 * sqrt(mc2 * mc2 + c * c * q * q);
-  return {{0.5 + mc2 / e2, 0.0}, {c * q / e2, 0.0}, {0.5 - mc2 / e2, 0.0}};
-}
-
+// The factors of one {r1, r2} block of spinor rows (left) or columns (right):
+//   kinetic    U(q) = cos(c dt s) - i sin(c dt s) (mh_c beta + q alpha_1) / s = [[a, b], [b, d]] with
+//              a = C - i mh_c S/s, d = C + i mh_c S/s, b = -i q S/s; the right side has the dt -> -dt
+//              factor of P_minus_Lambda (= U(q)^dagger)
+//   projector  Lambda_+(q) = 1/2 (1 + (m c^2 beta + c q alpha_1) / E) (DiracElectronProjector /
+//              Filter_Kernel with sign +1, :674-760)
 }  // namespace
 
 // ------------------------------------------------------------------ x sweep
@@ -76,34 +54,121 @@ __device__ __forceinline__ Blk projector_block(double q, double mc2, double c) {
 // :2500-2540, applied at :3636-3678): W <- Lambda_+(q1) W Lambda_+(q2) in the (p, lambda)
 // picture, q1,2 = p +/- lambda/2 (q1 = q2 = p in the KvN form, whose filter sets lambda = 0,
 // GPU_WignerDiracKvN2D_4x4.py:775), then the edge absorber that follows it; no pending factor.
-template <typename S, typename T, int N, int R, int BLOCK, bool FILTER = false>
-__device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int group, int tile, cplx<T>* lds) {
-  constexpr int TT = N / R, ROWS = BLOCK / TT;
-  constexpr int LSZ = Padded<N, R>::size;
-  const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
-  const int row = tile * ROWS + team;
-  const size_t plane = size_t(d.P) * size_t(d.X);
-  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(d.W)) + size_t(row) * N;
-  const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(d.twX_hi), reinterpret_cast<const cplx<T>*>(d.twX_lo)};
-  LdsRow<T> view{lds + team * LSZ};
-  // a team inside one wave (radix 8 up to N = 512): wave-local exchanges
-  using Sync = std::conditional_t<(TT <= 64), WaveSync, BlockSync>;
-  const TwMem<T> twm{tw};
-  const double s = FILTER ? 1.0 : *gmem(d.scale);
+//
+// Shape of a block: radix-8 teams with the four planes of a group in registers (two exchanges
+// per transform, wave-local up to N = 512), and up to N = 1024 the four groups of its rows,
+// because they share their factors: a sqrt, a sincos and a division per cell and side, as much
+// FP64 work as the cell's transforms when every group evaluates its own.  The block evaluates
+// them once into LDS while the state's loads are in flight, and only at q1: lambda_{N-i} =
+// -lambda_i, so that q2 of bin i is q1 of bin N - i (of an extra entry at i = N/2).
+// 512^2 complex128: 60.1 -> 26.8 us a sweep (134 MB: 5.0 TB/s; a pass that only scales the state
+// takes 22 us); whole steps 115 -> 88 us, at 1024^2 553 -> 430, 2048 x 512 525 -> 347 and with the
+// step filter at 512^2 229 -> 142 us.  At 2048 four groups would be 1024 lanes of 128 registers
+// each: one group per block there.
+template <int N>
+struct DiracX {
+  static constexpr int R = 8, TT = N / R;
+  static constexpr int GPB = N <= 1024 ? 4 : 1;  // groups per block
+  static constexpr int BLOCK = GPB * TT;  // one row (small states: more blocks)
+  static constexpr int ROWS = BLOCK / (TT * GPB);
+  static constexpr int LSZ = Padded<N, R>::size;
+  static constexpr int kTeams = BLOCK / TT;
+  // LDS entries of type T per team array, and the table of (N + 1) FP64 pairs per row
+  static constexpr int kTab = ROWS * (N + 1);
+};
 
+// One side's factor [[(c, s), i b], [i b, (c, -s)]] (kinetic) or [[c, b], [b, s]] (filter) on the
+// pair (t, u).
+struct DiracSide {
+  double c, s, b;
+};
+template <bool FILTER>
+__device__ __forceinline__ void dirac_pair(const DiracSide& k, cplx<double>& t, cplx<double>& u) {
+  const cplx<double> p = t, q = u;
+  if constexpr (FILTER) {
+    t = {fma(k.c, p.x, k.b * q.x), fma(k.c, p.y, k.b * q.y)};
+    u = {fma(k.b, p.x, k.s * q.x), fma(k.b, p.y, k.s * q.y)};
+  } else {
+    t = {fma(k.c, p.x, -fma(k.s, p.y, k.b * q.y)), fma(k.c, p.y, fma(k.s, p.x, k.b * q.x))};
+    u = {fma(k.c, q.x, fma(k.s, q.y, -(k.b * p.y))), fma(k.c, q.y, fma(-k.s, q.x, k.b * p.x))};
+  }
+}
+
+// Scheduling fence on values: they are complete here and nothing computed from them moves in
+// front of this point.
+template <typename T>
+__device__ __forceinline__ void pin(cplx<T>& v) {
+  asm volatile("" : "+v"(v.x), "+v"(v.y));
+}
+template <typename T, int R>
+__device__ __forceinline__ void pin(cplx<T> (&v)[R]) {
+#pragma unroll
+  for (int j = 0; j < R; ++j) pin(v[j]);
+}
+
+template <typename S, typename T, int N, bool FILTER = false>
+__device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block, cplx<T>* lds, cplx<double>* tab) {
+  using G = DiracX<N>;
+  constexpr int R = G::R, TT = G::TT, ROWS = G::ROWS;
+  const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
+  const int tile = G::GPB == 4 ? block : block >> 2;
+  const int group = G::GPB == 4 ? team % 4 : block & 3;
+  const int rloc = G::GPB == 4 ? team / 4 : team;
+  const int row = tile * ROWS + rloc;
+  const size_t plane = size_t(d.P) * size_t(N);
+  const gptr<cplx<S>> W = gmem(reinterpret_cast<cplx<S>*>(d.W));
+  const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(d.twX_hi), reinterpret_cast<const cplx<T>*>(d.twX_lo)};
+  LdsRow<T> view{lds + team * G::LSZ};
+  using Sync = std::conditional_t<(TT <= 64), WaveSync, BlockSync>;
+  const double s = FILTER ? 1.0 : *gmem(d.scale);
+  // planes of group g = 2 (row pair) + (column pair), in the order [r1 c1, r1 c2, r2 c1, r2 c2]:
+  // row pairs {0, 3}, {1, 2} of spinor rows, the same of columns
+  const int gr = group >> 1, gc = group & 1;
+  auto plane_of = [&](int q) {
+    const int r = (q >> 1) ? 3 - gr : gr, c = (q & 1) ? 3 - gc : gc;
+    return 4 * r + c;
+  };
+  TwRegs<T, N, R> twr;
+  load_twiddles<T, N, R>(twr, t, tw);
   cplx<T> v[4][R];
+  // 32-bit byte offsets (16 planes of 2048^2 complex128 are 1 GiB), recomputed from an opaque
+  // copy of the lane index for the stores: no address stays live across the transforms
+  auto offset = [&](int q, int lane) {
+    return (unsigned(plane_of(q)) * unsigned(plane) + unsigned(row) * unsigned(N) + unsigned(lane)) * unsigned(sizeof(cplx<S>));
+  };
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const gptr<cplx<S>> src = W + size_t(kDiracGroups[group][q]) * plane;
+    const unsigned off = offset(q, t);
 #pragma unroll
-    for (int j = 0; j < R; ++j) v[q][j] = to_arith<T>(gload(src + t + j * TT));
+    for (int j = 0; j < R; ++j) v[q][j] = to_arith<T>(gload(at_off(W + j * TT, off)));
   }
+  // the factors at q1 = p + lambda_i/2: (cos(c dt s), sin(c dt s) / s), or the projector's
+  // (m c^2, c q) / (2 E); entry N is q1 = p + N/2 dlambda/2
+#pragma unroll 1
+  for (int e = tid; e < G::kTab; e += G::BLOCK) {
+    const int r = e / (N + 1), i = e % (N + 1);
+    const double p = d.kvn && !FILTER ? 0.0 : d.dp * double(fidx(tile * ROWS + r, d.P));
+    const double lam = d.dlambda * double(i < N ? fidx(i, N) : N / 2);
+    const double q1 = FILTER && d.kvn ? p : p + 0.5 * lam;
+    if constexpr (FILTER) {
+      const double e2 = 2.0 * sqrt(d.proj_mc2 * d.proj_mc2 + d.proj_c * d.proj_c * q1 * q1);
+      tab[e] = {d.proj_mc2 / e2, d.proj_c * q1 / e2};
+    } else {
+      const double sq = sqrt(d.mh_c * d.mh_c + q1 * q1);
+      double sn, cs;
+      sincos_fp64(d.c_dt * sq, &sn, &cs);
+      tab[e] = {cs, sn / sq};
+    }
+  }
+  // (one transform's, or one bin's, temporaries at a time: interleaved, and with a last pass spread
+  // over both sides of the branch below, they spilled 104 VGPRs at N = 512)
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-#pragma unroll
-    for (int j = 0; j < R; ++j) v[q][j] = cscale(v[q][j], T(s));
-    team_fft<T, N, R, -1, LdsRow<T>, Sync>(v[q], t, view, twm);
+    pin(v[q]);
+    team_fft<T, N, R, -1, LdsRow<T>, Sync>(v[q], t, view, twr);
+    pin(v[q]);
   }
+  __syncthreads();
 
   const double p = d.dp * double(fidx(row, d.P));
   if (!FILTER && d.antiparticle && (group == 0 || group == 3) && t == 0) {
@@ -112,52 +177,58 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int group,
     const double e2 = 2.0 * sqrt(d.proj_mc2 * d.proj_mc2 + d.proj_c * d.proj_c * p * p);
     const double aa = 0.5 - d.proj_mc2 / e2, bb = -d.proj_c * p / e2, dd = 0.5 + d.proj_mc2 / e2;
     const double c = aa * double(v[0][0].x) + bb * (double(v[1][0].x) + double(v[2][0].x)) + dd * double(v[3][0].x);
-    gmem(d.rowpart)[(group == 0 ? 0 : 1) * d.P + row] = c;
+    gmem(d.rowpart)[(group == 0 ? 0 : 1) * d.P + row] = s * c;
   }
 
+  // the pending factor and the 1/N of the inverse transform ride on the left factor
+  const double g = s * (1.0 / N);
+  const double mass = d.kvn ? 0.0 : d.mh_c;  // KvN: the diagonal is cos alone (GPU_WignerDiracKvN2D_4x4.py:183-189, 283-289)
+  const double pk = d.kvn ? 0.0 : p;
+  const cplx<double>* row_tab = tab + rloc * (N + 1);
 #pragma unroll
   for (int j = 0; j < R; ++j) {
-    const double lam = d.dlambda * double(fidx(t + j * TT, N));
-    Blk K, Rt;
+    const int i = opaque_v(t) + j * TT;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) pin(v[q][j]);
+    const int i2 = j == R / 2 && i == N / 2 ? N : (N - i) & (N - 1);
+    const cplx<double> e1 = row_tab[i], e2 = row_tab[i2];
+    DiracSide K, Rt;
     if constexpr (FILTER) {
-      const double h = d.kvn ? 0.0 : 0.5 * lam;
-      K = projector_block(p + h, d.proj_mc2, d.proj_c);
-      Rt = projector_block(p - h, d.proj_mc2, d.proj_c);
-    } else if (d.kvn) {
-      // KvN kinetic factors at q = +/- lambda/2 (GPU_WignerDiracKvN2D_4x4.py:183-189, 283-289)
-      K = kinetic_block(0.5 * lam, d.mh_c, d.c_dt, 1.0, 0.0);
-      Rt = kinetic_block(-0.5 * lam, d.mh_c, d.c_dt, -1.0, 0.0);
+      K = {g * (0.5 + e1.x), g * (0.5 - e1.x), g * e1.y};
+      Rt = {0.5 + e2.x, 0.5 - e2.x, e2.y};
     } else {
-      K = kinetic_block(p + 0.5 * lam, d.mh_c, d.c_dt, 1.0);
-      Rt = kinetic_block(p - 0.5 * lam, d.mh_c, d.c_dt, -1.0);
+      const double h = 0.5 * (d.dlambda * double(fidx(i, N)));
+      const double f1 = g * e1.y;
+      K = {g * e1.x, -mass * f1, -(pk + h) * f1};
+      Rt = {e2.x, mass * e2.y, (pk - h) * e2.y};  // dt -> -dt: the sine's sign
     }
-    const cplx<double> w0 = widen(v[0][j]), w1 = widen(v[1][j]), w2 = widen(v[2][j]), w3 = widen(v[3][j]);
-    // K B
-    const cplx<double> x0 = cadd(cmul(K.a, w0), cmul(K.b, w2));
-    const cplx<double> x1 = cadd(cmul(K.a, w1), cmul(K.b, w3));
-    const cplx<double> x2 = cadd(cmul(K.b, w0), cmul(K.d, w2));
-    const cplx<double> x3 = cadd(cmul(K.b, w1), cmul(K.d, w3));
-    // (K B) Rt
-    v[0][j] = narrow<T>(cadd(cmul(x0, Rt.a), cmul(x1, Rt.b)));
-    v[1][j] = narrow<T>(cadd(cmul(x0, Rt.b), cmul(x1, Rt.d)));
-    v[2][j] = narrow<T>(cadd(cmul(x2, Rt.a), cmul(x3, Rt.b)));
-    v[3][j] = narrow<T>(cadd(cmul(x2, Rt.b), cmul(x3, Rt.d)));
+    cplx<double> w0 = widen(v[0][j]), w1 = widen(v[1][j]), w2 = widen(v[2][j]), w3 = widen(v[3][j]);
+    dirac_pair<FILTER>(K, w0, w2);
+    dirac_pair<FILTER>(K, w1, w3);
+    dirac_pair<FILTER>(Rt, w0, w1);
+    dirac_pair<FILTER>(Rt, w2, w3);
+    v[0][j] = narrow<T>(w0);
+    v[1][j] = narrow<T>(w1);
+    v[2][j] = narrow<T>(w2);
+    v[3][j] = narrow<T>(w3);
   }
 
-  const T inv = T(1.0 / N);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    team_fft<T, N, R, +1, LdsRow<T>, Sync>(v[q], t, view, twm);
-    const gptr<cplx<S>> dst = W + size_t(kDiracGroups[group][q]) * plane;
+    pin(v[q]);
+    team_fft<T, N, R, +1, LdsRow<T>, Sync>(v[q], t, view, twr);
+    pin(v[q]);
+    const int ts = opaque_v(t);
+    const unsigned off = offset(q, ts);
     if constexpr (FILTER) {
+      if (d.fmask) {
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const T f = d.fmask ? T(gmem(d.fmask)[t + j * TT] * (1.0 / N)) : inv;
-        store_stream(dst + t + j * TT, to_arith<S>(cscale(v[q][j], f)));
+        for (int j = 0; j < R; ++j) v[q][j] = cscale(v[q][j], T(gmem(d.fmask)[ts + j * TT]));
       }
-    } else {
+    }
 #pragma unroll
-      for (int j = 0; j < R; ++j) store_stream(dst + t + j * TT, to_arith<S>(cscale(v[q][j], inv)));
+    for (int j = 0; j < R; ++j) {
+      store_stream(at_off(W + j * TT, off), to_arith<S>(v[q][j]));
     }
   }
 }
@@ -677,19 +748,7 @@ __device__ __forceinline__ void dirac_podm_body(const DiracPlan& d, int tile, cp
 constexpr int kDiracXBlock = 256;
 constexpr int kDiracPBlock = 256;
 
-// radix of the x sweep (4 planes live per lane) and of the p sweep (1 plane live)
-template <int N>
-constexpr int dirac_rx() {
-  return N >= 512 ? 8 : 4;
-}
-// radix of the kinetic x sweep for the state type S: at 512 a complex128 state takes radix 4
-// (two waves per row, 203 VGPRs, two waves per SIMD); radix 8 needs more than the 512
-// registers of a lane there and spilled 40 VGPRs to scratch (+35% memory traffic, 6% slower
-// per step).  The complex64 state keeps radix 8 (no scratch, 5% faster than radix 4).
-template <int N, typename S>
-constexpr int dirac_rx_state() {
-  return (N == 512 && sizeof(S) == 8) ? 4 : dirac_rx<N>();
-}
+// radix of the p sweep (1 plane live)
 template <int N>
 constexpr int dirac_rp() {
   return N >= 512 ? 8 : 4;  // at 512 radix 4 (three waves per SIMD) is 8% slower per step
@@ -736,11 +795,12 @@ __device__ __forceinline__ int dirac_col_tile() {
 // waves per SIMD at 512 and below, one above), and one kernel for all sides would take the
 // largest one's occupancy.
 template <typename S, typename T, int N, bool FILTER>
-__global__ void __launch_bounds__(kDiracXBlock) dirac_xsweep_kernel(const DiracPlan* __restrict__ dp) {
-  __shared__ cplx<T> lds[dirac_lds_elems<kDiracXBlock>()];
-  const DiracPlan& d = *dp;
-  const int group = int(blockIdx.x & 3u), tile = int(blockIdx.x >> 2);
-  dirac_xsweep_body<S, T, N, dirac_rx_state<N, S>(), kDiracXBlock, FILTER>(d, group, tile, lds);
+__global__ void __launch_bounds__(DiracX<N>::BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
+dirac_xsweep_kernel(const DiracPlan* __restrict__ dp) {
+  using G = DiracX<N>;
+  __shared__ cplx<T> lds[G::kTeams * G::LSZ];
+  __shared__ cplx<double> tab[G::kTab];
+  dirac_xsweep_body<S, T, N, FILTER>(*dp, int(blockIdx.x), lds, tab);
 }
 
 template <typename S, typename T, int N, bool CL>
@@ -1030,22 +1090,18 @@ __global__ void __launch_bounds__(256) dirac_gpshift_kernel(const DiracPlan* __r
 }
 
 // ------------------------------------------------------------------ launchers
-template <int N, typename S>
-constexpr int xsweep_rows() {
-  return kDiracXBlock / (N / dirac_rx_state<N, S>());
-}
 template <int N>
 constexpr int psweep_cols() {
   return kDiracPBlock / (N / dirac_rp<N>());
 }
 
-// blocks of the x sweep for a state of precision code prec (0: complex128)
-int dirac_x_blocks(int prec, int X, int P) {
-  int rows = 0;
-#define BODY(n) rows = prec == 0 ? xsweep_rows<n, double>() : xsweep_rows<n, float>()
+// blocks of the x sweep
+int dirac_x_blocks(int X, int P) {
+  int rows = 0, per = 0;
+#define BODY(n) rows = DiracX<n>::ROWS, per = 4 / DiracX<n>::GPB
   WH_DIRAC_DISPATCH(X, BODY)
 #undef BODY
-  return rows > 0 && P % rows == 0 ? 4 * (P / rows) : -1;
+  return rows > 0 && P % rows == 0 ? per * (P / rows) : -1;
 }
 
 int dirac_p_blocks(int X, int P) {
@@ -1058,15 +1114,10 @@ int dirac_p_blocks(int X, int P) {
 
 template <typename S, typename T, bool FILTER>
 hipError_t dirac_x_launch(int X, const DiracPlan* d, int nblocks, hipStream_t s) {
-  const dim3 g(nblocks), b(kDiracXBlock);
-  switch (X) {
-    case 128: hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, 128, FILTER>), g, b, 0, s, d); break;
-    case 256: hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, 256, FILTER>), g, b, 0, s, d); break;
-    case 512: hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, 512, FILTER>), g, b, 0, s, d); break;
-    case 1024: hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, 1024, FILTER>), g, b, 0, s, d); break;
-    case 2048: hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, 2048, FILTER>), g, b, 0, s, d); break;
-    default: return hipErrorInvalidValue;
-  }
+#define BODY(n) \
+  hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, n, FILTER>), dim3(nblocks), dim3(DiracX<n>::BLOCK), 0, s, d)
+  WH_DIRAC_DISPATCH(X, BODY)
+#undef BODY
   return hipGetLastError();
 }
 
