@@ -228,7 +228,9 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      store_stream(at_off(W + j * TT, off), to_arith<S>(v[q][j]));
+      // written back, not streamed: the p sweep then finds the state in the last-level cache (a
+      // copy with these two access patterns, 512^2: 50 us a pair streamed, 37 us written back)
+      store_cached(at_off(W + j * TT, off), to_arith<S>(v[q][j]));
     }
   }
 }
@@ -343,109 +345,286 @@ __device__ __forceinline__ void dirac_store_colsums(const DiracPlan& d, int tile
 //   quarter 2: 1 4 | 11 14,  quarter 3: 2 7 | 8 13 (no column sums)
 // Each quarter writes only its own column sums.  With 16 planes per tile (one block) the 512^2
 // sweep had one wave per SIMD on half of the CUs; two class pairs per tile filled the CUs, four
-// quarters give two waves per SIMD (at two multiplier evaluations per block instead of one).
-__constant__ int kDiracQuarter[4][2][2] = {{{0, 5}, {10, 15}}, {{3, 6}, {9, 12}}, {{1, 4}, {11, 14}}, {{2, 7}, {8, 13}}};
-__constant__ int kDiracQuarterClass[4][2] = {{0, 3}, {1, 2}, {0, 3}, {1, 2}};
-template <typename S, typename T, int N, int R, int BLOCK, bool CL>
-__device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, int quarter, cplx<T>* lds) {
-  constexpr int TT = N / R;
-  constexpr int C = BLOCK / TT;  // columns per tile
+// quarters give two waves per SIMD.
+__constant__ int kDiracQuarter[4][4] = {{0, 5, 10, 15}, {3, 6, 9, 12}, {1, 4, 11, 14}, {2, 7, 8, 13}};
+
+// Radix-8 teams.  Up to P = 512 a column's team lies in one wave: the loads cover rows of C = 4
+// consecutive columns, the first exchange moves each column to a team of consecutive lanes
+// (team_fft_remap) and the store moves it back, two block barriers a plane where a team spread over
+// the waves needs one per exchange and direction.  Planes alternate between two LDS arrays, so
+// that the next plane's first exchange need not wait for this one's store, and the next plane is
+// loaded while this one is transformed.  With friction (CL) a lane holds a second copy of its
+// column instead of the next plane's, reads p and theta from LDS, and there is one array.
+// The two classes' multipliers differ by e^{2im} (one product per element instead of a sincos).
+// 512^2 complex128 (134 MB): 45.5 -> 33.2 us a sweep, a step 88 -> 70 us, with friction 146 -> 95
+// (whose operator is summed by powers); 512 x 2048 589 -> 368 and 1143 -> 477 us.  The two sweeps'
+// access patterns alone, copying, take 37 us a step.
+template <int N, bool CL>
+struct DiracP {
+  static constexpr int R = 8, TT = N / R;
+  static constexpr bool kWave = TT <= 64;
+  static constexpr int BLOCK = kWave ? 4 * TT : 256;
+  static constexpr int C = BLOCK / TT;  // columns per tile
+  // (a multiple of 16 entries plus 4: the four columns of the load layout on different banks)
+  static constexpr int LSZ = kWave ? N + N / R + 4 : Padded<N, R>::size;
+  static constexpr int kArrays = kWave && !CL ? 2 : 1;
+  static constexpr int kTab = CL ? 2 * N : 1;  // friction: p and theta / N of the column's elements
+};
+
+template <typename S, typename T, int N, bool CL>
+__device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, int quarter, cplx<T>* lds, T* tab) {
+  using G = DiracP<N, CL>;
+  constexpr int R = G::R, TT = G::TT, C = G::C, LSZ = G::LSZ;
+  constexpr bool kWave = G::kWave;
+  constexpr bool kAhead = kWave && !CL;
+  using View = std::conditional_t<kWave, LdsRow<T>, LdsStrided<T, C>>;
+  using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
   const int tid = threadIdx.x;
-  const int c = tid % C, t = tid / C;
+  const int cl = tid % C, tl = tid / C;                                  // load layout
+  const int cc = kWave ? tid / TT : cl, tc = kWave ? tid % TT : tl;      // compute layout
   const int X = d.X;
-  const int col = tile * C + c;
-  const size_t plane = size_t(d.P) * size_t(X);
+  const int col = tile * C + cc;
+  const size_t plane = size_t(N) * size_t(X);
   const gptr<cplx<S>> W0 = gmem(reinterpret_cast<cplx<S>*>(d.W));
   const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(d.twP_hi), reinterpret_cast<const cplx<T>*>(d.twP_lo)};
-  LdsStrided<T, C> view{lds + c};
-  const int step = *gmem(d.step);
+  const int step = *cmem(d.step);
 
-  // Bopp phase dt (V0(x - theta/2) - V0(x + theta/2)) of this lane's elements (shared by the 16 planes)
-  const double x = d.dx * double(fidx(col, X));
+  // Class multiplier r e^{-i (ph + m)} / N: ph the Bopp phase dt (V0(x - theta/2) - V0(x + theta/2)) (KvN:
+  // e^{i dt V0'(x) theta} for every plane, KvN_XTheta_Kernel, GPU_WignerDiracKvN2D_4x4.py:356-420),
+  // m = F- - F+ (lo, lo), F- + F+ (lo, hi), -(F- + F+) (hi, lo), -(F- - F+) (hi, hi), F -/+ =
+  // Mass(x -/+ theta/2) c^2 dt; a constant mass gives 0, 2F, -2F, 0.  A quarter's second class has -m.
+  // What the first ones are made of is loaded before the state (vector loads return in order).
+  const bool table = !d.kvn && d.pot_deg < 0;
+  const gptr<const double> mass = d.kvn ? nullptr : gmem((quarter & 1) ? d.mass_sm : d.mass_dm);
+  const double mconst = (quarter & 1) && !d.kvn ? 2.0 * d.mass_phase : 0.0;
   const double mask = d.xmask ? gmem(d.xmask)[col] : 1.0;
-  double ph[R];
+  double r[R], ph[R], gv[R], mv[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    r[j] = 1.0;
+    ph[j] = gv[j] = 0.0;
+    mv[j] = mconst;
+  }
+  if (d.theta_decay) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) r[j] = gmem(d.theta_decay)[tc + j * TT];
+  }
+  if (table) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) ph[j] = gmem(d.pot_dv)[size_t(tc + j * TT) * X + col];
+  }
+  const bool gp = !d.kvn && d.gp_coeff != 0.0;
+  if (gp) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) gv[j] = gmem(d.G)[size_t(tc + j * TT) * X + col];
+  }
+  if (mass) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) mv[j] = mass[size_t(tc + j * TT) * X + col];
+  }
+  double dvx = 0.0;
+  if (d.kvn && d.pot_deg < 0) dvx = gmem(d.dv0)[col];
+  // Re tr W of each element (quarter 0), or its p_host (quarter 1)
+  double aux[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) aux[j] = 0.0;
+  if (quarter == 1) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) aux[j] = gmem(d.p_host)[tc + j * TT];
+  }
+  if constexpr (CL) {  // (visible after the first transform's block barrier)
+    for (int i = tid; i < N; i += G::BLOCK) {
+      tab[i] = T(gmem(d.p_host)[i]);
+      tab[N + i] = T(gmem(d.theta_host)[i] * (1.0 / N));
+    }
+  }
+  TwRegs<T, N, R> twr;
+  load_twiddles<T, N, R>(twr, tc, tw);
+
+  const unsigned jstride = unsigned(TT) * unsigned(X) * unsigned(sizeof(cplx<S>));
+  auto offset = [&](int i) {
+    return (unsigned(i / C) * unsigned(X) + unsigned(tile * C + i % C)) * unsigned(sizeof(cplx<S>));
+  };
+  auto load = [&](cplx<T>(&v)[R], int k) {
+    const unsigned off = offset(opaque_v(tid));
+    const gptr<cplx<S>> W = W0 + size_t(k) * plane;
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload(at_off(W, off + unsigned(j) * jstride)));
+  };
+  cplx<T> v[R], next[kAhead ? R : 1];
+  load(v, kDiracQuarter[quarter][0]);
+  if constexpr (kAhead) load(next, kDiracQuarter[quarter][1]);
+  cplx<double> M[R];
   {
+    const double x = d.dx * double(fidx(col, X));
     const int prow = step < d.pot_rows ? step : d.pot_rows - 1;
-    const BoppOdd bopp = bopp_odd(cmem(d.pot) + size_t(prow) * (kMaxDeg + 1), d.pot_deg, x, 1.0);
-    // KvN: e^{i dt V0'(x) theta} for every plane (KvN_XTheta_Kernel, GPU_WignerDiracKvN2D_4x4.py:356-420)
-    double dvx = 0.0;
+    const cptr<double> cf = cmem(d.pot) + size_t(prow) * (kMaxDeg + 1);
     if (d.kvn) {
-      if (d.pot_deg >= 0) {
-        const cptr<double> cf = cmem(d.pot) + size_t(prow) * (kMaxDeg + 1);
-        for (int n = d.pot_deg; n >= 1; --n) dvx = fma(dvx, x, double(n) * cf[n]);
-      } else {
-        dvx = gmem(d.dv0)[col];
-      }
+      for (int n = d.pot_deg; n >= 1; --n) dvx = fma(dvx, x, double(n) * cf[n]);
+#pragma unroll
+      for (int j = 0; j < R; ++j) ph[j] = -dvx * (d.dtheta * double(fidx(tc + j * TT, N)));
+    } else if (!table) {
+      const BoppOdd bopp = bopp_odd(cf, d.pot_deg, x, 1.0);
+#pragma unroll
+      for (int j = 0; j < R; ++j) ph[j] = bopp(0.5 * (d.dtheta * double(fidx(tc + j * TT, N))));
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) ph[j] *= d.dt;
+    if (gp) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) ph[j] += d.dt * d.gp_coeff * gv[j];
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-      const int i = t + j * TT;
-      const double th = d.dtheta * double(fidx(i, N));
-      if (d.kvn) {
-        ph[j] = -d.dt * dvx * th;
-        continue;
-      }
-      const double dv = d.pot_deg >= 0 ? bopp(0.5 * th) : gmem(d.pot_dv)[size_t(i) * X + col];
-      ph[j] = d.dt * dv;
-      if (d.gp_coeff != 0.0) ph[j] += d.dt * d.gp_coeff * gmem(d.G)[size_t(i) * X + col];
+      M[j] = expmi(r[j] * mask * (1.0 / N), ph[j] + mv[j]);
+      pin(M[j]);
     }
   }
+  // sums of this quarter's planes: {Re, Im} of sum W, sum p W, sum p^2 W (quarter 0) or sum p_host W
+  // (quarter 1), and sum beta W (quarter 0)
+  double acc[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) acc[q] = 0.0;
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+    const int k = kDiracQuarter[quarter][q];
+    if constexpr (kAhead) {
+      if (q > 0 && q < 3) load(next, kDiracQuarter[quarter][q + 1]);
+    } else {
+      if (q > 0) load(v, k);
+    }
+    if (q == 2 && mass) {  // the second class: e^{2 i m} of the first
+      const int t = opaque_v(tc);
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        M[j] = cmul(M[j], expmi(1.0, -2.0 * mass[size_t(t + j * TT) * X + col]));
+        pin(M[j]);
+      }
+    } else if (q == 2 && mconst != 0.0) {
+      const cplx<double> e = expmi(1.0, -2.0 * mconst);
+#pragma unroll
+      for (int j = 0; j < R; ++j) M[j] = cmul(M[j], e);
+    }
+    cplx<T>* arr = lds + (G::kArrays > 1 ? (q & 1) * C * LSZ : 0);
+    if (kWave && G::kArrays == 1 && q > 0) __syncthreads();  // the last store has been read from the array
+    const View view{kWave ? arr + cc * LSZ : arr + cl};
+    if constexpr (kWave) {
+      team_fft_remap<T, N, R, -1>(v, tl, LdsRow<T>{arr + cl * LSZ}, tc, view, twr);
+    } else {
+      team_fft<T, N, R, -1, View, Sync>(v, tc, view, twr);
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = apply(v[j], M[j]);
+    team_fft<T, N, R, +1, View, Sync>(v, tc, view, twr);
+    pin(v);
 
-  double acc[kDNCol];
+    if constexpr (CL) {
+      // CaldeiraDissipatorOrder2 (GPU_WignerDirac2D_4x4.py:3011-3030), host grids: D(Y) = F_p^-1[ theta
+      // F_p[ p Y ] ]; LW2 = W + a D W; W + 2 a D LW2 = W + 2 a D W + 2 a^2 D^2 W, a = i dt gamma (by powers:
+      // one copy of the column less)
+      cplx<T> y[R];
 #pragma unroll
-  for (int q = 0; q < kDNCol; ++q) acc[q] = 0.0;
-  double trre[R];
+      for (int j = 0; j < R; ++j) y[j] = v[j];
+      for (int o = 0; o < 2; ++o) {
 #pragma unroll
-  for (int j = 0; j < R; ++j) trre[j] = 0.0;
+        for (int j = 0; j < R; ++j) y[j] = cscale(y[j], tab[tc + j * TT]);
+        team_fft<T, N, R, -1, View, Sync>(y, tc, view, twr);
+#pragma unroll
+        for (int j = 0; j < R; ++j) y[j] = cscale(y[j], tab[N + tc + j * TT]);
+        team_fft<T, N, R, +1, View, Sync>(y, tc, view, twr);
+        const double re = o == 0 ? 0.0 : -2.0 * d.cl_a * d.cl_a, im = o == 0 ? 2.0 * d.cl_a : 0.0;
+#pragma unroll
+        for (int j = 0; j < R; ++j) v[j] = o == 0 ? cadd(v[j], mul_i(y[j], T(im))) : cadd(v[j], cscale(y[j], T(re)));
+      }
+    }
 
-  const T inv = T(1.0 / N);
-  const unsigned boff = (unsigned(t) * unsigned(X) + unsigned(col)) * unsigned(sizeof(cplx<S>));
-  // planes by mass-phase class: spinor rows {1,2} or {3,4} x columns {1,2} or {3,4}.  Class
-  // multiplier r e^{-i (ph + m)}: m = F- - F+ (lo, lo), F- + F+ (lo, hi), -(F- + F+) (hi, lo),
-  // -(F- - F+) (hi, hi), F -/+ = Mass(x -/+ theta/2) c^2 dt; a constant mass gives 0, 2F, -2F, 0.
-  for (int ci = 0; ci < 2; ++ci) {
-    const int cls = kDiracQuarterClass[quarter][ci];
-    cplx<double> M[R];
+    pin(v);
+    const int ta = opaque_v(tc);
+    if (quarter == 0) {
+      const double sb = q < 2 ? 1.0 : -1.0;
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const int i = t + j * TT;
-      double m;
-      if (d.mass_dm) {
-        const size_t e = size_t(i) * X + col;
-        m = cls == 0 ? gmem(d.mass_dm)[e] : cls == 1 ? gmem(d.mass_sm)[e] : cls == 2 ? -gmem(d.mass_sm)[e] : -gmem(d.mass_dm)[e];
+      for (int j = 0; j < R; ++j) {
+        const double p = d.dp * double(fidx(ta + j * TT, N));
+        const double wr = double(v[j].x), wi = double(v[j].y);
+        acc[0] += wr;
+        acc[1] += wi;
+        acc[2] = fma(p, wr, acc[2]);
+        acc[3] = fma(p, wi, acc[3]);
+        acc[4] = fma(p * p, wr, acc[4]);
+        acc[5] = fma(p * p, wi, acc[5]);
+        acc[6] = fma(sb, wr, acc[6]);
+        acc[7] = fma(sb, wi, acc[7]);
+        aux[j] += wr;
+      }
+    } else if (quarter == 1) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        const double p = d.dp * double(fidx(ta + j * TT, N));
+        const double wr = double(v[j].x), wi = double(v[j].y);
+        acc[0] += wr;
+        acc[1] += wi;
+        acc[2] = fma(p, wr, acc[2]);
+        acc[3] = fma(p, wi, acc[3]);
+        acc[4] = fma(aux[j], wr, acc[4]);
+        acc[5] = fma(aux[j], wi, acc[5]);
+      }
+    }
+    if constexpr (kWave) {  // back to the load layout: natural order through the team's array
+      Sync::sync();
+#pragma unroll
+      for (int j = 0; j < R; ++j) *view.ptr(padr<R>(tc + j * TT)) = v[j];
+      __syncthreads();
+      const LdsRow<T> view_l{arr + cl * LSZ};
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = *view_l.ptr(padr<R>(tl + j * TT));
+    }
+    const unsigned off = offset(opaque_v(tid));
+    const gptr<cplx<S>> W = W0 + size_t(k) * plane;
+#pragma unroll
+    for (int j = 0; j < R; ++j) store_cached(at_off(W, off + unsigned(j) * jstride), to_arith<S>(v[j]));
+    if constexpr (kAhead) {
+#pragma unroll
+      for (int j = 0; j < R; ++j) v[j] = next[j];
+    }
+  }
+  if (quarter >= 2) return;
+
+  // column sums: the quarter's entries in DiracCol order
+  double neg = 0.0;
+#pragma unroll
+  for (int j = 0; j < R; ++j) neg += aux[j] < 0.0 ? aux[j] : 0.0;
+  if constexpr (kWave) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc[q] = group_sum<TT>(acc[q]);
+    neg = group_sum<TT>(neg);
+    if (tc == TT - 1) {
+      const gptr<double> cs = gmem(d.colsums) + size_t(col) * kDNCol;
+      if (quarter == 0) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) cs[kDcTrRe + q] = acc[q];
+        cs[kDcBetaRe] = acc[6];
+        cs[kDcBetaIm] = acc[7];
+        cs[kDcNeg] = neg;
       } else {
-        m = cls == 1 ? 2.0 * d.mass_phase : cls == 2 ? -2.0 * d.mass_phase : 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) cs[kDcA1Re + q] = acc[q];
       }
-      if (d.kvn) m = 0.0;
-      const double r = (d.theta_decay ? gmem(d.theta_decay)[i] : 1.0) * mask;
-      M[j] = expmi(r, ph[j] + m);
     }
-    for (int q = 0; q < 2; ++q) {
-      const int k = kDiracQuarter[quarter][ci][q];
-      const gptr<cplx<S>> W = W0 + size_t(k) * plane;
-      cplx<T> v[R];
+  } else {
+    double all[kDNCol];
 #pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = to_arith<T>(gload(at_off(W + size_t(j * TT) * X, boff)));
-      team_fft<T, N, R, -1>(v, t, view, tw);
+    for (int q = 0; q < kDNCol; ++q) all[q] = 0.0;
 #pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = apply(v[j], M[j]);
-      team_fft<T, N, R, +1>(v, t, view, tw);
-#pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = cscale(v[j], inv);
-
-      if constexpr (CL) dirac_cl2<T, N, R>(v, d, t, view, tw);
-
-      dirac_accumulate<T, R, TT>(d, k, v, t, acc, trre);
-#pragma unroll
-      for (int j = 0; j < R; ++j) store_stream(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[j]));
+    for (int q = 0; q < 6; ++q) {
+      all[kDcTrRe + q] = quarter == 0 ? acc[q] : 0.0;
+      all[kDcA1Re + q] = quarter == 1 ? acc[q] : 0.0;
     }
+    all[kDcBetaRe] = acc[6];
+    all[kDcBetaIm] = acc[7];
+    all[kDcNeg] = neg;
+    dirac_store_colsums<G::BLOCK, C>(d, tile, all, lds, quarter);
   }
-#pragma unroll
-  for (int j = 0; j < R; ++j) acc[kDcNeg] += trre[j] < 0.0 ? trre[j] : 0.0;
-
-  if (quarter < 2) dirac_store_colsums<BLOCK, C>(d, tile, acc, lds, quarter);
 }
-
 
 // ------------------------------------------------------------------ p sweeps with vector potentials
 // With A = (A1, A2, A3) != 0 the potential factors P-(x - theta/2) (left) and P+(x + theta/2)
@@ -558,7 +737,7 @@ __device__ __forceinline__ void dirac_pleft_body(const DiracPlan& d, int tile, c
     for (int q = 0; q < 4; ++q) {
       const gptr<cplx<S>> W = W0 + size_t(4 * q + jc) * plane;
 #pragma unroll
-      for (int j = 0; j < R; ++j) store_stream(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
+      for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
     }
   }
 }
@@ -615,7 +794,7 @@ __device__ __forceinline__ void dirac_pright_body(const DiracPlan& d, int tile, 
       const gptr<cplx<S>> W = W0 + size_t(k) * plane;
       if (d.odm) {  // ODM damping follows in the theta picture (dirac_podm_body with A)
 #pragma unroll
-        for (int j = 0; j < R; ++j) store_stream(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
+        for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
         continue;
       }
       team_fft<T, N, R, +1>(v[q], t, view, tw);
@@ -624,7 +803,7 @@ __device__ __forceinline__ void dirac_pright_body(const DiracPlan& d, int tile, 
       if constexpr (CL) dirac_cl2<T, N, R>(v[q], d, t, view, tw);
       dirac_accumulate<T, R, TT>(d, k, v[q], t, acc, trre);
 #pragma unroll
-      for (int j = 0; j < R; ++j) store_stream(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
+      for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
     }
   }
   if (d.odm) return;  // dirac_podm_body transforms back and writes the column sums
@@ -736,7 +915,7 @@ __device__ __forceinline__ void dirac_podm_body(const DiracPlan& d, int tile, cp
       dirac_accumulate<T, R, TT>(d, kp[q], v[q], t, acc, trre);
       const gptr<cplx<S>> W = W0 + size_t(kp[q]) * plane;
 #pragma unroll
-      for (int j = 0; j < R; ++j) store_stream(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
+      for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), to_arith<S>(v[q][j]));
     }
   }
 #pragma unroll
@@ -746,13 +925,7 @@ __device__ __forceinline__ void dirac_podm_body(const DiracPlan& d, int tile, cp
 
 // ------------------------------------------------------------------ kernels
 constexpr int kDiracXBlock = 256;
-constexpr int kDiracPBlock = 256;
 
-// radix of the p sweep (1 plane live)
-template <int N>
-constexpr int dirac_rp() {
-  return N >= 512 ? 8 : 4;  // at 512 radix 4 (three waves per SIMD) is 8% slower per step
-}
 // radix of the vector-potential p sweeps (4 planes live per lane and two factor matrices)
 template <int N>
 constexpr int dirac_rv() {
@@ -804,11 +977,15 @@ dirac_xsweep_kernel(const DiracPlan* __restrict__ dp) {
 }
 
 template <typename S, typename T, int N, bool CL>
-__global__ void __launch_bounds__(kDiracPBlock) dirac_psweep_kernel(const DiracPlan* __restrict__ dp) {
-  __shared__ cplx<T> lds[dirac_lds_elems<kDiracPBlock>()];
+__global__ void __launch_bounds__((DiracP<N, CL>::BLOCK)) __attribute__((amdgpu_waves_per_eu(2)))
+dirac_psweep_kernel(const DiracPlan* __restrict__ dp) {
+  using G = DiracP<N, CL>;
+  constexpr int kLds = G::kArrays * G::C * G::LSZ, kRed = G::BLOCK * kDNCol * 8 / int(sizeof(cplx<T>));
+  __shared__ cplx<T> lds[!G::kWave && kRed > kLds ? kRed : kLds];
+  __shared__ T tab[G::kTab];
   const DiracPlan& d = *dp;
   const int u = dirac_col_tile();
-  dirac_psweep_body<S, T, N, dirac_rp<N>(), kDiracPBlock, CL>(d, u >> 2, u & 3, lds);
+  dirac_psweep_body<S, T, N, CL>(d, u >> 2, u & 3, lds, tab);
 }
 
 template <typename S, typename T>
@@ -1090,11 +1267,6 @@ __global__ void __launch_bounds__(256) dirac_gpshift_kernel(const DiracPlan* __r
 }
 
 // ------------------------------------------------------------------ launchers
-template <int N>
-constexpr int psweep_cols() {
-  return kDiracPBlock / (N / dirac_rp<N>());
-}
-
 // blocks of the x sweep
 int dirac_x_blocks(int X, int P) {
   int rows = 0, per = 0;
@@ -1106,7 +1278,7 @@ int dirac_x_blocks(int X, int P) {
 
 int dirac_p_blocks(int X, int P) {
   int cols = 0;
-#define BODY(n) cols = psweep_cols<n>()
+#define BODY(n) cols = (DiracP<n, false>::C)
   WH_DIRAC_DISPATCH(P, BODY)
 #undef BODY
   return cols > 0 && X % cols == 0 ? 4 * (X / cols) : -1;  // four blocks (quarters) per tile
@@ -1134,15 +1306,10 @@ hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks,
 
 template <typename S, typename T, bool CL>
 hipError_t dirac_p_launch(int P, const DiracPlan* d, int nblocks, hipStream_t s) {
-  const dim3 g(nblocks), b(kDiracPBlock);
-  switch (P) {
-    case 128: hipLaunchKernelGGL((dirac_psweep_kernel<S, T, 128, CL>), g, b, 0, s, d); break;
-    case 256: hipLaunchKernelGGL((dirac_psweep_kernel<S, T, 256, CL>), g, b, 0, s, d); break;
-    case 512: hipLaunchKernelGGL((dirac_psweep_kernel<S, T, 512, CL>), g, b, 0, s, d); break;
-    case 1024: hipLaunchKernelGGL((dirac_psweep_kernel<S, T, 1024, CL>), g, b, 0, s, d); break;
-    case 2048: hipLaunchKernelGGL((dirac_psweep_kernel<S, T, 2048, CL>), g, b, 0, s, d); break;
-    default: return hipErrorInvalidValue;
-  }
+#define BODY(n) \
+  hipLaunchKernelGGL((dirac_psweep_kernel<S, T, n, CL>), dim3(nblocks), dim3((DiracP<n, CL>::BLOCK)), 0, s, d)
+  WH_DIRAC_DISPATCH(P, BODY)
+#undef BODY
   return hipGetLastError();
 }
 
