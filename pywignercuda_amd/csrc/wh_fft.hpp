@@ -64,6 +64,41 @@ __device__ __forceinline__ cplx<T> gload(gptr<cplx<T>> p) {
   return gload<T>(gptr<const cplx<T>>(p));
 }
 
+// element of a uniform row base at a per-lane 32-bit byte offset (SGPR base +
+// VGPR offset addressing: one offset register per lane for all strided elements)
+template <typename T>
+__device__ __forceinline__ cplx<T>& at_off(cplx<T>* base, unsigned boff) {
+  return *reinterpret_cast<cplx<T>*>(reinterpret_cast<char*>(base) + boff);
+}
+template <typename T>
+__device__ __forceinline__ gptr<cplx<T>> at_off(gptr<cplx<T>> base, unsigned boff) {
+  return reinterpret_cast<gptr<cplx<T>>>(reinterpret_cast<gptr<char>>(base) + boff);
+}
+template <typename T>
+__device__ __forceinline__ gptr<const cplx<T>> at_off(gptr<const cplx<T>> base, unsigned boff) {
+  return reinterpret_cast<gptr<const cplx<T>>>(reinterpret_cast<gptr<const char>>(base) + boff);
+}
+
+// Streaming store of a state element: the sweep writes each element once and the next
+// sweep reads it from another CU, so the line is not kept dirty in this CU's L2 (less
+// write-back at the end of the kernel).
+template <typename S>
+__device__ __forceinline__ void store_stream(gptr<cplx<S>> p, cplx<S> v) {
+  typedef S vec2 __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(vec2{v.x, v.y}, reinterpret_cast<gptr<vec2>>(p));
+}
+
+// Write-back store of a state element, for sweeps whose store instruction covers half of
+// each 128-byte line (the p sweep's C-column rows): the neighbouring tile, on the same XCD at
+// about the same time, fills the other half in L2 before the line is written back.  With
+// streaming stores the half lines went out separately (+39% WRITE_SIZE on a 64 x 1024^2
+// FP64 batch; +1.2% with this store).
+template <typename S>
+__device__ __forceinline__ void store_cached(gptr<cplx<S>> p, cplx<S> v) {
+  typedef S vec2 __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<gptr<vec2>>(p) = vec2{v.x, v.y};
+}
+
 template <typename T>
 __device__ __forceinline__ cplx<T> cadd(cplx<T> a, cplx<T> b) { return {a.x + b.x, a.y + b.y}; }
 template <typename T>
@@ -179,6 +214,16 @@ template <int N, int PR>
 struct Padded {
   static constexpr int size = N + N / PR + 1;
 };
+
+// Padding of a column's LDS array of N + N/R entries where C columns are transposed between the load
+// layout (C columns x consecutive rows in a wave) and wave teams: the C columns of a row then start
+// 256 / C bytes apart in the 64 banks (with one entry, four columns met in the same banks: a third of
+// the LDS cycles of a 512^2 sweep).
+template <typename E, int C>
+constexpr int col_pad() {
+  constexpr int p = 256 / int(sizeof(cplx<E>)) / C;
+  return p > 1 ? p : 1;
+}
 
 // LDS views of one team's working array.  ptr(pb) is the address of padded
 // index pb; S is the element stride between consecutive padded indices.  The element

@@ -84,43 +84,8 @@ __device__ __forceinline__ cplx<T> scale_load(cplx<T> v, const double* s) {
   return apply(v, cplx<double>{cmem(s)[0], cmem(s)[1]});
 }
 
-// element of a uniform row base at a per-lane 32-bit byte offset (SGPR base +
-// VGPR offset addressing: one offset register per lane for all strided elements)
-template <typename T>
-__device__ __forceinline__ cplx<T>& at_off(cplx<T>* base, unsigned boff) {
-  return *reinterpret_cast<cplx<T>*>(reinterpret_cast<char*>(base) + boff);
-}
-template <typename T>
-__device__ __forceinline__ gptr<cplx<T>> at_off(gptr<cplx<T>> base, unsigned boff) {
-  return reinterpret_cast<gptr<cplx<T>>>(reinterpret_cast<gptr<char>>(base) + boff);
-}
-template <typename T>
-__device__ __forceinline__ gptr<const cplx<T>> at_off(gptr<const cplx<T>> base, unsigned boff) {
-  return reinterpret_cast<gptr<const cplx<T>>>(reinterpret_cast<gptr<const char>>(base) + boff);
-}
-
 template <typename T>
 __device__ __forceinline__ cplx<T> mul_i(cplx<T> a, T s) { return {-s * a.y, s * a.x}; }
-
-// Streaming store of a state element: the sweep writes each element once and the next
-// sweep reads it from another CU, so the line is not kept dirty in this CU's L2 (less
-// write-back at the end of the kernel).
-template <typename S>
-__device__ __forceinline__ void store_stream(gptr<cplx<S>> p, cplx<S> v) {
-  typedef S vec2 __attribute__((ext_vector_type(2)));
-  __builtin_nontemporal_store(vec2{v.x, v.y}, reinterpret_cast<gptr<vec2>>(p));
-}
-
-// Write-back store of a state element, for sweeps whose store instruction covers half of
-// each 128-byte line (the p sweep's C-column rows): the neighbouring tile, on the same XCD at
-// about the same time, fills the other half in L2 before the line is written back.  With
-// streaming stores the half lines went out separately (+39% WRITE_SIZE on a 64 x 1024^2
-// FP64 batch; +1.2% with this store).
-template <typename S>
-__device__ __forceinline__ void store_cached(gptr<cplx<S>> p, cplx<S> v) {
-  typedef S vec2 __attribute__((ext_vector_type(2)));
-  *reinterpret_cast<gptr<vec2>>(p) = vec2{v.x, v.y};
-}
 
 // state storage S <-> arithmetic T (complex64 states with FP64 arithmetic convert at the
 // sweep's load and store; every other combination is the identity)
@@ -129,8 +94,8 @@ __device__ __forceinline__ cplx<T> to_arith(cplx<S> v) {
   return {T(v.x), T(v.y)};
 }
 
-// Largest LDS footprint over the supported sizes for a (block, radix) variant:
-// ROWS*Padded(N) = (BLOCK/(N/R)) * (N + N/R + 1) elements.
+// Largest LDS footprint over the supported sizes for a (block, radix) variant: ROWS*Padded(N) =
+// (BLOCK/(N/R)) * (N + N/R + 1) elements, and up to 32 more for col_pad.
 template <int BLOCK, int R>
 constexpr int lds_elems() {
   int m = 0;
@@ -140,7 +105,7 @@ constexpr int lds_elems() {
     const int e = rows * (N + N / R + 1);
     m = e > m ? e : m;
   }
-  return m;
+  return m + 32;
 }
 
 template <int N, int R, int BLOCK>
@@ -485,10 +450,11 @@ template <typename T, int N, int R, int BLOCK, typename E = T>
 struct PSweep {
   static constexpr int TT = N / R;
   static constexpr int C = BLOCK / TT;  // columns per tile
-  static constexpr int LSZ = Padded<N, R>::size;
   // wave teams: a column's team lies inside one wave and the transform has an exchange
   // at which the lanes can leave the load layout (then every later exchange is wave-local)
   static constexpr bool kWave = TT <= 64 && num_passes(N, R) >= 2;
+  static constexpr int LSZ = kWave ? N + N / R + col_pad<E, C>() : Padded<N, R>::size;
+  static_assert(C * LSZ <= lds_elems<BLOCK, R>(), "LDS array");
   using View = std::conditional_t<kWave, LdsRow<E>, LdsStrided<E, C>>;
   using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
 
