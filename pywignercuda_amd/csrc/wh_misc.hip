@@ -234,75 +234,107 @@ __global__ void set_scale_kernel(const Member* members, double re, double im) {
 }
 
 // ------------------------------------------------------------------ plain axis transforms
-template <typename T, int N, int R, int ROWS, int DIR>
-__global__ void __launch_bounds__(ROWS*(N / R))
+// Teams of one wave (radix 8 up to N = 512, radix 16 at 1024) exchange without block barriers and hold
+// their twiddles in registers, loaded with the state.  A row block is one wave (or the team), so that
+// a few hundred rows reach every CU: blocks of 256 lanes left half of them idle at 512 x 1024.
+// A forward and an inverse pair over both axes with two clones, us, before -> after (radix 16 for every
+// length, block barriers, 256 lanes a block): 2048^2 complex128 239 -> 147, complex64 205 -> 119; 1024^2
+// 65 -> 60 and 64 -> 44; 512 x 1024 47 -> 38; below, the calls' host time (38 us) covers the kernels.
+template <typename T, int N>
+struct FftShape {
+  static constexpr int R = N <= 512 ? 8 : 16, TT = N / R;
+  static constexpr bool kWave = TT <= 64;
+  static constexpr int ROWS = TT >= 64 ? 1 : 64 / TT;             // rows per block
+  static constexpr int C = N <= 512 ? 8 : N <= 1024 ? 4 : 2;      // columns per block
+  using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
+};
+
+template <typename T, int N, int DIR>
+__global__ void __launch_bounds__((FftShape<T, N>::ROWS * FftShape<T, N>::TT))
     fft_rows_kernel(void* data, int rows, int normalize, Twiddles<T> tw) {
-  constexpr int TT = N / R;
+  using G = FftShape<T, N>;
+  constexpr int R = G::R, TT = G::TT, ROWS = G::ROWS;
   constexpr int LSZ = Padded<N, R>::size;
   __shared__ cplx<T> lds[ROWS * LSZ];
   const int tid = threadIdx.x;
   const int team = tid / TT, t = tid % TT;
   const int row = blockIdx.x * ROWS + team;
   const bool active = row < rows;
-  cplx<T>* W = reinterpret_cast<cplx<T>*>(data) + size_t(active ? row : 0) * N;
+  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data)) + size_t(active ? row : 0) * N;
   LdsRow<T> view{lds + team * LSZ};
+  TwRegs<T, N, R> twr;
+  load_twiddles<T, N, R>(twr, t, tw);
   cplx<T> v[R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = active ? W[t + j * TT] : cplx<T>{T(0), T(0)};
-  team_fft<T, N, R, DIR>(v, t, view, tw);
+  for (int j = 0; j < R; ++j) v[j] = gload(W + t + j * TT);
+  team_fft<T, N, R, DIR, LdsRow<T>, typename G::Sync>(v, t, view, twr);
   const T f = normalize ? T(1.0 / N) : T(1);
   if (active) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) W[t + j * TT] = cscale(v[j], f);
+    for (int j = 0; j < R; ++j) store_cached(W + t + j * TT, cscale(v[j], f));
   }
 }
 
-template <typename T, int N, int R, int C, int DIR>
-__global__ void __launch_bounds__(C*(N / R))
+// Loads and stores cover rows of C consecutive columns; a wave's team takes its column over at the
+// first exchange and hands it back before the store.
+template <typename T, int N, int DIR>
+__global__ void __launch_bounds__((FftShape<T, N>::C * FftShape<T, N>::TT))
     fft_cols_kernel(void* data, int X, int normalize, Twiddles<T> tw) {
-  constexpr int TT = N / R;
-  constexpr int LSZ = Padded<N, R>::size;
+  using G = FftShape<T, N>;
+  constexpr int R = G::R, TT = G::TT, C = G::C;
+  constexpr int LSZ = N + N / R + col_pad<T, C>();
   __shared__ cplx<T> lds[C * LSZ];
   const int tid = threadIdx.x;
-  const int c = tid % C, t = tid / C;
-  const int col = blockIdx.x * C + c;
-  cplx<T>* W = reinterpret_cast<cplx<T>*>(data);
-  LdsStrided<T, C> view{lds + c};
-  const unsigned boff = (unsigned(t) * unsigned(X) + unsigned(col)) * unsigned(sizeof(cplx<T>));
+  const int cl = tid % C, tl = tid / C;
+  const int cc = G::kWave ? tid / TT : cl, tc = G::kWave ? tid % TT : tl;
+  // neighbouring tiles, which share 128-byte lines, on one XCD
+  const int nt = int(gridDim.x), b = int(blockIdx.x);
+  const int tile = nt % 8 == 0 ? (b % 8) * (nt / 8) + b / 8 : b;
+  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data));
+  const unsigned boff = (unsigned(tl) * unsigned(X) + unsigned(tile * C + cl)) * unsigned(sizeof(cplx<T>));
+  TwRegs<T, N, R> twr;
+  load_twiddles<T, N, R>(twr, tc, tw);
   cplx<T> v[R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = *reinterpret_cast<cplx<T>*>(reinterpret_cast<char*>(W + size_t(j * TT) * X) + boff);
-  team_fft<T, N, R, DIR>(v, t, view, tw);
+  for (int j = 0; j < R; ++j) v[j] = gload(at_off(W + size_t(j * TT) * X, boff));
+  if constexpr (G::kWave) {
+    const LdsRow<T> view_l{lds + cl * LSZ}, view_c{lds + cc * LSZ};
+    team_fft_remap<T, N, R, DIR>(v, tl, view_l, tc, view_c, twr);
+    WaveSync::sync();
+#pragma unroll
+    for (int j = 0; j < R; ++j) *view_c.ptr(padr<R>(tc + j * TT)) = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; ++j) v[j] = *view_l.ptr(padr<R>(tl + j * TT));
+  } else {
+    team_fft<T, N, R, DIR, LdsStrided<T, C>, BlockSync>(v, tl, LdsStrided<T, C>{lds + cl}, twr);
+  }
   const T f = normalize ? T(1.0 / N) : T(1);
 #pragma unroll
-  for (int j = 0; j < R; ++j)
-    *reinterpret_cast<cplx<T>*>(reinterpret_cast<char*>(W + size_t(j * TT) * X) + boff) = cscale(v[j], f);
+  for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), cscale(v[j], f));
 }
 
 // ------------------------------------------------------------------ launchers
 namespace {
 constexpr int kR = 16;
-template <int N>
-constexpr int fft_rows_per_block() {
-  return (256 / (N / kR)) < 1 ? 1 : 256 / (N / kR);
-}
+// columns a plan's batch has to be a multiple of (a multiple of every kernel's C)
 template <typename T, int N>
 constexpr int fft_cols_per_block() {
   constexpr int c = 256 / (N / kR);
+  static_assert((c > 64 ? 64 : c) % FftShape<T, N>::C == 0, "whole tiles");
   return c < 1 ? 1 : (c > 64 ? 64 : c);
 }
 template <typename T, int N, int DIR>
 hipError_t fft_rows_n(void* d, int rows, int norm, Twiddles<T> tw, hipStream_t s) {
-  constexpr int ROWS = fft_rows_per_block<N>();
-  hipLaunchKernelGGL((fft_rows_kernel<T, N, kR, ROWS, DIR>), dim3((rows + ROWS - 1) / ROWS),
-                     dim3(ROWS * (N / kR)), 0, s, d, rows, norm, tw);
+  using G = FftShape<T, N>;
+  hipLaunchKernelGGL((fft_rows_kernel<T, N, DIR>), dim3((rows + G::ROWS - 1) / G::ROWS), dim3(G::ROWS * G::TT), 0, s,
+                     d, rows, norm, tw);
   return hipGetLastError();
 }
 template <typename T, int N, int DIR>
 hipError_t fft_cols_n(void* d, int X, int norm, Twiddles<T> tw, hipStream_t s) {
-  constexpr int C = fft_cols_per_block<T, N>();
-  hipLaunchKernelGGL((fft_cols_kernel<T, N, kR, C, DIR>), dim3(X / C), dim3(C * (N / kR)), 0, s, d, X,
-                     norm, tw);
+  using G = FftShape<T, N>;
+  hipLaunchKernelGGL((fft_cols_kernel<T, N, DIR>), dim3(X / G::C), dim3(G::C * G::TT), 0, s, d, X, norm, tw);
   return hipGetLastError();
 }
 #define WH_FFT_SWITCH(N, CALL)         \
