@@ -60,10 +60,11 @@ int odm_cols_per_tile(int P);
 int odm_radix();
 int odm_block();
 hipError_t launch_odm(int prec, int kind, const SweepArgs& a, int nwork, double weight, double sgn, hipStream_t s);
-hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s);
+hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks, int tiles, int parity, hipStream_t s);
 hipError_t launch_dirac_psweep(int prec, int P, bool cl, const DiracPlan* d, int nblocks, hipStream_t s);
 hipError_t launch_dirac_colsum(int prec, const DiracPlan* d, int X, hipStream_t s);
-hipError_t launch_dirac_reduce(const DiracPlan* d, int state_add, int renorm, int anti, int inc, hipStream_t s);
+hipError_t launch_dirac_reduce(const DiracPlan* d, int state_add, int renorm, int anti, int inc, int parity,
+                               hipStream_t s);
 hipError_t launch_dirac_expr_table(const DiracPlan* d, int cells, int depth, hipStream_t s);
 hipError_t launch_dirac_expr_obs(const DiracPlan* d, int X, int depth, int state_add, hipStream_t s);
 hipError_t launch_dirac_mass_table(const DiracPlan* d, int cells, int depth, hipStream_t s);
@@ -78,6 +79,7 @@ hipError_t launch_dirac_podm(int prec, const DiracPlan* d, int nblocks, hipStrea
 hipError_t launch_dirac_fsweep(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s);
 hipError_t launch_dirac_gpshift(const DiracPlan* d, int nblocks, hipStream_t s);
 int dirac_p_blocks(int X, int P);
+int dirac_p_tiles(int X, int P);
 }  // namespace wh
 
 namespace {
@@ -1456,12 +1458,13 @@ struct wh_dirac {
   wh_dirac_desc d{};
   wh::DiracPlan host{};  // host mirror of the device plan
   DevBuf plan_dev, pot, pot_dv, theta_decay, xmask, x_host, p_host, theta_host, dv0, vsum, mass_dm, mass_sm;
-  DevBuf colsums, rowpart, scale, step, rho, G, lambda_host, acoef_rows, pot_expr, dpot_expr, mass_expr;
+  DevBuf colsums, rowpart, tilepart, scale, step, rho, G, lambda_host, acoef_rows, pot_expr, dpot_expr, mass_expr;
   DevBuf a_expr[3], a_tab, asum;
   TwSet twx, twp;
   int xblocks = 0, pblocks = 0, gpblocks = 0, pgblocks = 0;
   hipStream_t capture_stream = nullptr;
   std::map<std::tuple<hipStream_t, int>, GraphEntry> graphs;
+  bool joined = false;  // the record rides on the next kinetic sweep
   int graph_chunk = 16;
   bool plan_uploaded = false;
   ~wh_dirac() {
@@ -1531,7 +1534,7 @@ int dirac_validate(const wh_dirac_desc* d) {
 // A = 0 with ODM damping (one sweep over plane quads).
 // The record row and normalisation of the state at time index step + state_add; with a V0
 // program, its dV0/dx and V0 at that time first.
-int dirac_reduce(wh_dirac* e, int state_add, int renorm, int anti, int inc, hipStream_t s) {
+int dirac_reduce(wh_dirac* e, int state_add, int renorm, int anti, int inc, hipStream_t s, int parity = 0) {
   const auto* dp = e->plan_dev.as<wh::DiracPlan>();
   if (e->host.pot_expr_len > 0) {
     const int depth = std::max(e->host.pot_expr_depth, e->host.dpot_expr_depth);
@@ -1539,7 +1542,7 @@ int dirac_reduce(wh_dirac* e, int state_add, int renorm, int anti, int inc, hipS
   }
   if (e->host.asum)
     WH_LAUNCH(wh::launch_dirac_a_sum(dp, e->d.x_dim, e->host.a_expr_depth, state_add, s), "dirac_a_sum");
-  WH_LAUNCH(wh::launch_dirac_reduce(dp, state_add, renorm, anti, inc, s), "dirac_reduce");
+  WH_LAUNCH(wh::launch_dirac_reduce(dp, state_add, renorm, anti, inc, parity, s), "dirac_reduce");
   return WH_SUCCESS;
 }
 
@@ -1574,12 +1577,15 @@ int dirac_potential_sweep(wh_dirac* e, hipStream_t s) {
 }
 
 // One iteration: kinetic sweep, potential sweep, observables of the new state + renormalisation.
-int dirac_iteration(wh_dirac* e, hipStream_t s) {
+// Joined plans (e->joined) leave the latter to the next iteration's kinetic sweep (behind: there is
+// an iteration before this one; the run closes with a reduce); parity alternates.
+int dirac_iteration(wh_dirac* e, hipStream_t s, int behind = 0, int parity = 0) {
   const auto* dp = e->plan_dev.as<wh::DiracPlan>();
   const int prec = e->d.precision;
   if (e->d.gp_coeff != 0.0) WH_LAUNCH(wh::launch_dirac_gpshift(dp, e->gpblocks, s), "dirac_gpshift");
-  WH_LAUNCH(wh::launch_dirac_xsweep(prec, e->d.x_dim, dp, e->xblocks, s), "dirac_xsweep");
+  WH_LAUNCH(wh::launch_dirac_xsweep(prec, e->d.x_dim, dp, e->xblocks, behind, parity, s), "dirac_xsweep");
   WH_TRY(dirac_potential_sweep(e, s));
+  if (e->joined) return WH_SUCCESS;
   if (e->host.filter) {
     // antiparticle step filter and the absorber after it; the record then needs the column
     // sums of the filtered state
@@ -1590,8 +1596,9 @@ int dirac_iteration(wh_dirac* e, hipStream_t s) {
   return WH_SUCCESS;
 }
 
-int dirac_iterations(wh_dirac* e, int count, hipStream_t s) {
-  for (int k = 0; k < count; ++k) WH_TRY(dirac_iteration(e, s));
+// `count` iterations, of which the first has index `first` of its run.
+int dirac_iterations(wh_dirac* e, int first, int count, hipStream_t s) {
+  for (int k = first; k < first + count; ++k) WH_TRY(dirac_iteration(e, s, e->joined && k > 0, e->joined ? k & 1 : 0));
   return WH_SUCCESS;
 }
 
@@ -1607,7 +1614,8 @@ int dirac_ensure_graph(wh_dirac* e, hipStream_t s, hipGraphExec_t* exec) {
       WH_HIP(hipStreamCreateWithFlags(&e->capture_stream, hipStreamNonBlocking), "hipStreamCreate");
     GraphEntry g;
     WH_HIP(hipStreamBeginCapture(e->capture_stream, hipStreamCaptureModeThreadLocal), "BeginCapture");
-    const int rc = dirac_iterations(e, chunk, e->capture_stream);
+    // from index 1: an odd parity first, and an even number of iterations
+    const int rc = dirac_iterations(e, 1, chunk, e->capture_stream);
     const hipError_t err = hipStreamEndCapture(e->capture_stream, &g.graph);
     if (rc) {
       if (g.graph) (void)hipGraphDestroy(g.graph);
@@ -1622,15 +1630,15 @@ int dirac_ensure_graph(wh_dirac* e, hipStream_t s, hipGraphExec_t* exec) {
   return WH_SUCCESS;
 }
 
-// Replays `count` iterations from the step graph (whole chunks), the rest launched directly.
+// The run's iterations from index 1 on: whole chunks replayed from the step graph, the rest launched
+// directly.
 int dirac_run_graph(wh_dirac* e, int count, hipStream_t s) {
   hipGraphExec_t exec = nullptr;
   WH_TRY(dirac_ensure_graph(e, s, &exec));
-  while (count >= e->graph_chunk) {
+  int first = 1;
+  for (; count >= e->graph_chunk; count -= e->graph_chunk, first += e->graph_chunk)
     WH_HIP(hipGraphLaunch(exec, s), "GraphLaunch");
-    count -= e->graph_chunk;
-  }
-  return dirac_iterations(e, count, s);
+  return dirac_iterations(e, first, count, s);
 }
 
 }  // namespace
@@ -1682,7 +1690,8 @@ extern "C" int wh_dirac_create(const wh_dirac_desc* desc, wh_dirac** out) {
   WH_TRY(e->p_host.upload(d.p_host, P * sizeof(double)));
   WH_TRY(e->theta_host.upload(d.theta_host, P * sizeof(double)));
   WH_TRY(e->colsums.alloc(X * wh::kDNCol * sizeof(double)));
-  WH_TRY(e->rowpart.alloc(2 * P * sizeof(double)));
+  WH_TRY(e->rowpart.alloc(4 * P * sizeof(double)));
+  WH_TRY(e->tilepart.alloc(size_t(wh::kDNPart) * X * sizeof(double)));
   const double one = 1.0;
   WH_TRY(e->scale.upload(&one, sizeof(one)));
   const int zero = 0;
@@ -1701,6 +1710,8 @@ extern "C" int wh_dirac_create(const wh_dirac_desc* desc, wh_dirac** out) {
   std::memset(&h, 0, sizeof(h));
   h.colsums = e->colsums.as<double>();
   h.rowpart = e->rowpart.as<double>();
+  h.tilepart = e->tilepart.as<double>();
+  h.ptiles = wh::dirac_p_tiles(d.x_dim, d.p_dim);
   h.scale = e->scale.as<double>();
   h.step = e->step.as<int>();
   h.pot = e->pot.as<double>();
@@ -1802,6 +1813,10 @@ extern "C" int wh_dirac_create(const wh_dirac_desc* desc, wh_dirac** out) {
   h.c_host = d.c_host;
   h.mc2_host = d.mc2_host;
   h.transmission_x = d.transmission_x;
+  // the record and factor of a step can be an item of the next x sweep where nothing between the
+  // sweeps needs them: no density of the Gross-Pitaevskii phase, no filter, and the diagonal
+  // potential sweep (which writes the tile sums) with dV0/dx known before it
+  e->joined = d.gp_coeff == 0.0 && !h.filter && !h.odm && !h.general && h.pot_expr_len == 0 && e->graph_chunk % 2 == 0;
   *out = e.release();
   return WH_SUCCESS;
 }
@@ -1838,7 +1853,8 @@ extern "C" int wh_dirac_kinetic(wh_dirac* e, void* W, void* stream) {
   if (!W) return fail(WH_INVALID_VALUE, "wh_dirac_kinetic: W is NULL");
   hipStream_t s = static_cast<hipStream_t>(stream);
   WH_TRY(dirac_bind(e, W, e->host.obs, e->host.obs_base, 0, true, s));
-  WH_LAUNCH(wh::launch_dirac_xsweep(e->d.precision, e->d.x_dim, e->plan_dev.as<wh::DiracPlan>(), e->xblocks, s), "dirac_xsweep");
+  WH_LAUNCH(wh::launch_dirac_xsweep(e->d.precision, e->d.x_dim, e->plan_dev.as<wh::DiracPlan>(), e->xblocks, 0, 0, s),
+            "dirac_xsweep");
   return WH_SUCCESS;
 }
 
@@ -1869,10 +1885,12 @@ extern "C" int wh_dirac_run(wh_dirac* e, void* W, int first_step, int n_steps, d
     hipGraphExec_t exec = nullptr;
     WH_TRY(dirac_ensure_graph(e, s, &exec));  // ready for a later, longer run
   }
-  if (graph_pays(e->graph_chunk, use_graph, n_steps))
-    WH_TRY(dirac_run_graph(e, n_steps, s));
-  else
-    WH_TRY(dirac_iterations(e, n_steps, s));
+  WH_TRY(dirac_iterations(e, 0, std::min(n_steps, 1), s));
+  if (graph_pays(e->graph_chunk, use_graph, n_steps - 1))
+    WH_TRY(dirac_run_graph(e, n_steps - 1, s));
+  else if (n_steps > 1)
+    WH_TRY(dirac_iterations(e, 1, n_steps - 1, s));
+  if (e->joined && n_steps > 0) WH_TRY(dirac_reduce(e, 1, 1, 1, 1, s, (n_steps - 1) & 1));
   WH_LAUNCH(wh::launch_dirac_finish(storage_code(e->d.precision), dp, e->d.p_dim, s), "dirac_finish");
   return WH_SUCCESS;
 }

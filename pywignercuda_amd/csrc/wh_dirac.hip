@@ -107,7 +107,8 @@ __device__ __forceinline__ void pin(cplx<T> (&v)[R]) {
 }
 
 template <typename S, typename T, int N, bool FILTER = false>
-__device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block, cplx<T>* lds, cplx<double>* tab) {
+__device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block, bool tiles, int parity, cplx<T>* lds,
+                                                  cplx<double>* tab, double* red) {
   using G = DiracX<N>;
   constexpr int R = G::R, TT = G::TT, ROWS = G::ROWS;
   const int tid = threadIdx.x, team = tid / TT, t = tid % TT;
@@ -120,7 +121,11 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
   const Twiddles<T> tw{reinterpret_cast<const cplx<T>*>(d.twX_hi), reinterpret_cast<const cplx<T>*>(d.twX_lo)};
   LdsRow<T> view{lds + team * G::LSZ};
   using Sync = std::conditional_t<(TT <= 64), WaveSync, BlockSync>;
-  const double s = FILTER ? 1.0 : *gmem(d.scale);
+  // the pending factor: in d.scale, or from the tiles' norms (the record item computes the same)
+  double s = 1.0, part = 0.0;
+  if (!FILTER && !tiles) s = *gmem(d.scale);
+  const gptr<const double> norms = gmem(d.tilepart) + size_t(kDoNorm) * N;
+  if (!FILTER && tiles && tid < d.ptiles) part = norms[tid];
   // planes of group g = 2 (row pair) + (column pair), in the order [r1 c1, r1 c2, r2 c1, r2 c2]:
   // row pairs {0, 3}, {1, 2} of spinor rows, the same of columns
   const int gr = group >> 1, gc = group & 1;
@@ -168,7 +173,18 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
     team_fft<T, N, R, -1, LdsRow<T>, Sync>(v[q], t, view, twr);
     pin(v[q]);
   }
+  if (!FILTER && tiles) {
+    for (int i = tid + G::BLOCK; i < d.ptiles; i += G::BLOCK) part += norms[i];
+    part = group_sum<64>(part);
+    if (tid % 64 == 63) red[tid / 64] = part;
+  }
   __syncthreads();
+  if (!FILTER && tiles) {
+    double n = 0.0;
+#pragma unroll
+    for (int w = 0; w < G::BLOCK / 64; ++w) n += red[w];
+    s = 1.0 / (d.dxdp * n);
+  }
 
   const double p = d.dp * double(fidx(row, d.P));
   if (!FILTER && d.antiparticle && (group == 0 || group == 3) && t == 0) {
@@ -177,7 +193,7 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
     const double e2 = 2.0 * sqrt(d.proj_mc2 * d.proj_mc2 + d.proj_c * d.proj_c * p * p);
     const double aa = 0.5 - d.proj_mc2 / e2, bb = -d.proj_c * p / e2, dd = 0.5 + d.proj_mc2 / e2;
     const double c = aa * double(v[0][0].x) + bb * (double(v[1][0].x) + double(v[2][0].x)) + dd * double(v[3][0].x);
-    gmem(d.rowpart)[(group == 0 ? 0 : 1) * d.P + row] = s * c;
+    gmem(d.rowpart)[(2 * parity + (group == 0 ? 0 : 1)) * d.P + row] = s * c;
   }
 
   // the pending factor and the 1/N of the inverse transform ride on the left factor
@@ -307,7 +323,7 @@ __device__ __forceinline__ bool dirac_col_owned(int part, int q) {
 }
 template <int BLOCK, int C, typename L>
 __device__ __forceinline__ void dirac_store_colsums(const DiracPlan& d, int tile, double (&acc)[kDNCol], L* lds,
-                                                    int part = -1) {
+                                                    int part = -1, double* csum = nullptr) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int off = C; off < 64; off <<= 1) {
@@ -335,6 +351,114 @@ __device__ __forceinline__ void dirac_store_colsums(const DiracPlan& d, int tile
 #pragma unroll
     for (int q = 0; q < kDNCol; ++q)
       if (dirac_col_owned(part, q)) gmem(d.colsums)[size_t(tile * C + tid) * kDNCol + q] = sm[q];
+    if (csum) {
+#pragma unroll
+      for (int q = 0; q < kDNCol; ++q) csum[tid * kDNCol + q] = sm[q];
+    }
+  }
+}
+
+// dV0/dx and V0 of coefficient row tstate at x
+__device__ __forceinline__ void dirac_host_poly(const DiracPlan& d, int tstate, double x, double& dv, double& vs) {
+  const int prow = tstate < d.pot_rows ? tstate : d.pot_rows - 1;
+  const cptr<double> cf = cmem(d.pot) + size_t(prow) * (kMaxDeg + 1);
+  dv = 0.0;
+  for (int n = d.pot_deg; n >= 1; --n) dv = fma(dv, x, double(n) * cf[n]);
+  vs = cf[d.pot_deg];
+  for (int n = d.pot_deg - 1; n >= 0; --n) vs = fma(vs, x, cf[n]);
+}
+
+// Record sums of a p sweep tile (one wave): lane c forms the terms of column c from its sums in csum
+// (of this quarter's kind), a group sum adds the columns.  The record of a step is then the sum of a
+// few hundred tiles, an item of the next x sweep, instead of a launch of its own over all columns
+// (10.5 us of a 70 us step at 512^2).
+template <int C>
+__device__ __forceinline__ void dirac_tile_partial(const DiracPlan& d, int tile, int quarter, int tstate,
+                                                   const double* csum, double dv, double vs) {
+  const int c = threadIdx.x % C;
+  const double* s = csum + c * kDNCol;
+  const double x = d.dx * double(fidx(tile * C + c, d.X));
+  const bool last = threadIdx.x == C - 1;
+  auto put = [&](int slot, double v) {
+    v = group_sum<C>(v);
+    if (last) gmem(d.tilepart)[size_t(slot) * d.X + tile] = v;
+  };
+  if (quarter == 0) {
+    if (d.pot_deg >= 0) dirac_host_poly(d, tstate, x, dv, vs);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const double tr = s[kDcTrRe + r], ptr = s[kDcPTrRe + r];
+      put(kDoX + r, x * tr);
+      put(kDoP + r, ptr);
+      put(kDoXP + r, x * ptr);
+      put(kDoXX + r, x * x * tr);
+      put(kDoPP + r, s[kDcP2TrRe + r]);
+      put(kDoDV + r, dv * tr);
+      put(kDoXDV + r, x * dv * tr);
+      put(kDoPDV + r, dv * ptr);
+      put(kDoEnergy + r, d.mc2_host * s[kDcBetaRe + r] + vs * tr);
+    }
+    put(kDoNeg, s[kDcNeg]);
+    put(kDoTrans, x > d.transmission_x ? s[kDcTrRe] : 0.0);
+    put(kDoNorm, s[kDcTrRe]);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      put(kDoA1 + r, s[kDcA1Re + r]);
+      put(kDoPA1 + r, s[kDcPA1Re + r]);
+      put(kDoXA1 + r, x * s[kDcA1Re + r]);
+      put(kDPartHA1 + r, d.c_host * s[kDcHA1Re + r]);
+    }
+  }
+}
+
+// The record of the state that the last p sweep left (one block beside the x sweep's): the row of
+// time index step + 1, the antiparticle entry of the row before from the last x sweep's row sums
+// (of parity `parity`), and the step index.
+template <int BLOCK>
+__device__ __forceinline__ void dirac_record_item(const DiracPlan& d, int parity, double* red) {
+  constexpr int W = BLOCK / 64, K = (kDNPart + W - 1) / W;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int step = *cmem(d.step);
+  double r[K], a = 0.0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) r[k] = 0.0;
+  for (int i = lane; i < d.ptiles; i += 64) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int slot = wave + k * W;
+      if (slot < kDNPart && slot != kDoAnti) r[k] += gmem(d.tilepart)[size_t(slot) * d.X + i];
+    }
+  }
+  if (d.antiparticle) {
+    for (int i = tid; i < 2 * d.P; i += BLOCK) a += gmem(d.rowpart)[2 * parity * d.P + i];
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int slot = wave + k * W;
+    const double t = group_sum<64>(r[k]);
+    if (lane == 63 && slot < kDNPart) red[slot] = t;
+  }
+  a = group_sum<64>(a);
+  if (lane == 63) red[kDNPart + wave] = a;
+  __syncthreads();
+  const double raw = d.dxdp * red[kDoNorm], f = 1.0 / raw;
+  double* o = d.obs + size_t(step + 1 - d.obs_base) * kDNObs;
+  if (tid < kDoAnti) {
+    double t = red[tid];
+    if (tid >= kDoEnergy && tid < kDoNeg) t = d.energy ? t + red[kDPartHA1 + tid - kDoEnergy] : 0.0;
+    gmem(o)[tid] = f * d.dxdp * t;
+  }
+  if (tid == 0) {
+    gmem(o)[kDoNorm] = f * raw;
+    gmem(o)[kDoRawNorm] = raw;
+    if (d.antiparticle) {
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) t += red[kDNPart + w];
+      gmem(o)[kDoAnti - kDNObs] = d.dxdp * t;
+    }
+    *gmem(const_cast<int*>(d.step)) = step + 1;
   }
 }
 
@@ -372,7 +496,8 @@ struct DiracP {
 };
 
 template <typename S, typename T, int N, bool CL>
-__device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, int quarter, cplx<T>* lds, T* tab) {
+__device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, int quarter, cplx<T>* lds, T* tab,
+                                                  double* csum) {
   using G = DiracP<N, CL>;
   constexpr int R = G::R, TT = G::TT, C = G::C, LSZ = G::LSZ;
   constexpr bool kWave = G::kWave;
@@ -424,6 +549,11 @@ __device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, 
   }
   double dvx = 0.0;
   if (d.kvn && d.pot_deg < 0) dvx = gmem(d.dv0)[col];
+  double host_dv = 0.0, host_v = 0.0;  // dV0/dx and sum V of column tid % C (tables)
+  if (quarter == 0 && d.pot_deg < 0) {
+    host_dv = gmem(d.dv0)[tile * C + tid % C];
+    host_v = gmem(d.vsum)[tile * C + tid % C];
+  }
   // Re tr W of each element (quarter 0), or its p_host (quarter 1)
   double aux[R];
 #pragma unroll
@@ -599,15 +729,16 @@ __device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, 
     neg = group_sum<TT>(neg);
     if (tc == TT - 1) {
       const gptr<double> cs = gmem(d.colsums) + size_t(col) * kDNCol;
+      double* ls = csum + cc * kDNCol;
       if (quarter == 0) {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) cs[kDcTrRe + q] = acc[q];
-        cs[kDcBetaRe] = acc[6];
-        cs[kDcBetaIm] = acc[7];
-        cs[kDcNeg] = neg;
+        for (int q = 0; q < 6; ++q) cs[kDcTrRe + q] = ls[kDcTrRe + q] = acc[q];
+        cs[kDcBetaRe] = ls[kDcBetaRe] = acc[6];
+        cs[kDcBetaIm] = ls[kDcBetaIm] = acc[7];
+        cs[kDcNeg] = ls[kDcNeg] = neg;
       } else {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) cs[kDcA1Re + q] = acc[q];
+        for (int q = 0; q < 6; ++q) cs[kDcA1Re + q] = ls[kDcA1Re + q] = acc[q];
       }
     }
   } else {
@@ -622,8 +753,10 @@ __device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, 
     all[kDcBetaRe] = acc[6];
     all[kDcBetaIm] = acc[7];
     all[kDcNeg] = neg;
-    dirac_store_colsums<G::BLOCK, C>(d, tile, all, lds, quarter);
+    dirac_store_colsums<G::BLOCK, C>(d, tile, all, lds, quarter, csum);
   }
+  __syncthreads();
+  if (tid < 64) dirac_tile_partial<C>(d, tile, quarter, step + 1, csum, host_dv, host_v);
 }
 
 // ------------------------------------------------------------------ p sweeps with vector potentials
@@ -969,11 +1102,16 @@ __device__ __forceinline__ int dirac_col_tile() {
 // largest one's occupancy.
 template <typename S, typename T, int N, bool FILTER>
 __global__ void __launch_bounds__(DiracX<N>::BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
-dirac_xsweep_kernel(const DiracPlan* __restrict__ dp) {
+dirac_xsweep_kernel(const DiracPlan* __restrict__ dp, int tiles, int parity) {
   using G = DiracX<N>;
   __shared__ cplx<T> lds[G::kTeams * G::LSZ];
   __shared__ cplx<double> tab[G::kTab];
-  dirac_xsweep_body<S, T, N, FILTER>(*dp, int(blockIdx.x), lds, tab);
+  __shared__ double red[kDNPart + G::BLOCK / 64];
+  if (!FILTER && tiles && blockIdx.x == gridDim.x - 1) {
+    dirac_record_item<G::BLOCK>(*dp, parity ^ 1, red);
+    return;
+  }
+  dirac_xsweep_body<S, T, N, FILTER>(*dp, int(blockIdx.x), tiles != 0, parity, lds, tab, red);
 }
 
 template <typename S, typename T, int N, bool CL>
@@ -983,9 +1121,10 @@ dirac_psweep_kernel(const DiracPlan* __restrict__ dp) {
   constexpr int kLds = G::kArrays * G::C * G::LSZ, kRed = G::BLOCK * kDNCol * 8 / int(sizeof(cplx<T>));
   __shared__ cplx<T> lds[!G::kWave && kRed > kLds ? kRed : kLds];
   __shared__ T tab[G::kTab];
+  __shared__ double csum[G::C * kDNCol];
   const DiracPlan& d = *dp;
   const int u = dirac_col_tile();
-  dirac_psweep_body<S, T, N, CL>(d, u >> 2, u & 3, lds, tab);
+  dirac_psweep_body<S, T, N, CL>(d, u >> 2, u & 3, lds, tab, csum);
 }
 
 template <typename S, typename T>
@@ -1090,7 +1229,7 @@ __global__ void __launch_bounds__(256) dirac_colsum_kernel(const DiracPlan* __re
 constexpr int kRedThreads = 256;
 constexpr int kRedQ = kDoNorm + 1;  // reduced quantities
 __global__ void __launch_bounds__(kRedThreads) dirac_reduce_kernel(const DiracPlan* __restrict__ dp, int state_add,
-                                                                   int renorm, int anti, int inc) {
+                                                                   int renorm, int anti, int inc, int parity) {
   const DiracPlan& d = *dp;
   __shared__ double red[kRedThreads][kRedQ + 1];
   const int step = *gmem(d.step);
@@ -1144,7 +1283,8 @@ __global__ void __launch_bounds__(kRedThreads) dirac_reduce_kernel(const DiracPl
   // antiparticle population from the row contributions of the loaded state (normalised)
   double a = 0.0;
   if (anti && d.antiparticle) {
-    for (int r = threadIdx.x; r < d.P; r += kRedThreads) a += gmem(d.rowpart)[r] + gmem(d.rowpart)[d.P + r];
+    const gptr<const double> rows = gmem(d.rowpart) + 2 * parity * d.P;
+    for (int r = threadIdx.x; r < d.P; r += kRedThreads) a += rows[r] + rows[d.P + r];
   }
   // per-wave sums (fixed xor trees), then the waves in order: red[0][q] holds the totals
   constexpr int kWaves = kRedThreads / 64;
@@ -1285,24 +1425,29 @@ int dirac_p_blocks(int X, int P) {
 }
 
 template <typename S, typename T, bool FILTER>
-hipError_t dirac_x_launch(int X, const DiracPlan* d, int nblocks, hipStream_t s) {
-#define BODY(n) \
-  hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, n, FILTER>), dim3(nblocks), dim3(DiracX<n>::BLOCK), 0, s, d)
+hipError_t dirac_x_launch(int X, const DiracPlan* d, int nblocks, int tiles, int parity, hipStream_t s) {
+#define BODY(n)                                                                                                     \
+  hipLaunchKernelGGL((dirac_xsweep_kernel<S, T, n, FILTER>), dim3(nblocks + (tiles ? 1 : 0)), dim3(DiracX<n>::BLOCK), 0, \
+                     s, d, tiles, parity)
   WH_DIRAC_DISPATCH(X, BODY)
 #undef BODY
   return hipGetLastError();
 }
 
 template <bool FILTER>
-hipError_t dirac_x_launch_prec(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s) {
-  if (prec == 0) return dirac_x_launch<double, double, FILTER>(X, d, nblocks, s);
-  if (prec == 1) return dirac_x_launch<float, float, FILTER>(X, d, nblocks, s);
-  return dirac_x_launch<float, double, FILTER>(X, d, nblocks, s);
+hipError_t dirac_x_launch_prec(int prec, int X, const DiracPlan* d, int nblocks, int tiles, int parity, hipStream_t s) {
+  if (prec == 0) return dirac_x_launch<double, double, FILTER>(X, d, nblocks, tiles, parity, s);
+  if (prec == 1) return dirac_x_launch<float, float, FILTER>(X, d, nblocks, tiles, parity, s);
+  return dirac_x_launch<float, double, FILTER>(X, d, nblocks, tiles, parity, s);
 }
 
-hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s) {
-  return dirac_x_launch_prec<false>(prec, X, d, nblocks, s);
+// tiles: the factor and the record of the state come from the last p sweep's tiles; parity: of the
+// iteration (the row sums of the one before are read meanwhile)
+hipError_t launch_dirac_xsweep(int prec, int X, const DiracPlan* d, int nblocks, int tiles, int parity, hipStream_t s) {
+  return dirac_x_launch_prec<false>(prec, X, d, nblocks, tiles, parity, s);
 }
+
+int dirac_p_tiles(int X, int P) { return dirac_p_blocks(X, P) / 4; }
 
 template <typename S, typename T, bool CL>
 hipError_t dirac_p_launch(int P, const DiracPlan* d, int nblocks, hipStream_t s) {
@@ -1354,7 +1499,7 @@ hipError_t launch_dirac_pgeneral(int prec, bool cl, const DiracPlan* d, int nblo
 }
 
 hipError_t launch_dirac_fsweep(int prec, int X, const DiracPlan* d, int nblocks, hipStream_t s) {
-  return dirac_x_launch_prec<true>(prec, X, d, nblocks, s);
+  return dirac_x_launch_prec<true>(prec, X, d, nblocks, 0, 0, s);
 }
 
 hipError_t launch_dirac_podm(int prec, const DiracPlan* d, int nblocks, hipStream_t s) {
@@ -1387,8 +1532,9 @@ hipError_t launch_dirac_gpshift(const DiracPlan* d, int nblocks, hipStream_t s) 
   return hipGetLastError();
 }
 
-hipError_t launch_dirac_reduce(const DiracPlan* d, int state_add, int renorm, int anti, int inc, hipStream_t s) {
-  hipLaunchKernelGGL(dirac_reduce_kernel, dim3(1), dim3(kRedThreads), 0, s, d, state_add, renorm, anti, inc);
+hipError_t launch_dirac_reduce(const DiracPlan* d, int state_add, int renorm, int anti, int inc, int parity,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(dirac_reduce_kernel, dim3(1), dim3(kRedThreads), 0, s, d, state_add, renorm, anti, inc, parity);
   return hipGetLastError();
 }
 

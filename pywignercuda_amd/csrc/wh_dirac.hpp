@@ -36,10 +36,15 @@ enum DiracObs {
   kDoNeg = 24, kDoTrans = 25, kDoAnti = 26, kDoNorm = 27, kDoRawNorm = 28
 };
 
+// Record sums of a tile's columns: DiracObs slots (the energy without its alpha_1 term, which the
+// tile's other block writes to two slots of its own).
+constexpr int kDPartHA1 = kDoRawNorm, kDNPart = kDPartHA1 + 2;
+
 struct DiracPlan {
   void* W;                     // [16][P][X]
   double* colsums;             // [X][kDNCol]
-  double* rowpart;             // [2][P] antiparticle contributions of plane groups 0 and 3
+  double* rowpart;             // [2][2][P] antiparticle contributions of plane groups 0 and 3, by iteration parity
+  double* tilepart;            // [kDNPart][X] record sums of each p sweep tile
   double* scale;               // [1] pending real factor 1/norm, applied on the next load
   double* obs;                 // [rows][kDNObs]
   const int* step;             // device time index
@@ -63,6 +68,7 @@ struct DiracPlan {
   const void* twP_hi;
   const void* twP_lo;
   int X, P, pot_rows, pot_deg;
+  int ptiles, pad3;                 // p sweep tiles (entries in use of a tilepart row)
   int obs_base, energy, antiparticle, pad0;
   double dx, dp, dtheta, dlambda;   // kernel steps ('%f')
   double mh_c;                      // mass_half * c          (kinetic shell)
