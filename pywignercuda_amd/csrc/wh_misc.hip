@@ -245,7 +245,7 @@ struct FftShape {
   static constexpr int R = N <= 512 ? 8 : 16, TT = N / R;
   static constexpr bool kWave = TT <= 64;
   static constexpr int ROWS = TT >= 64 ? 1 : 64 / TT;             // rows per block
-  static constexpr int C = N <= 512 ? 8 : N <= 1024 ? 4 : 2;      // columns per block
+  static constexpr int C = N <= 64 ? 8 : N <= 1024 ? 4 : 2;      // columns per block
   using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
 };
 
