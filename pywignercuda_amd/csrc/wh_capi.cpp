@@ -512,6 +512,24 @@ bool fits_all(const wh_ensemble* e, const wh::SweepVariant& v, bool x_axis, bool
   return true;
 }
 
+// The narrow form to take in place of variant v of table t (n entries to choose from, all entries), or
+// v: the widest form of its radix that gives every CU a block, or else the narrowest that fits.
+int narrowed(const wh_ensemble* e, const wh::SweepVariant* t, int n, int all, int v, bool x_axis, bool cl = false) {
+  if (t[v].tp || t[v].block != 256) return v;
+  size_t cells = 0;
+  for (const auto& m : e->mem) cells += size_t(m.X) * size_t(m.P);
+  const auto fills = [&](const wh::SweepVariant& w) { return cells / (size_t(w.R) * size_t(w.block)) >= size_t(wh::kCUs); };
+  for (int i = n; i < all && !fills(t[v]); ++i)  // (in order of their lanes)
+    if (t[i].R == t[v].R && t[i].block < t[v].block && fits_all(e, t[i], x_axis, cl)) v = i;
+  return v;
+}
+// (the x variant of a Gross-Pitaevskii plan also cuts its partial density sums: it stays)
+void narrow_variants(wh_ensemble* e) {
+  if (!e->gp()) e->xvar = narrowed(e, wh::kXVariants, wh::kNumX, wh::kAllX, e->xvar, true);
+  e->pvar = narrowed(e, wh::kPVariants, wh::kNumP, wh::kAllP, e->pvar, false);
+  e->pclvar = narrowed(e, wh::kPCLVariants, wh::kNumPCL, wh::kAllPCL, e->pclvar, false, true);
+}
+
 // p tiles of one variant, grouped by grid side (ascending), members in order within a size;
 // consecutive tiles of a member go to one XCD (blocks are dealt round-robin to the 8 XCDs)
 void p_tiles(const wh_ensemble* e, const wh::SweepVariant& pv, std::vector<unsigned>& wp) {
@@ -734,6 +752,7 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
   }
   WH_TRY(pick(wh::kPVariants, wh::kNumP, false, e->pvar));
   WH_TRY(pick(wh::kPCLVariants, wh::kNumPCL, false, e->pclvar, true));
+  narrow_variants(e.get());
   for (int i = 0; i < n; ++i) e->expr = e->expr || e->mem[i].pot_expr_len > 0;
   if (gp) {
     const wh::SweepVariant g{16, 256, 0};
@@ -1172,6 +1191,7 @@ extern "C" int wh_ensemble_set_variants(wh_ensemble* e, int xvar, int pvar, int 
   if (xvar >= 0) e->xvar = xvar;
   if (pvar >= 0) e->pvar = pvar;
   if (pclvar >= 0) e->pclvar = pclvar;
+  narrow_variants(e);
   return build_work_lists(e);
 }
 

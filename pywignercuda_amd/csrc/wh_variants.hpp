@@ -13,13 +13,20 @@ struct SweepVariant {
   int R, block, tp;
 };
 
-// index 0 is the default
-constexpr SweepVariant kXVariants[] = {{16, 256, 0}, {8, 256, 0}, {8, 512, 0}, {4, 256, 0}, {16, 256, 1}};
-constexpr SweepVariant kPVariants[] = {{16, 256, 0}, {8, 512, 0}, {8, 256, 0}, {16, 256, 1}};
-constexpr SweepVariant kPCLVariants[] = {{16, 256, 0}, {8, 256, 0}, {16, 256, 1}};
-constexpr int kNumX = sizeof(kXVariants) / sizeof(kXVariants[0]);
-constexpr int kNumP = sizeof(kPVariants) / sizeof(kPVariants[0]);
-constexpr int kNumPCL = sizeof(kPCLVariants) / sizeof(kPCLVariants[0]);
+// index 0 is the default.  The entries behind the first kNumX, kNumP, kNumPCL are narrow forms: a plan
+// takes one in place of the 256-lane form of its radix where its cells give that fewer blocks than
+// the chip has CUs (kCUs).  A block's exchanges share its CU's LDS pipe, so that a few wide blocks
+// wait for the LDS while other CUs are idle: the damped 128^2 step, 8 blocks of 256 lanes, takes 18.1
+// us, 32 blocks of 64 take 15.4; 256^2 18.9 and 15.7; 512 x 256 21.0 and 18.1.  Where 256-lane blocks
+// fill the CUs they are faster (whole 64-byte rows: 1024 x 512 31.6, with 128 lanes 33.9), and of the
+// narrow forms the widest that fills them (512^2: 23.6 with 256 lanes, 21.7 with 128, 22.8 with 64).
+constexpr SweepVariant kXVariants[] = {{16, 256, 0}, {8, 256, 0}, {8, 512, 0}, {4, 256, 0}, {16, 256, 1}, {8, 64, 0}, {4, 64, 0}};
+constexpr SweepVariant kPVariants[] = {{16, 256, 0}, {8, 512, 0}, {8, 256, 0}, {16, 256, 1}, {8, 128, 0}, {8, 64, 0}};
+constexpr SweepVariant kPCLVariants[] = {{16, 256, 0}, {8, 256, 0}, {16, 256, 1}, {8, 128, 0}, {8, 64, 0}};
+constexpr int kAllX = sizeof(kXVariants) / sizeof(kXVariants[0]), kNumX = kAllX - 2;
+constexpr int kAllP = sizeof(kPVariants) / sizeof(kPVariants[0]), kNumP = kAllP - 2;
+constexpr int kAllPCL = sizeof(kPCLVariants) / sizeof(kPCLVariants[0]), kNumPCL = kAllPCL - 2;
+constexpr int kCUs = 256;
 
 // largest grid side of the plain (x and p) throughput forms
 constexpr int kTpMaxN = 1024;
