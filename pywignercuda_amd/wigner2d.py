@@ -58,7 +58,15 @@ def _load_tuning():
 def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = False):
     """Variant indices (x, p, p+CL) chosen by pywignercuda_amd/tune.py for the largest grid.
 
-    batch: the plan holds enough cells to fill the GPU (the tuner's "batch" regime)."""
+    batch: the plan holds enough cells to fill the GPU (the tuner's "batch" regime).
+
+    The tuner times square grids.  A plan of a long side and few cells wants more lanes per
+    transform: up to 2^19 cells radix 16 leaves half of the chip's 1024 SIMDs without a wave
+    (us per step, complex128, radix 16 -> 8 in p, or in x -> 4 at 1024 and 8 at 2048: 256 x 1024
+    20.3 -> 17.3, with friction 32.7 -> 27.7, 128 x 2048 23.4 -> 20.3 and 46.7 -> 36.6, 1024 x 256
+    19.0 -> 17.5, 2048 x 128 21.2 -> 18.8; at 1024^2 radix 16 wins).  A complex128 state of 2^20 or
+    2^21 cells, which the L2s hold, wants radix 16 in x at every width (512 x 2048 39.7 -> 36.7,
+    2048 x 1024 51.6 -> 46.7; beyond them 2048^2 93.9 with radix 8, 104.6 with 16)."""
     tab = _load_tuning()
     t = tab.get(precision + "_batch", {}) if batch else {}
     if not t:
@@ -67,6 +75,13 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
     xv = t.get("x", {}).get(nx, -1)
     pv = t.get("p", {}).get(npp, -1)
     pcl = t.get("pcl", {}).get(npp, -1)
+    cells = sum(int(x) * int(p) for x, p in zip(sizes_x, sizes_p))
+    if t and not batch:
+        if cells <= 1 << 19:
+            pv, pcl = 2, 1  # radix 8
+            xv = {"1024": 3, "2048": 1}.get(nx, xv)  # radix 4, radix 8
+        elif precision == "fp64" and cells <= 1 << 21:
+            xv = 0  # radix 16
     return int(xv), int(pv), int(pcl)
 
 
