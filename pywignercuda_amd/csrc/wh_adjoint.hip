@@ -194,18 +194,25 @@ __global__ void __launch_bounds__(256) grad_reduce_kernel(const Member* members,
   }
 }
 
-// Adjoint tile geometry: radix 8, 256 lanes (two register arrays per lane).
-constexpr int kAdjR = 8, kAdjBlock = 256;
-int adj_cols(int P) { return kAdjBlock / (P / kAdjR); }
+// Adjoint tile geometry: radix 8 (two register arrays per lane), 256 lanes a block, or 128 where those
+// blocks would leave CUs idle (512^2: 11.3 -> 10.4 us a sweep).
+constexpr int kAdjR = 8;
+int adj_block(int X, int P) { return P <= 512 && X * P / (kAdjR * 256) < kCUs ? 128 : 256; }
+int adj_cols(int X, int P) { return adj_block(X, P) / (P / kAdjR); }
 size_t adj_moments(int X) { return size_t(X) * kAdjMom; }
 
-hipError_t launch_adj_psweep(int prec, const SweepArgs& a, const void* W_next, double* gcols, hipStream_t s) {
-  const dim3 g(a.ntiles), b(kAdjBlock);
-  if (prec == 0)
-    hipLaunchKernelGGL((adj_psweep_kernel<double, kAdjR, kAdjBlock>), g, b, 0, s, a, W_next, gcols);
+template <typename T>
+hipError_t adj_launch(int block, const SweepArgs& a, const void* W_next, double* gcols, hipStream_t s) {
+  if (block == 128)
+    hipLaunchKernelGGL((adj_psweep_kernel<T, kAdjR, 128>), dim3(a.ntiles), dim3(128), 0, s, a, W_next, gcols);
   else
-    hipLaunchKernelGGL((adj_psweep_kernel<float, kAdjR, kAdjBlock>), g, b, 0, s, a, W_next, gcols);
+    hipLaunchKernelGGL((adj_psweep_kernel<T, kAdjR, 256>), dim3(a.ntiles), dim3(256), 0, s, a, W_next, gcols);
   return hipGetLastError();
+}
+hipError_t launch_adj_psweep(int prec, int X, int P, const SweepArgs& a, const void* W_next, double* gcols,
+                             hipStream_t s) {
+  const int block = adj_block(X, P);
+  return prec == 0 ? adj_launch<double>(block, a, W_next, gcols, s) : adj_launch<float>(block, a, W_next, gcols, s);
 }
 
 hipError_t launch_grad_reduce(const Member* members, const double* gcols, int nsteps, double* grad, double scale,

@@ -50,10 +50,11 @@ hipError_t launch_set_scale(const Member* members, int nmembers, double re, doub
 hipError_t launch_fft_axis(int prec, int columns, int N, int dir, void* d, int batch, int norm,
                            const void* tw_hi, const void* tw_lo, hipStream_t s);
 int fft_cols_batch_multiple(int prec, int N);
-hipError_t launch_adj_psweep(int prec, const SweepArgs& a, const void* W_next, double* gcols, hipStream_t s);
+hipError_t launch_adj_psweep(int prec, int X, int P, const SweepArgs& a, const void* W_next, double* gcols,
+                             hipStream_t s);
 hipError_t launch_grad_reduce(const Member* members, const double* gcols, int nsteps, double* grad, double scale,
                               hipStream_t s);
-int adj_cols(int P);
+int adj_cols(int X, int P);
 size_t adj_moments(int X);
 int odm_rows_per_tile(int X);
 int odm_cols_per_tile(int P);
@@ -1350,7 +1351,7 @@ int check_adjoint(wh_ensemble* e) {
   if (e->d.precision == WH_C64_WIDE)
     return fail(WH_INVALID_TYPE, "the adjoint step runs on WH_C128 or WH_C64 states");
   const wh::Member& m = e->mem[0];
-  const int cols = wh::adj_cols(m.P);
+  const int cols = wh::adj_cols(m.X, m.P);
   if (cols < 1 || cols > 64 || m.X % cols != 0 || m.P < 128)
     return fail(WH_INVALID_SIZE, "adjoint sweep does not fit a %d x %d grid", m.P, m.X);
   return WH_SUCCESS;
@@ -1359,9 +1360,10 @@ int check_adjoint(wh_ensemble* e) {
 int adjoint_sweeps(wh_ensemble* e, void* Lambda, const void* W_next, int step, int k, hipStream_t s) {
   const wh::Member& m = e->mem[0];
   wh::SweepArgs a = sweep_args(e, 0, 1.0, step);
-  a.ntiles = m.X / wh::adj_cols(m.P);
+  a.ntiles = m.X / wh::adj_cols(m.X, m.P);
   a.W_dst = Lambda;
-  WH_LAUNCH(wh::launch_adj_psweep(e->d.precision, a, W_next, e->gcols.as<double>() + size_t(k) * wh::adj_moments(m.X), s),
+  WH_LAUNCH(wh::launch_adj_psweep(e->d.precision, m.X, m.P, a, W_next,
+                                  e->gcols.as<double>() + size_t(k) * wh::adj_moments(m.X), s),
             "adj_psweep");
   return xsweep(e, wh::kConj, s, Lambda, Lambda);
 }
