@@ -32,7 +32,7 @@ hipError_t launch_psweep_f64(int variant, bool cl, const SweepArgs& a, int nwork
 hipError_t launch_psweep_f32(int variant, bool cl, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_expr_table(const Member* members, int member, int X, int P, int depth, const int* step,
                              int step_add, int use_arg, double hbar_half, hipStream_t s);
-hipError_t launch_gpshift(const SweepArgs& a, int nwork, hipStream_t s);
+hipError_t launch_gpshift(bool narrow, const SweepArgs& a, int nwork, hipStream_t s);
 hipError_t launch_colsum(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s);
 hipError_t launch_observe_noalloc(int prec, Member m, hipStream_t s);
 int noalloc_max_x();
@@ -402,6 +402,7 @@ struct wh_ensemble {
   DevBuf mem_dev;
   std::map<int, std::unique_ptr<TwSet>> tw;  // by size
   int xvar = 0, pvar = 0, pclvar = 0;
+  bool gp_narrow = false;  // form of the Gross-Pitaevskii shift
   bool expr = false;  // a member's V is an expression program: tables before each p sweep
   // p work lists: one for the plain p variant and one for the Caldeira-Leggett p variant
   // (a tile spans block * R / P columns, which differs between the two variant tables;
@@ -578,7 +579,7 @@ int build_work_lists(wh_ensemble* e) {
     const size_t cells = size_t(m.X) * size_t(m.P);
     for (size_t t = 0; t < (cells + wh::kScaleChunk - 1) / wh::kScaleChunk; ++t) ws.push_back(hi | unsigned(t));
     if (e->gp()) {
-      const int grows = wh::tile_lines(m.X, wh::SweepVariant{16, 256, 0});
+      const int grows = wh::tile_lines(m.X, e->gp_narrow ? wh::kGpNarrow : wh::kGpWide);
       for (int t = 0; t < m.P / grows; ++t) wg.push_back(hi | unsigned(t));
     }
     if (e->odm()) {
@@ -756,7 +757,11 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
   narrow_variants(e.get());
   for (int i = 0; i < n; ++i) e->expr = e->expr || e->mem[i].pot_expr_len > 0;
   if (gp) {
-    const wh::SweepVariant g{16, 256, 0};
+    size_t cells = 0;
+    for (int i = 0; i < n; ++i) cells += size_t(e->mem[i].X) * size_t(e->mem[i].P);
+    e->gp_narrow = cells / (size_t(wh::kGpWide.R) * size_t(wh::kGpWide.block)) < size_t(wh::kCUs);
+    for (int i = 0; i < n; ++i) e->gp_narrow = e->gp_narrow && e->mem[i].X <= 512;  // teams of one wave
+    const wh::SweepVariant g = e->gp_narrow ? wh::kGpNarrow : wh::kGpWide;
     for (int i = 0; i < n; ++i) {
       const auto& m = e->mem[i];
       if (!wh::variant_fits(m.X, g) || m.P % wh::tile_lines(m.X, g) != 0)
@@ -896,7 +901,7 @@ int gpshift(wh_ensemble* e, int flags, hipStream_t s) {
   wh::SweepArgs a = sweep_args(e, flags, 1.0, 0);
   a.work = e->work_gp.buf.as<unsigned>();
   a.ntiles = e->n == 1 ? e->work_gp.n - 1 : 0;  // the record item is the last
-  WH_LAUNCH(wh::launch_gpshift(a, e->work_gp.n, s), "gpshift");
+  WH_LAUNCH(wh::launch_gpshift(e->gp_narrow, a, e->work_gp.n, s), "gpshift");
   return WH_SUCCESS;
 }
 // density after the kinetic step from the x sweep's partial sums

@@ -28,6 +28,10 @@ constexpr int kAllP = sizeof(kPVariants) / sizeof(kPVariants[0]), kNumP = kAllP 
 constexpr int kAllPCL = sizeof(kPCLVariants) / sizeof(kPCLVariants[0]), kNumPCL = kAllPCL - 2;
 constexpr int kCUs = 256;
 
+// The Gross-Pitaevskii shift: rows of G in teams of one wave at most (radix 8, sides up to 512) where
+// kGpWide's blocks would be fewer than the CUs.
+constexpr SweepVariant kGpWide{16, 256, 0}, kGpNarrow{8, 64, 0};
+
 // largest grid side of the plain (x and p) throughput forms
 constexpr int kTpMaxN = 1024;
 
