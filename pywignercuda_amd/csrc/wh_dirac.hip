@@ -7,11 +7,11 @@
 //                  P_minus_Lambda, Fourier_4X4_Lambda_To_X_GPU; :159-351, 2622-2676, 3514-3558).
 //                 The kinetic factor only couples spinor rows {1,4}, {2,3} and columns {1,4},
 //                 {2,3}, so the 16 planes fall into 4 closed groups of 4 (e.g. W11 W14 W41 W44)
-//                 and a team keeps one group in registers.  The lambda = 0 bin of groups
+//                 and a team keeps one group in registers; a block shares a row's factors.  The lambda = 0 bin of groups
 //                 {11,14,41,44} and {22,23,32,33} gives the antiparticle population of the
 //                 loaded state (AntiParticlePopulation, :2436-2466: the filtered trace summed
 //                 over x is Tr[Lambda_-(p) sum_x W(x, p)]).
-//   dirac_psweep  one team per column x, all 16 planes in turn:  FFT_p -> e^{-dt D theta^2}
+//   dirac_psweep  one team per column x, four planes in turn:  FFT_p -> e^{-dt D theta^2}
 //                 e^{-i dt (V0(x - theta/2) - V0(x + theta/2))} times the constant mass phase of
 //                 the plane -> iFFT_p / P -> [Caldeira-Leggett order 2] -> edge absorber ->
 //                 column sums for the observables and the trace norm
@@ -21,9 +21,10 @@
 //                 With A = 0 the potential factors are diagonal: P-(y) = e^{-iF} on spinor rows
 //                 1, 2 and e^{+iF} on rows 3, 4 (F = mass_half c^2 dt), so plane W_ij picks up
 //                 e^{-2iF} (i in {1,2}, j in {3,4}), e^{+2iF} (i in {3,4}, j in {1,2}) or 1.
-//   dirac_reduce  one block: observables of the normalised state, trace norm -> pending
-//                 factor 1/norm applied by the next x sweep's load (Wigner_4X4_Normalize,
-//                 :2740-2775 and the reductions of :3429-3492).
+//   record        observables of the normalised state, trace norm -> pending factor 1/norm that rides
+//                 on the next x sweep's left factor (Wigner_4X4_Normalize, :2740-2775 and the
+//                 reductions of :3429-3492): an item of that sweep, from tile sums of the p sweep
+//                 (dirac_record_item), or a launch over the column sums (dirac_reduce_kernel).
 #include <hip/hip_runtime.h>
 
 #include "wh_dirac.hpp"
