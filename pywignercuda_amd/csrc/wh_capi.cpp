@@ -21,6 +21,7 @@
 
 #include "../../include/wignerhip.h"
 #include "wh_bloch.hpp"
+#include "wh_devbuf.hpp"
 #include "wh_dirac.hpp"
 #include "wh_kernels.hpp"
 #include "wh_variants.hpp"
@@ -123,24 +124,10 @@ bool sweep_size_supported(int n) { return n >= 128 && n <= 2048 && size_supporte
 size_t state_bytes(int prec) { return prec == WH_C128 ? 16 : 8; }
 int storage_code(int prec) { return prec == WH_C128 ? WH_C128 : WH_C64; }
 
-// device allocation owned by a plan
-struct DevBuf {
-  void* p = nullptr;
-  size_t bytes = 0;
-  DevBuf() = default;
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
+// device allocation owned by a plan, with the library's status codes
+struct DevBuf : wh::DeviceBuffer {
   int alloc(size_t n) {
-    if (p) (void)hipFree(p);
-    bytes = n;
-    hipError_t e = hipMalloc(&p, n ? n : 16);
-    if (e != hipSuccess) {
-      p = nullptr;
-      return hip_fail(e, "hipMalloc");
-    }
+    WH_HIP(replace(n), "hipMalloc");
     return WH_SUCCESS;
   }
   int upload(const void* host, size_t n) {
