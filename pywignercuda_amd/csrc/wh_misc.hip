@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include "wh_fft.hpp"
+#include "wh_index.hpp"
 #include "wh_kernels.hpp"
 
 namespace wh {
@@ -290,13 +291,12 @@ __global__ void __launch_bounds__((FftShape<T, N>::C * FftShape<T, N>::TT))
   // neighbouring tiles, which share 128-byte lines, on one XCD
   const int nt = int(gridDim.x), b = int(blockIdx.x);
   const int tile = nt % 8 == 0 ? (b % 8) * (nt / 8) + b / 8 : b;
-  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data));
-  const unsigned boff = (unsigned(tl) * unsigned(X) + unsigned(tile * C + cl)) * unsigned(sizeof(cplx<T>));
+  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data)) + col_element(tl, X, tile * C + cl);
   TwRegs<T, N, R> twr;
   load_twiddles<T, N, R>(twr, tc, tw);
   cplx<T> v[R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = gload(at_off(W + size_t(j * TT) * X, boff));
+  for (int j = 0; j < R; ++j) v[j] = gload(W + col_element(j * TT, X, 0));
   if constexpr (G::kWave) {
     const LdsRow<T> view_l{lds + cl * LSZ}, view_c{lds + cc * LSZ};
     team_fft_remap<T, N, R, DIR>(v, tl, view_l, tc, view_c, twr);
@@ -311,7 +311,7 @@ __global__ void __launch_bounds__((FftShape<T, N>::C * FftShape<T, N>::TT))
   }
   const T f = normalize ? T(1.0 / N) : T(1);
 #pragma unroll
-  for (int j = 0; j < R; ++j) store_cached(at_off(W + size_t(j * TT) * X, boff), cscale(v[j], f));
+  for (int j = 0; j < R; ++j) store_cached(W + col_element(j * TT, X, 0), cscale(v[j], f));
 }
 
 // ------------------------------------------------------------------ launchers
