@@ -480,12 +480,20 @@ class Wigner2D(_PlanBase):
         """Backward pass over len(states) steps from W_first (the state before step first_step):
         states [n, P, X] is scratch for the states after each step, Lam is carried back in place,
         grads ([n, 9] float64, device) receives dL/da of each step."""
+        import torch
+
         n = int(states.shape[0])
+        if n < 1:
+            raise ValueError("states holds no step")
         self._check_state(W_first)
         self._check_state(Lam)
         self._check_state(states[0])
-        if not states.is_contiguous() or not grads.is_contiguous() or tuple(grads.shape) != (n, WH_MAX_DEG + 1):
-            raise ValueError(f"states must be contiguous and grads a contiguous [{n}, {WH_MAX_DEG + 1}] tensor")
+        if not states.is_contiguous():
+            raise ValueError(f"states must be a contiguous [{n}, {self.P}, {self.X}] tensor")
+        # the kernels write doubles: any other type or device would be written past its end
+        if (grads.dtype != torch.float64 or not grads.is_cuda or grads.device != states.device
+                or not grads.is_contiguous() or tuple(grads.shape) != (n, WH_MAX_DEG + 1)):
+            raise ValueError(f"grads must be a contiguous float64 [{n}, {WH_MAX_DEG + 1}] tensor on {states.device}")
         _lib.check(_lib.lib().wh_wigner2d_adjoint_segment(self._plan, _lib.dptr(W_first), _lib.dptr(states),
                                                           _lib.dptr(Lam), int(first_step), n, _lib.dptr(grads),
                                                           _lib.current_stream_handle()),
