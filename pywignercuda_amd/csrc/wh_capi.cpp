@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <string>
@@ -1336,6 +1337,13 @@ int check_plain(const wh_ensemble* e, const char* who) {
     return fail(WH_INVALID_VALUE, "%s covers the Lie scheme without damping or Gross-Pitaevskii", who);
   return WH_SUCCESS;
 }
+// the sweeps load and store whole complex elements
+int check_aligned(const wh_ensemble* e, const char* who, std::initializer_list<const void*> states) {
+  const size_t align = state_bytes(e->d.precision);
+  for (const void* w : states)
+    if (reinterpret_cast<uintptr_t>(w) % align) return fail(WH_UNALIGNED_DATA, "%s: state %p", who, w);
+  return WH_SUCCESS;
+}
 int check_adjoint(wh_ensemble* e) {
   WH_TRY(check_plain(e, "the adjoint step"));
   if (e->mem[0].pot_deg < 0)
@@ -1385,6 +1393,7 @@ extern "C" int wh_wigner2d_steps(wh_wigner2d* p, const void* W_in, void* W_out, 
                 n_steps);
   wh_ensemble* e = p->e;
   WH_TRY(check_plain(e, "wh_wigner2d_steps"));
+  WH_TRY(check_aligned(e, "wh_wigner2d_steps", {W_in, W_out}));
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (e->table_dirty) WH_TRY(sync_table(e, true, s));
   for (int k = 0; k < n_steps; ++k) WH_TRY(plain_step(e, k == 0 ? W_in : W_out, W_out, first_step + k, s));
@@ -1414,6 +1423,9 @@ extern "C" int wh_wigner2d_adjoint_segment(wh_wigner2d* p, const void* W_first, 
                 "n_steps %d", W_first, states, Lambda, (void*)grads, first_step, n_steps);
   wh_ensemble* e = p->e;
   WH_TRY(check_adjoint(e));
+  WH_TRY(check_aligned(e, "wh_wigner2d_adjoint_segment", {W_first, states, Lambda}));
+  if (reinterpret_cast<uintptr_t>(grads) % sizeof(double))
+    return fail(WH_UNALIGNED_DATA, "wh_wigner2d_adjoint_segment: grads %p", (void*)grads);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (e->table_dirty) WH_TRY(sync_table(e, true, s));
   WH_TRY(adjoint_room(e, n_steps, s));
