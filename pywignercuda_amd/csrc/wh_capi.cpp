@@ -390,6 +390,7 @@ struct wh_ensemble {
   DevBuf mem_dev;
   std::map<int, std::unique_ptr<TwSet>> tw;  // by size
   int xvar = 0, pvar = 0, pclvar = 0;
+  int gp_xvar = 0;  // x variant of a Gross-Pitaevskii plan's partial density sums
   bool gp_narrow = false;  // form of the Gross-Pitaevskii shift
   bool expr = false;  // a member's V is an expression program: tables before each p sweep
   // p work lists: one for the plain p variant and one for the Caldeira-Leggett p variant
@@ -513,7 +514,7 @@ int narrowed(const wh_ensemble* e, const wh::SweepVariant* t, int n, int all, in
     if (t[i].R == t[v].R && t[i].block < t[v].block && fits_all(e, t[i], x_axis, cl)) v = i;
   return v;
 }
-// (the x variant of a Gross-Pitaevskii plan also cuts its partial density sums: it stays)
+// (the x variant of a Gross-Pitaevskii plan also cuts its partial density sums: no narrow form)
 void narrow_variants(wh_ensemble* e) {
   if (!e->gp()) e->xvar = narrowed(e, wh::kXVariants, wh::kNumX, wh::kAllX, e->xvar, true);
   e->pvar = narrowed(e, wh::kPVariants, wh::kNumP, wh::kAllP, e->pvar, false);
@@ -732,13 +733,14 @@ int ensemble_create(const wh_ensemble_desc* desc, const wh_member_desc* members,
   };
   WH_TRY(pick(wh::kXVariants, wh::kNumX, true, e->xvar));
   if (gp) {
-    // fixed for the plan's life (the partial sums are cut by its rows per tile): the radix that is
-    // fastest for a single grid of the widest member's side, measured per x sweep: 4 up to 256,
-    // 8 at 512 (7.4 us at 512^2; radix 16: 9.4) and 2048, 16 at 1024
+    // (the partial sums are cut by its rows per tile) the radix that is fastest for a single grid of
+    // the widest member's side, measured per x sweep: 4 up to 256, 8 at 512 (7.4 us at 512^2; radix
+    // 16: 9.4) and 2048, 16 at 1024
     int side = 0;
     for (const auto& m : e->mem) side = std::max(side, m.X);
     const int v = side <= 256 ? 3 : side == 1024 ? 0 : 1;
     if (fits_all(e.get(), wh::kXVariants[v], true)) e->xvar = v;
+    e->gp_xvar = e->xvar;
   }
   WH_TRY(pick(wh::kPVariants, wh::kNumP, false, e->pvar));
   WH_TRY(pick(wh::kPCLVariants, wh::kNumPCL, false, e->pclvar, true));
@@ -1180,8 +1182,10 @@ extern "C" int wh_ensemble_set_variants(wh_ensemble* e, int xvar, int pvar, int 
     return fail(WH_INVALID_VALUE, "p variant %d does not fit every member", pvar);
   if (pclvar >= 0 && !fits_all(e, wh::kPCLVariants[pclvar], false, true))
     return fail(WH_INVALID_VALUE, "p+CL variant %d does not fit every member", pclvar);
-  if (e->gp() && xvar >= 0 && xvar != e->xvar)
-    return fail(WH_INVALID_VALUE, "the x variant of a Gross-Pitaevskii plan is fixed at creation");
+  // The partial density sums are cut by the rows per tile of the plan's own choice; the default has
+  // at least as many rows at every side, so that its tiles fit the same buffer.
+  if (e->gp() && xvar > 0 && xvar != e->gp_xvar)
+    return fail(WH_INVALID_VALUE, "the x variant of a Gross-Pitaevskii plan is the default or the one of its creation");
   if (xvar >= 0) e->xvar = xvar;
   if (pvar >= 0) e->pvar = pvar;
   if (pclvar >= 0) e->pclvar = pclvar;

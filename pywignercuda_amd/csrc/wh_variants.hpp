@@ -43,4 +43,14 @@ constexpr bool variant_fits(int N, SweepVariant v, bool cl = false) {
 // rows per x-sweep tile / columns per p-sweep tile
 constexpr int tile_lines(int N, SweepVariant v) { return v.block / (N / v.R); }
 
+// the x variants of a Gross-Pitaevskii plan: the default (index 0) has at least as many rows per tile as
+// the two others it may be created with, at every side (its partial density sums fit their buffer)
+constexpr bool default_fits_partials() {
+  for (int N = 128; N <= 2048; N *= 2)
+    for (int v : {1, 3})
+      if (!variant_fits(N, kXVariants[0]) || tile_lines(N, kXVariants[0]) < tile_lines(N, kXVariants[v])) return false;
+  return true;
+}
+static_assert(default_fits_partials(), "partial density sums");
+
 }  // namespace wh
