@@ -593,17 +593,38 @@ struct PSweep {
     for (int j = 0; j < R; ++j) v[j] = apply(v[j], M[j]);
   }
 
-  // D(Y) = F_p^{-1}[ theta * F_p[ sigma(p) Y ] ]   (Theta_fp_Damping, FFT.py:1135-1143);
-  // sg, th: sigma and theta / N of this lane's elements (the 1/N of the inverse transform is a
-  // power of two: exact), read once per sweep
-  template <class Tw>
-  __device__ __forceinline__ static void cl_operator(cplx<T> (&y)[R], const T (&sg)[R], const T (&th)[R], int t,
-                                                     View view, const Tw& tw) {
+  // The friction operator's factors of this lane's elements: sigma, and theta / N (the 1/N of the
+  // inverse transform is a power of two: exact).  REGS: read once per sweep.
+  template <bool REGS>
+  struct Friction {
+    T sg[REGS ? R : 1], th[REGS ? R : 1];
+    gptr<const double> sigma, theta;
+    __device__ __forceinline__ void load(CMember& m, int t) {
+      sigma = gmem(m.sigma_p);
+      theta = gmem(m.theta_host);
+      if constexpr (REGS) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], sg[j]);
+        for (int j = 0; j < R; ++j) {
+          sg[j] = T(sigma[t + j * TT]);
+          th[j] = T(theta[t + j * TT] * (1.0 / N));
+        }
+      }
+    }
+    __device__ __forceinline__ void by_sigma(cplx<T> (&y)[R], int t) const {
+#pragma unroll
+      for (int j = 0; j < R; ++j) y[j] = cscale(y[j], REGS ? sg[REGS ? j : 0] : T(sigma[t + j * TT]));
+    }
+    __device__ __forceinline__ void by_theta(cplx<T> (&y)[R], int t) const {
+#pragma unroll
+      for (int j = 0; j < R; ++j) y[j] = cscale(y[j], REGS ? th[REGS ? j : 0] : T(theta[t + j * TT] * (1.0 / N)));
+    }
+  };
+  // D(Y) = F_p^{-1}[ theta * F_p[ sigma(p) Y ] ]   (Theta_fp_Damping, FFT.py:1135-1143)
+  template <class F, class Tw>
+  __device__ __forceinline__ static void cl_operator(cplx<T> (&y)[R], const F& f, int t, View view, const Tw& tw) {
+    f.by_sigma(y, t);
     team_fft<T, N, R, -1, View, Sync>(y, t, view, tw);
-#pragma unroll
-    for (int j = 0; j < R; ++j) y[j] = cscale(y[j], th[j]);
+    f.by_theta(y, t);
     team_fft<T, N, R, +1, View, Sync>(y, t, view, tw);
   }
 };
@@ -648,16 +669,18 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   const bool early = kEarly && PS::early(a, m);
   typename PS::MulLoads ml;
   if (early) PS::mul_loads(ml, a, m, tc, col, step);
-  // the friction tables and the host values of one column per lane: in registers when the state is
-  T sg[CL ? R : 1], th[CL ? R : 1];
-  double decay[CL ? R : 1];  // (a plan with friction always has the table)
-  if constexpr (CL) {
+  // The friction tables: in registers with the state, or read again for every operator.  Where a CU
+  // has one block the wave is alone on its SIMD and the registers are there (FP64, 1024^2: 45.8 us a
+  // step, read again 48.4).  Radix-16 lanes in FP32 arithmetic, and the throughput form, run two waves
+  // per SIMD only without them (FP32, P = 2048: 214 VGPRs, with them 326; 2048^2 steps: FP32 arithmetic
+  // 202 -> 153 us, complex64 states 198 -> 159, complex128 213 -> 174).
+  constexpr bool kTabRegs = CL && (R <= 8 || (sizeof(T) == 8 && !TP));
+  typename PS::template Friction<kTabRegs> friction;
+  double decay[kTabRegs ? R : 1];  // (a plan with friction always has the table)
+  if constexpr (CL) friction.load(m, tc);
+  if constexpr (kTabRegs && kEarly) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      if constexpr (kEarly) decay[j] = gmem(m.theta_decay)[tc + j * TT];
-      sg[j] = T(gmem(m.sigma_p)[tc + j * TT]);
-      th[j] = T(gmem(m.theta_host)[tc + j * TT] * (1.0 / N));
-    }
+    for (int j = 0; j < R; ++j) decay[j] = gmem(m.theta_decay)[tc + j * TT];
   }
   TilePartials part{0.0, 0.0};
   const bool behind_join = !CL && (a.flags & kTileScale);  // an ODM join's partials give the pending factor
@@ -688,7 +711,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
     team_fft<T, N, R, -1, View, Sync>(v, tc, view_c, twsrc);
   }
   const auto theta_decay = [&]() {
-    if constexpr (CL) {
+    if constexpr (kTabRegs) {
 #pragma unroll
       for (int j = 0; j < R; ++j) v[j] = apply(v[j], cplx<double>{decay[j], 0.0});
     } else if (m.theta_decay) {
@@ -702,7 +725,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = apply(v[j], f);
   }
-  if constexpr (CL && !kEarly) {  // in flight while potential() evaluates its multipliers
+  if constexpr (kTabRegs && !kEarly) {  // in flight while potential() evaluates its multipliers
     const int t = opaque_v(tc);
 #pragma unroll
     for (int j = 0; j < R; ++j) decay[j] = gmem(m.theta_decay)[t + j * TT];
@@ -723,13 +746,13 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
     for (int j = 0; j < R; ++j) d[j] = v[j];
     const T c1 = T(2.0 * a.cl_a), c2 = T((-10.0 / 3.0) * a.cl_a * a.cl_a),
             c3 = T((-4.0 / 3.0) * a.cl_a * a.cl_a * a.cl_a);
-    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
+    PS::cl_operator(d, friction, tc, view_c, twsrc);
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = cadd(v[j], mul_i(d[j], c1));
-    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
+    PS::cl_operator(d, friction, tc, view_c, twsrc);
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = cadd(v[j], cscale(d[j], c2));
-    PS::cl_operator(d, sg, th, tc, view_c, twsrc);
+    PS::cl_operator(d, friction, tc, view_c, twsrc);
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = cadd(v[j], mul_i(d[j], c3));
   }
@@ -934,8 +957,10 @@ __device__ __forceinline__ void gpshift_body(const SweepArgs& a, CMember& m, int
 
 // Two waves per SIMD (<= 256 VGPRs) for the plain sweeps: a batch of grids overlaps one
 // wave's loads and stores with the other's transforms; three for the throughput form
-// (TP: table twiddles, exchanges in the storage precision).  The Caldeira-Leggett p sweep
-// holds three state copies and keeps the full register file of one wave.
+// (TP: table twiddles, exchanges in the storage precision).  The Caldeira-Leggett p sweep holds
+// two state copies: its plain forms may take the full register file of one wave, its throughput
+// form fits two, and exchanges in the arithmetic precision there (rounding the exchanges to
+// complex64 gains nothing: 2048^2 161 us a step in FP64, 162 rounded).
 template <typename S, typename T, bool TP>
 using LdsElem = std::conditional_t<TP, S, T>;
 template <typename S, typename T, int R, int BLOCK, bool TP>
@@ -960,7 +985,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TP ?
 
 template <typename S, typename T, int R, int BLOCK, bool CL, bool TP>
 __device__ __forceinline__ void psweep_entry(const SweepArgs& a) {
-  using E = LdsElem<S, T, TP>;
+  using E = LdsElem<S, T, TP && !CL>;
   __shared__ cplx<E> lds[lds_elems<BLOCK, R>() + kPTailBytes / sizeof(cplx<E>)];
   const unsigned w = p_item(a);
   CMember& m = member_at(a.members, w >> 16);

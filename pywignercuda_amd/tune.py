@@ -108,19 +108,25 @@ def tune_single(prec, N, reps, cl=False, xvar=None):
     return out
 
 
-def tune_batch(prec, N, reps):
+def tune_batch(prec, N, reps, cl=False):
+    """Variant of each sweep for an ensemble; cl: of the Caldeira-Leggett p sweep, with the other
+    sweeps as the table has them."""
     import torch
 
     bytes_per = N * N * (16 if prec == "fp64" else 8)
     n = max(2, min(512, (1 << 30) // bytes_per))
     m = dict(X=N, P=N, X_amp=10.0, P_amp=10.0, potential="0.5*pow(x,2) + 0.1*pow(x,4)",
              dpotential="x + 0.4*pow(x,3)")
-    ens = WignerEnsemble([m] * n, 1.0, 1.0, 0.01, precision=prec, variants=(0, 0, 0))
+    kw = {}
+    if cl:
+        m.update(fp_damping="fabs(p)", D_theta=0.1)
+        kw.update(gamma=0.1, damping="CaldeiraLeggett")
+    ens = WignerEnsemble([m] * n, 1.0, 1.0, 0.01, precision=prec, variants=None if cl else (0, 0, 0), **kw)
     states = [torch.zeros((N, N), dtype=ens.dtype, device=ens.device) for _ in range(n)]
     for s in states:
         s[0, 0] = 1.0
     out = {}
-    for table, name in ((0, "x"), (1, "p")):
+    for table, name in ((2, "pcl"),) if cl else ((0, "x"), (1, "p")):
         best = None
         for v in _variants(table):
             args = [-1, -1, -1]
@@ -159,7 +165,7 @@ def main():
                     single.setdefault(k + "_us", {})[str(N)] = round(v[1], 2)
             print(f"{prec} {N}: single {r} cl {rc}", flush=True)
             if not a.no_batch:
-                rb = tune_batch(prec, N, a.reps)
+                rb = {**tune_batch(prec, N, a.reps), **tune_batch(prec, N, a.reps, cl=True)}
                 for k, v in rb.items():
                     if v is not None:
                         batch.setdefault(k, {})[str(N)] = v[0]

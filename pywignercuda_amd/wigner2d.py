@@ -77,6 +77,12 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
     pcl = t.get("pcl", {}).get(npp, -1)
     cells = sum(int(x) * int(p) for x, p in zip(sizes_x, sizes_p))
     if t and not batch:
+        # friction at P >= 1024: two waves per SIMD (tables read per operator) where every CU gets two
+        # blocks, below that one wave with the tables in registers (us per step, one -> two waves:
+        # 2048 x 128 46 -> 54, 1024^2 46 -> 48, 2048 x 512 61 -> 68, 1024 x 2048 82 -> 72, 2048 x 1024
+        # 107 -> 89, 2048^2 213 -> 175).  FP32 arithmetic fits two waves in either form.
+        if precision != "fp32fast" and npp in ("1024", "2048") and pcl >= 0:
+            pcl = 2 if cells >= 1 << 21 else 0
         if cells <= 1 << 19:
             pv, pcl = 2, 1  # radix 8
             xv = {"1024": 3, "2048": 1}.get(nx, xv)  # radix 4, radix 8
