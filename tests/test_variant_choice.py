@@ -28,3 +28,13 @@ def test_friction_form_by_cells(precision):
         assert choice(precision, X, P, True, members)[2] == 2, (P, X, members)
     for P, X in ((1024, 1024), (2048, 512)):
         assert choice(precision, X, P, True)[2] == 0, (P, X)
+
+
+@pytest.mark.parametrize("cl", [False, True])
+@pytest.mark.parametrize("P", [1024, 2048])
+def test_complex128_keeps_radix_16_in_long_columns(P, cl):
+    """Radix 8 leaves a larger residue in <p^2> there (see tuned_variants)."""
+    for X in (128, 256, 512, 1024, 2048):
+        for members in (1, 2, 16, 64):
+            _, pv, pcl = choice("fp64", X, P, cl, members)
+            assert radix(1, max(pv, 0)) == 16 and radix(2, max(pcl, 0)) == 16, (X, members)
