@@ -68,9 +68,13 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
     2048 x 128 22.9 -> 19.8, with friction 46.2 -> 36.2) but further from the exact steps: its twiddle
     roundings leave a fixed residue at the edges of p, which <p^2> weighs most (72 steps against 80-bit
     ones, largest relative error, radix 16 -> 8: 1024 1.7e-13 -> 8.7e-13, 2048 3.8e-13 -> 9.0e-13).
-    A complex128 state of 2^20 or 2^21 cells, which the L2s hold, wants radix 16 in x at every width
-    (512 x 2048 39.7 -> 36.7, 2048 x 1024 51.6 -> 46.7; beyond them 2048^2 93.9 with radix 8, 104.6
-    with 16)."""
+    Complex128 states of 2^20 or 2^21 cells together, which the L2s hold, want radix 16 in x where a
+    side is 512 or more (512 x 2048 39.7 -> 36.7, 2048 x 1024 51.6 -> 46.7, four grids of 512^2
+    34.0 -> 28.4, eight 41.1 -> 41.4; beyond them 2048^2 93.9 with radix 8, 104.6 with 16).  Ensembles
+    of smaller sides would gain as well (64 x 128^2 32.1 -> 28.7, 16 x 256^2 32.7 -> 27.5; 128 x 128^2
+    and 32 x 256^2 equal) but keep the tuner's radix 4, which is more exact (state after 72 steps
+    against 80-bit ones, radix 4 -> 16: 128 1.6e-14 -> 2.0e-14, 256 1.6e-14 -> 1.8e-14; at 512 radix 8
+    gives 2.2e-14 and 16 1.9e-14)."""
     tab = _load_tuning()
     t = tab.get(precision + "_batch", {}) if batch else {}
     if not t:
@@ -91,7 +95,7 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
             if precision != "fp64":
                 pv, pcl = 2, 1  # radix 8
             xv = {"1024": 3, "2048": 1}.get(nx, xv)  # radix 4, radix 8
-        elif precision == "fp64" and cells <= 1 << 21:
+        elif precision == "fp64" and cells <= 1 << 21 and int(nx) >= 512:
             xv = 0  # radix 16
     return int(xv), int(pv), int(pcl)
 

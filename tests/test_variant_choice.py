@@ -38,3 +38,11 @@ def test_complex128_keeps_radix_16_in_long_columns(P, cl):
         for members in (1, 2, 16, 64):
             _, pv, pcl = choice("fp64", X, P, cl, members)
             assert radix(1, max(pv, 0)) == 16 and radix(2, max(pcl, 0)) == 16, (X, members)
+
+
+def test_small_sides_keep_their_radix_in_ensembles():
+    """Radix 16 in x for 2^20 and 2^21 cells of complex128 is for sides of 512 and more."""
+    for side, members in ((128, 64), (128, 128), (256, 16), (256, 32)):
+        assert radix(0, choice("fp64", side, side, members=members)[0]) == 4, (side, members)
+    for X, P, members in ((512, 2048, 1), (2048, 512, 1), (2048, 1024, 1), (512, 512, 4), (512, 512, 8), (1024, 1024, 2)):
+        assert radix(0, choice("fp64", X, P, members=members)[0]) == 16, (X, P, members)
