@@ -12,6 +12,7 @@
 #include "wh_fft.hpp"
 #include "wh_index.hpp"
 #include "wh_kernels.hpp"
+#include "wh_variants.hpp"
 
 namespace wh {
 
@@ -235,25 +236,42 @@ __global__ void set_scale_kernel(const Member* members, double re, double im) {
 }
 
 // ------------------------------------------------------------------ plain axis transforms
-// Teams of one wave (radix 8 up to N = 512, radix 16 at 1024) exchange without block barriers and hold
-// their twiddles in registers, loaded with the state.  A row block is one wave (or the team), so that
-// a few hundred rows reach every CU: blocks of 256 lanes left half of them idle at 512 x 1024.
-// A forward and an inverse pair over both axes with two clones, us, before -> after (radix 16 for every
-// length, block barriers, 256 lanes a block): 2048^2 complex128 239 -> 147, complex64 205 -> 119; 1024^2
+// Narrow form: teams of one wave (radix 8 up to N = 512, radix 16 at 1024) exchange without block barriers
+// and hold their twiddles in registers, loaded with the state.  A row block is one wave (or the team), so
+// that a few hundred rows reach every CU: blocks of 256 lanes left half of them idle at 512 x 1024.
+// A forward and an inverse pair over both axes with two clones, us, against radix 16, block barriers and
+// 256 lanes a block for every length: 2048^2 complex128 239 -> 147, complex64 205 -> 119; 1024^2
 // 65 -> 60 and 64 -> 44; 512 x 1024 47 -> 38; below, the calls' host time (38 us) covers the kernels.
-template <typename T, int N>
+// Wide form (large batches, the rules are in fft_rows_n and fft_cols_n): radix 16 in blocks of 256 lanes.
+// Its rows of columns are whole 128-byte lines (64 bytes at complex64 512) and it exchanges once less; a
+// narrow block's rows of 4 columns are 32 or 64 bytes, too short once the batch is beyond the L2s.
+template <typename T, int N, bool WIDE>
 struct FftShape {
-  static constexpr int R = N <= 512 ? 8 : 16, TT = N / R;
-  static constexpr bool kWave = TT <= 64;
-  static constexpr int ROWS = TT >= 64 ? 1 : 64 / TT;             // rows per block
-  static constexpr int C = N <= 64 ? 8 : N <= 1024 ? 4 : 2;      // columns per block
-  using Sync = std::conditional_t<kWave, WaveSync, BlockSync>;
+  static constexpr int R = WIDE || N > 512 ? 16 : 8, TT = N / R;
+  static constexpr int kLines = 256 / TT < 1 ? 1 : 256 / TT;                                // of a wide block
+  static constexpr int ROWS = WIDE ? kLines : TT >= 64 ? 1 : 64 / TT;                       // rows per block
+  static constexpr int C = WIDE ? (kLines > 64 ? 64 : kLines) : N <= 64 ? 8 : N <= 1024 ? 4 : 2;  // columns per block
+  // teams of one wave; wide rows only in FP32, where they are faster (512 x 32768: 43 us, with block
+  // barriers 47; FP64 the other way round beyond the caches: 512 x 262144 727 and 805)
+  static constexpr bool kWaveRows = TT <= 64 && (!WIDE || sizeof(T) == 4), kWaveCols = TT <= 64 && !WIDE;
 };
 
-template <typename T, int N, int DIR>
-__global__ void __launch_bounds__((FftShape<T, N>::ROWS * FftShape<T, N>::TT))
+template <bool REGS, typename T, int N, int R>
+__device__ __forceinline__ auto fft_twiddles(int t, const Twiddles<T>& tw) {
+  if constexpr (REGS) {
+    TwRegs<T, N, R> r;
+    load_twiddles<T, N, R>(r, t, tw);
+    return r;
+  } else {
+    return TwMem<T>{tw};
+  }
+}
+
+template <typename T, int N, bool WIDE, int DIR>
+__global__ void __launch_bounds__((FftShape<T, N, WIDE>::ROWS * FftShape<T, N, WIDE>::TT))
     fft_rows_kernel(void* data, int rows, int normalize, Twiddles<T> tw) {
-  using G = FftShape<T, N>;
+  using G = FftShape<T, N, WIDE>;
+  using Sync = std::conditional_t<G::kWaveRows, WaveSync, BlockSync>;
   constexpr int R = G::R, TT = G::TT, ROWS = G::ROWS;
   constexpr int LSZ = Padded<N, R>::size;
   __shared__ cplx<T> lds[ROWS * LSZ];
@@ -263,12 +281,21 @@ __global__ void __launch_bounds__((FftShape<T, N>::ROWS * FftShape<T, N>::TT))
   const bool active = row < rows;
   const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data)) + size_t(active ? row : 0) * N;
   LdsRow<T> view{lds + team * LSZ};
-  TwRegs<T, N, R> twr;
-  load_twiddles<T, N, R>(twr, t, tw);
+  const auto twsrc = fft_twiddles<!WIDE, T, N, R>(t, tw);
   cplx<T> v[R];
+  if constexpr (G::kWaveRows || !WIDE) {
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = gload(W + t + j * TT);
-  team_fft<T, N, R, DIR, LdsRow<T>, typename G::Sync>(v, t, view, twr);
+    for (int j = 0; j < R; ++j) v[j] = gload(W + t + j * TT);
+  } else {
+    // in a branch, in front of which the compiler moves no twiddle load (2048 x 65536 complex128:
+    // 728 us, without the branch 764)
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      v[j] = {T(0), T(0)};
+      if (active) v[j] = gload(W + t + j * TT);
+    }
+  }
+  team_fft<T, N, R, DIR, LdsRow<T>, Sync>(v, t, view, twsrc);
   const T f = normalize ? T(1.0 / N) : T(1);
   if (active) {
 #pragma unroll
@@ -277,29 +304,38 @@ __global__ void __launch_bounds__((FftShape<T, N>::ROWS * FftShape<T, N>::TT))
 }
 
 // Loads and stores cover rows of C consecutive columns; a wave's team takes its column over at the
-// first exchange and hands it back before the store.
-template <typename T, int N, int DIR>
-__global__ void __launch_bounds__((FftShape<T, N>::C * FftShape<T, N>::TT))
+// first exchange and hands it back before the store.  FAR: offsets in 64 bits (offsets_fit_32).
+template <typename T, int N, bool WIDE, bool FAR, int DIR>
+__global__ void __launch_bounds__((FftShape<T, N, WIDE>::C * FftShape<T, N, WIDE>::TT))
     fft_cols_kernel(void* data, int X, int normalize, Twiddles<T> tw) {
-  using G = FftShape<T, N>;
+  using G = FftShape<T, N, WIDE>;
   constexpr int R = G::R, TT = G::TT, C = G::C;
-  constexpr int LSZ = N + N / R + col_pad<T, C>();
+  constexpr int LSZ = G::kWaveCols ? N + N / R + col_pad<T, C>() : Padded<N, R>::size;
   __shared__ cplx<T> lds[C * LSZ];
   const int tid = threadIdx.x;
   const int cl = tid % C, tl = tid / C;
-  const int cc = G::kWave ? tid / TT : cl, tc = G::kWave ? tid % TT : tl;
-  // neighbouring tiles, which share 128-byte lines, on one XCD
+  const int cc = G::kWaveCols ? tid / TT : cl, tc = G::kWaveCols ? tid % TT : tl;
+  // neighbouring tiles that share 128-byte lines on one XCD (whole lines go in order: complex128
+  // 256 x 131072 204 us, by XCD 217)
+  constexpr bool kShared = C * int(sizeof(cplx<T>)) < 128;
   const int nt = int(gridDim.x), b = int(blockIdx.x);
-  const int tile = nt % 8 == 0 ? (b % 8) * (nt / 8) + b / 8 : b;
-  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data)) + col_element(tl, X, tile * C + cl);
-  TwRegs<T, N, R> twr;
-  load_twiddles<T, N, R>(twr, tc, tw);
+  const int tile = kShared && nt % 8 == 0 ? (b % 8) * (nt / 8) + b / 8 : b;
+  const gptr<cplx<T>> W = gmem(reinterpret_cast<cplx<T>*>(data));
+  const int col = tile * C + cl;
+  const unsigned boff = (unsigned(tl) * unsigned(X) + unsigned(col)) * unsigned(sizeof(cplx<T>));
+  const auto element = [&](int j) {
+    if constexpr (FAR)
+      return W + col_element(tl + j * TT, X, col);
+    else
+      return at_off(W + col_element(j * TT, X, 0), boff);
+  };
+  const auto twsrc = fft_twiddles<!WIDE, T, N, R>(tc, tw);
   cplx<T> v[R];
 #pragma unroll
-  for (int j = 0; j < R; ++j) v[j] = gload(W + col_element(j * TT, X, 0));
-  if constexpr (G::kWave) {
+  for (int j = 0; j < R; ++j) v[j] = gload(element(j));
+  if constexpr (G::kWaveCols) {
     const LdsRow<T> view_l{lds + cl * LSZ}, view_c{lds + cc * LSZ};
-    team_fft_remap<T, N, R, DIR>(v, tl, view_l, tc, view_c, twr);
+    team_fft_remap<T, N, R, DIR>(v, tl, view_l, tc, view_c, twsrc);
     WaveSync::sync();
 #pragma unroll
     for (int j = 0; j < R; ++j) *view_c.ptr(padr<R>(tc + j * TT)) = v[j];
@@ -307,35 +343,63 @@ __global__ void __launch_bounds__((FftShape<T, N>::C * FftShape<T, N>::TT))
 #pragma unroll
     for (int j = 0; j < R; ++j) v[j] = *view_l.ptr(padr<R>(tl + j * TT));
   } else {
-    team_fft<T, N, R, DIR, LdsStrided<T, C>, BlockSync>(v, tl, LdsStrided<T, C>{lds + cl}, twr);
+    team_fft<T, N, R, DIR, LdsStrided<T, C>, BlockSync>(v, tl, LdsStrided<T, C>{lds + cl}, twsrc);
   }
   const T f = normalize ? T(1.0 / N) : T(1);
 #pragma unroll
-  for (int j = 0; j < R; ++j) store_cached(W + col_element(j * TT, X, 0), cscale(v[j], f));
+  for (int j = 0; j < R; ++j) store_cached(element(j), cscale(v[j], f));
 }
 
 // ------------------------------------------------------------------ launchers
 namespace {
 constexpr int kR = 16;
+constexpr size_t kLargeBatch = size_t(512) << 20;  // bytes: twice the last-level cache
 // columns a plan's batch has to be a multiple of (a multiple of every kernel's C)
 template <typename T, int N>
 constexpr int fft_cols_per_block() {
-  constexpr int c = 256 / (N / kR);
-  static_assert((c > 64 ? 64 : c) % FftShape<T, N>::C == 0, "whole tiles");
-  return c < 1 ? 1 : (c > 64 ? 64 : c);
+  constexpr int c = 256 / (N / kR), cols = c < 1 ? 1 : (c > 64 ? 64 : c);
+  static_assert(cols % FftShape<T, N, false>::C == 0 && cols % FftShape<T, N, true>::C == 0, "whole tiles");
+  return cols;
 }
+template <typename T, int N, bool WIDE, int DIR>
+hipError_t fft_rows_form(void* d, int rows, int norm, Twiddles<T> tw, hipStream_t s) {
+  using G = FftShape<T, N, WIDE>;
+  hipLaunchKernelGGL((fft_rows_kernel<T, N, WIDE, DIR>), dim3((rows + G::ROWS - 1) / G::ROWS), dim3(G::ROWS * G::TT), 0,
+                     s, d, rows, norm, tw);
+  return hipGetLastError();
+}
+// Wide rows: complex64 of 128..512 from a wide block per CU on (us, narrow -> wide: 512 x 4096 11.1 -> 8.6,
+// 512 x 32768 64.3 -> 43.2, 256 x 32768 24.8 -> 22.5, 128 x 32768 11.5 -> 9.7), every type and length
+// from 512 MiB on, twice the last-level cache (complex128 2048 x 65536 807 -> 728, 512 x 262144 767 -> 727,
+// 256 x 262144 398 -> 373; below that the narrow form: 512 x 32768 63.0 and 71.2).
 template <typename T, int N, int DIR>
 hipError_t fft_rows_n(void* d, int rows, int norm, Twiddles<T> tw, hipStream_t s) {
-  using G = FftShape<T, N>;
-  hipLaunchKernelGGL((fft_rows_kernel<T, N, DIR>), dim3((rows + G::ROWS - 1) / G::ROWS), dim3(G::ROWS * G::TT), 0, s,
-                     d, rows, norm, tw);
+  const bool many = sizeof(T) == 4 && N >= 128 && N <= 512 && rows / FftShape<T, N, true>::ROWS >= kCUs;
+  const bool large = size_t(rows) * N * sizeof(cplx<T>) >= kLargeBatch;
+  return many || large ? fft_rows_form<T, N, true, DIR>(d, rows, norm, tw, s)
+                       : fft_rows_form<T, N, false, DIR>(d, rows, norm, tw, s);
+}
+template <typename T, int N, bool WIDE, bool FAR, int DIR>
+hipError_t fft_cols_form(void* d, int X, int norm, Twiddles<T> tw, hipStream_t s) {
+  using G = FftShape<T, N, WIDE>;
+  hipLaunchKernelGGL((fft_cols_kernel<T, N, WIDE, FAR, DIR>), dim3(X / G::C), dim3(G::C * G::TT), 0, s, d, X, norm, tw);
   return hipGetLastError();
 }
+// Wide columns up to N = 512 from a wide block per CU on (us, narrow -> wide: complex64 128 x 32768
+// 15.2 -> 10.2, 256 x 8192 10.5 -> 7.6, 512 x 4096 13.4 -> 8.0; complex128 512 x 4096 12.3 -> 10.1,
+// 256 x 262144 579 -> 414; below that 256 x 2048 4.9 -> 5.1).  Complex128 of 64, whose narrow rows of 8
+// columns are whole lines, only from 512 MiB on (64 x 32768 8.1 -> 10.9, 64 x 524288 225 -> 196).  At 1024
+// and 2048 a narrow block has as many columns.
 template <typename T, int N, int DIR>
 hipError_t fft_cols_n(void* d, int X, int norm, Twiddles<T> tw, hipStream_t s) {
-  using G = FftShape<T, N>;
-  hipLaunchKernelGGL((fft_cols_kernel<T, N, DIR>), dim3(X / G::C), dim3(G::C * G::TT), 0, s, d, X, norm, tw);
-  return hipGetLastError();
+  if (!offsets_fit_32(FftShape<T, N, (N <= 512)>::TT, X, sizeof(cplx<T>)))  // 64 GiB and more
+    return fft_cols_form<T, N, (N <= 512), true, DIR>(d, X, norm, tw, s);
+  if constexpr (N <= 512) {
+    const bool many = (sizeof(T) == 4 || N >= 128) && X / FftShape<T, N, true>::C >= kCUs;
+    const bool large = size_t(X) * N * sizeof(cplx<T>) >= kLargeBatch;
+    if (many || large) return fft_cols_form<T, N, true, false, DIR>(d, X, norm, tw, s);
+  }
+  return fft_cols_form<T, N, false, false, DIR>(d, X, norm, tw, s);
 }
 #define WH_FFT_SWITCH(N, CALL)         \
   switch (N) {                         \

@@ -28,16 +28,32 @@ def test_column_element_indices(tmp_path):
     assert got == [r * X + c for r, X, c in PLACES]
 
 
+def test_where_byte_offsets_fit_32_bits(tmp_path):
+    cxx = shutil.which("g++")
+    if cxx is None:
+        pytest.skip("needs g++")
+    cases = [(rows, X, size) for rows in (4, 8, 32, 64, 128) for size in (8, 16)
+             for X in (64, 2 ** 32 // (rows * size) - 1, 2 ** 32 // (rows * size), 2 ** 32 // (rows * size) + 1, 2 ** 31 - 64)]
+    src, exe = tmp_path / "fit.cpp", tmp_path / "fit"
+    src.write_text('#include "wh_index.hpp"\n#include <cstdio>\nint main() {\n' + "".join(
+        f'  std::printf("%d\\n", int(wh::offsets_fit_32({r}, {X}, {s})));\n' for r, X, s in cases) + "}\n")
+    subprocess.run([cxx, "-std=c++17", f"-I{CSRC}", str(src), "-o", str(exe)], check=True)
+    got = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split()
+    # the largest offset is that of the last element of row rows - 1
+    assert got == [str(int((r * X - 1) * s < 2 ** 32)) for r, X, s in cases]
+
+
 @pytest.mark.gpu
-def test_columns_beyond_four_gigabytes_per_team(cuda):
-    """64 x 38404096 complex128 (39 GB): the offset of lane row 7 passes 2^32 bytes."""
+@pytest.mark.parametrize("n,X", [(64, 38404096), (1024, 4325376)])
+def test_columns_beyond_four_gigabytes_per_team(cuda, n, X):
+    """complex128: the byte offset of the last of eight lane rows (39 GB), and of the last of the 64 lane
+    rows of length 1024 (71 GB, the kernels with 64-bit offsets), passes 2^32."""
     import torch
 
     from pywignercuda_amd import cufft_wrapper as cw
 
-    n, X = 64, 38404096
-    if torch.cuda.mem_get_info()[0] < 60 << 30:
-        pytest.skip("needs 60 GB of free device memory")
+    if torch.cuda.mem_get_info()[0] < (n * X * 16 >> 30) + 20 << 30:
+        pytest.skip("needs that much free device memory")
     cols = [0, 1, 63, 55960, X // 2, X - 65, X - 1]
     W = torch.zeros((n, X), dtype=torch.complex128, device=cuda)
     try:
@@ -49,8 +65,8 @@ def test_columns_beyond_four_gigabytes_per_team(cuda):
         cw.fft_Z2Z(W, W, plan)
         ref = np.fft.fft(a.numpy(), axis=0)
         got = np.stack([W[:, c].cpu().numpy() for c in cols], axis=1)
-        # one transform's rounding: eps log2(n) relative to the largest element
-        assert np.abs(got - ref).max() <= 2.3e-16 * 6 * 4 * np.abs(ref).max()
+        # one transform's rounding: eps log2(n) on each side, relative to the largest element
+        assert np.abs(got - ref).max() <= 2.3e-16 * np.log2(n) * 4 * np.abs(ref).max()
         for c in cols:
             W[:, c] = 0
         for row in W:  # (row by row: no second array of this size)
