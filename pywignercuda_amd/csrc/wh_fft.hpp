@@ -131,21 +131,32 @@ constexpr double cos16(int k) {
   return t[k & 15];
 }
 
+constexpr double kHalfRootLow = -4.8336466567264565186e-17;  // sqrt(1/2) less the double next to it
+
 // a * (c + i s) with constants known at compile time; FP32 adds the products
 // with the low parts of the constants.
+// EXACT (FP64, odd multiples of pi/4): with the low part of sqrt(1/2).  Its rounding scales half of a
+// radix-8 butterfly's terms by 1 - 7e-17 in every pass and both directions, a fixed perturbation that
+// adds up over the steps: <p^2> after 72 steps at P = 1024 is 8.7e-13 off with it (radix 16: 1.7e-13).
 template <typename T>
 struct ConstMul;
 template <>
 struct ConstMul<double> {
-  template <int K, int DIR>
+  template <int K, int DIR, bool EXACT>
   __device__ __forceinline__ static cplx<double> mul(cplx<double> a) {
     constexpr double C = cos16(K), S = (DIR < 0 ? -1.0 : 1.0) * cos16(K + 12);
+    if constexpr (EXACT && K % 4 == 2) {  // C (1 +- i), the low part added before the one rounding
+      constexpr double lo = C > 0.0 ? kHalfRootLow : -kHalfRootLow;
+      const double d = (S > 0.0) == (C > 0.0) ? a.x - a.y : a.x + a.y;
+      const double e = (S > 0.0) == (C > 0.0) ? a.x + a.y : a.y - a.x;
+      return {fma(d, C, d * lo), fma(e, C, e * lo)};
+    }
     return {a.x * C - a.y * S, a.x * S + a.y * C};
   }
 };
 template <>
 struct ConstMul<float> {
-  template <int K, int DIR>
+  template <int K, int DIR, bool EXACT>
   __device__ __forceinline__ static cplx<float> mul(cplx<float> a) {
     constexpr double C = cos16(K), S = (DIR < 0 ? -1.0 : 1.0) * cos16(K + 12);
     constexpr float ch = float(C), sh = float(S);
@@ -156,7 +167,7 @@ struct ConstMul<float> {
 };
 
 // a * exp(DIR * 2*pi*i * K / M), M | 16; the special angles are exact.
-template <int DIR, int K, int M, typename T>
+template <int DIR, int K, int M, bool EXACT, typename T>
 __device__ __forceinline__ cplx<T> rot(cplx<T> a) {
   constexpr int k = ((K % M) * (16 / M)) & 15;
   if constexpr (k == 0) {
@@ -168,37 +179,37 @@ __device__ __forceinline__ cplx<T> rot(cplx<T> a) {
   } else if constexpr (k == 4 || k == 12) {
     return {-a.y, a.x};  // * (+i)
   } else {
-    return ConstMul<T>::template mul<k, DIR>(a);
+    return ConstMul<T>::template mul<k, DIR, EXACT>(a);
   }
 }
 
 // Radix-2 decimation-in-frequency butterflies of one stage of length L at offset OFF.
-template <int DIR, int L, int OFF, int I, typename T>
+template <int DIR, int L, int OFF, int I, bool EXACT, typename T>
 struct DifStage {
   __device__ __forceinline__ static void run(cplx<T>* v) {
     if constexpr (I < L / 2) {
       cplx<T> a = v[OFF + I], b = v[OFF + I + L / 2];
       v[OFF + I] = cadd(a, b);
-      v[OFF + I + L / 2] = rot<DIR, I, L>(csub(a, b));
-      DifStage<DIR, L, OFF, I + 1, T>::run(v);
+      v[OFF + I + L / 2] = rot<DIR, I, L, EXACT>(csub(a, b));
+      DifStage<DIR, L, OFF, I + 1, EXACT, T>::run(v);
     }
   }
 };
-template <int DIR, int L, int OFF, typename T>
+template <int DIR, int L, int OFF, bool EXACT, typename T>
 struct Dif {
   __device__ __forceinline__ static void run(cplx<T>* v) {
     if constexpr (L > 1) {
-      DifStage<DIR, L, OFF, 0, T>::run(v);
-      Dif<DIR, L / 2, OFF, T>::run(v);
-      Dif<DIR, L / 2, OFF + L / 2, T>::run(v);
+      DifStage<DIR, L, OFF, 0, EXACT, T>::run(v);
+      Dif<DIR, L / 2, OFF, EXACT, T>::run(v);
+      Dif<DIR, L / 2, OFF + L / 2, EXACT, T>::run(v);
     }
   }
 };
 
 // In-register r-point DFT:  y_q = sum_j x_j exp(DIR*2*pi*i*j*q/r), r | 16.
-template <int DIR, int r, typename T>
+template <int DIR, int r, bool EXACT, typename T>
 __device__ __forceinline__ void dft(cplx<T>* x) {
-  Dif<DIR, r, 0, T>::run(x);
+  Dif<DIR, r, 0, EXACT, T>::run(x);
   cplx<T> y[r];
 #pragma unroll
   for (int q = 0; q < r; ++q) y[q] = x[bitrev(q, ilog2(r))];
@@ -321,6 +332,7 @@ template <typename T, int N, int R>
 struct TwRegs;
 template <int N, int R>
 struct TwRegs<double, N, R> {
+  static constexpr bool kExact = false;
   cplx<double> hi[TwSlots<N, R>::count];
   template <int DIR>
   __device__ __forceinline__ cplx<double> mul(cplx<double> x, int slot, int) const {
@@ -330,6 +342,7 @@ struct TwRegs<double, N, R> {
 };
 template <int N, int R>
 struct TwRegs<float, N, R> {
+  static constexpr bool kExact = false;
   cplx<float> hi[TwSlots<N, R>::count], lo[TwSlots<N, R>::count];
   template <int DIR>
   __device__ __forceinline__ cplx<float> mul(cplx<float> x, int slot, int) const {
@@ -341,9 +354,11 @@ struct TwRegs<float, N, R> {
   }
 };
 
-// Table-backed source with the same interface (twiddle index idx, slot unused).
-template <typename T>
+// Table-backed source with the same interface (twiddle index idx, slot unused).  EXACT: transforms with
+// it take the low part of sqrt(1/2) (ConstMul).
+template <typename T, bool EXACT = false>
 struct TwMem {
+  static constexpr bool kExact = EXACT;
   Twiddles<T> tw;
   template <int DIR>
   __device__ __forceinline__ cplx<T> mul(cplx<T> x, int, int idx) const {
@@ -444,9 +459,9 @@ struct PassIO {
       static_for<1, r>([&](auto J) {
         constexpr int j = decltype(J)::value;
         x[j] = tw.template mul<DIR>(x[j], TwSlots<N, R>::off(P) + j - 1, (j * tstep) & (N - 1));
-        x[j] = rot<DIR, (j * mm) % R, R>(x[j]);
+        x[j] = rot<DIR, (j * mm) % R, R, Tw::kExact>(x[j]);
       });
-      dft<DIR, r>(x);
+      dft<DIR, r, Tw::kExact>(x);
       if constexpr (P == NP - 1) {
         // last pass: outputs land on t + TT*(mm + q*nb) -> strided register layout
 #pragma unroll
@@ -481,9 +496,9 @@ struct PassIO {
       static_for<1, r>([&](auto J) {
         constexpr int j = decltype(J)::value;
         x[j] = tw.template mul<DIR>(x[j], TwSlots<N, R>::off(P) + j - 1, (j * tl) & (N - 1));
-        x[j] = rot<DIR, (j * mm) % R, R>(x[j]);
+        x[j] = rot<DIR, (j * mm) % R, R, Tw::kExact>(x[j]);
       });
-      dft<DIR, r>(x);
+      dft<DIR, r, Tw::kExact>(x);
 #pragma unroll
       for (int q = 0; q < r; ++q) o[mm + q * nb] = x[q];
     });
@@ -559,7 +574,7 @@ struct TeamPass {
 template <typename T, int N, int R, int DIR, class Lds, class Sync = BlockSync, class Tw = TwMem<T>>
 __device__ __forceinline__ void team_fft(cplx<T> (&v)[R], int t, Lds lds, const Tw& tw) {
   static_assert(N % R == 0 && R <= 16 && (R & (R - 1)) == 0 && N >= R, "radix");
-  dft<DIR, R>(v);  // pass 0: butterfly b = t reads v[j] = a[t + j*TT], no twiddle
+  dft<DIR, R, Tw::kExact>(v);  // pass 0: butterfly b = t reads v[j] = a[t + j*TT], no twiddle
   TeamPass<T, N, R, DIR, 1, Sync, Lds, Tw>::run(v, t, lds, tw);
 }
 template <typename T, int N, int R, int DIR, class Lds>
@@ -574,7 +589,7 @@ __device__ __forceinline__ void team_fft(cplx<T> (&v)[R], int t, Lds lds, Twiddl
 template <typename T, int N, int R, int DIR, class Lds, class Tw>
 __device__ __forceinline__ void team_fft_remap(cplx<T> (&v)[R], int tl, Lds lw, int tc, Lds lc, const Tw& tw) {
   static_assert(num_passes(N, R) >= 2, "the remap happens at the first exchange");
-  dft<DIR, R>(v);
+  dft<DIR, R, Tw::kExact>(v);
   PassIO<T, N, R, 1>::write(v, opaque_v(tl), lw);
   __syncthreads();
   const int t = opaque_v(tc);

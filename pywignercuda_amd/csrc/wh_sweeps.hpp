@@ -666,6 +666,8 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
   // radix-8 lanes have the registers to keep the multipliers over the first transform (radix-16
   // lanes spill: -13% on 32 grids of 1024^2)
   constexpr bool kEarly = R <= 8 && !TP;
+  // complex128 columns that radix 8 takes from radix 16 (plans of few cells)
+  constexpr bool kExact = sizeof(S) == 8 && R == 8 && N >= 1024;
   const bool early = kEarly && PS::early(a, m);
   typename PS::MulLoads ml;
   if (early) PS::mul_loads(ml, a, m, tc, col, step);
@@ -696,7 +698,7 @@ __device__ __forceinline__ void psweep_body(const SweepArgs& a, CMember& m, int 
       load_twiddles<T, N, R>(r, tc, tw);
       return r;
     } else {
-      return TwMem<T>{tw};
+      return TwMem<T, kExact>{tw};
     }
   }();
   cplx<double> M[R];

@@ -61,13 +61,13 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
     batch: the plan holds enough cells to fill the GPU (the tuner's "batch" regime).
 
     The tuner times square grids.  A plan of a long side and few cells wants more lanes per
-    transform: up to 2^19 cells radix 16 leaves half of the chip's 1024 SIMDs without a wave.  In x
-    that is radix 4 at 1024 and 8 at 2048 (us per step, complex128: 1024 x 256 19.0 -> 17.5,
-    2048 x 128 21.2 -> 18.8; at 1024^2 radix 16 wins), in p radix 8 for complex64 states.  Complex128
-    states keep radix 16 in p at 1024 and 2048, where radix 8 is faster (1024 x 128 17.6 -> 14.1,
-    2048 x 128 22.9 -> 19.8, with friction 46.2 -> 36.2) but further from the exact steps: its twiddle
-    roundings leave a fixed residue at the edges of p, which <p^2> weighs most (72 steps against 80-bit
-    ones, largest relative error, radix 16 -> 8: 1024 1.7e-13 -> 8.7e-13, 2048 3.8e-13 -> 9.0e-13).
+    transform: up to 2^19 cells radix 16 leaves half of the chip's 1024 SIMDs without a wave
+    (us per step, complex128, radix 16 -> 8 in p, or in x -> 4 at 1024 and 8 at 2048: 256 x 1024
+    20.3 -> 17.3, with friction 32.7 -> 27.7, 128 x 2048 23.4 -> 20.3 and 46.7 -> 36.6, 1024 x 256
+    19.0 -> 17.5, 2048 x 128 21.2 -> 18.8; at 1024^2 radix 16 wins).  In p these radix-8 transforms
+    carry sqrt(1/2) with its low part and are then the more exact ones (<p^2> after 72 steps against
+    80-bit ones, radix 16 and 8: P = 1024 1.7e-13 and 3.2e-14, 2048 3.8e-13 and 9.0e-14; radix 8
+    without the low part 8.7e-13 and 9.0e-13).
     Complex128 states of 2^20 or 2^21 cells together, which the L2s hold, want radix 16 in x where a
     side is 512 or more (512 x 2048 39.7 -> 36.7, 2048 x 1024 51.6 -> 46.7, four grids of 512^2
     34.0 -> 28.4, eight 41.1 -> 41.4; beyond them 2048^2 93.9 with radix 8, 104.6 with 16).  Ensembles
@@ -92,8 +92,7 @@ def tuned_variants(precision: str, sizes_x, sizes_p, cl: bool, batch: bool = Fal
         if precision != "fp32fast" and npp in ("1024", "2048") and pcl >= 0:
             pcl = 2 if cells >= 1 << 21 else 0
         if cells <= 1 << 19:
-            if precision != "fp64":
-                pv, pcl = 2, 1  # radix 8
+            pv, pcl = 2, 1  # radix 8
             xv = {"1024": 3, "2048": 1}.get(nx, xv)  # radix 4, radix 8
         elif precision == "fp64" and cells <= 1 << 21 and int(nx) >= 512:
             xv = 0  # radix 16

@@ -30,16 +30,6 @@ def test_friction_form_by_cells(precision):
         assert choice(precision, X, P, True)[2] == 0, (P, X)
 
 
-@pytest.mark.parametrize("cl", [False, True])
-@pytest.mark.parametrize("P", [1024, 2048])
-def test_complex128_keeps_radix_16_in_long_columns(P, cl):
-    """Radix 8 leaves a larger residue in <p^2> there (see tuned_variants)."""
-    for X in (128, 256, 512, 1024, 2048):
-        for members in (1, 2, 16, 64):
-            _, pv, pcl = choice("fp64", X, P, cl, members)
-            assert radix(1, max(pv, 0)) == 16 and radix(2, max(pcl, 0)) == 16, (X, members)
-
-
 def test_small_sides_keep_their_radix_in_ensembles():
     """Radix 16 in x for 2^20 and 2^21 cells of complex128 is for sides of 512 and more."""
     for side, members in ((128, 64), (128, 128), (256, 16), (256, 32)):
