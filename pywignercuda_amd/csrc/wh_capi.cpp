@@ -44,7 +44,6 @@ hipError_t launch_reduce(const ReduceArgs& a, int nmembers, int* done, hipStream
 hipError_t launch_colpart_reduce(const Member* members, int nmembers, int max_x, int xradix, int xblock,
                                  hipStream_t s);
 hipError_t launch_scale(int prec, const Member* members, const unsigned* work, int nwork, hipStream_t s);
-hipError_t launch_set_int(int* p, int v, hipStream_t s);
 hipError_t launch_bind(const BindArgs& a, hipStream_t s);
 hipError_t launch_dirac_bind(DiracPlan* d, void* W, double* obs, int obs_base, int* step, int step_v, double* scale,
                              int reset_scale, hipStream_t s);
@@ -1053,9 +1052,9 @@ int run_graph(wh_ensemble* e, int count, hipStream_t s) {
   return iterations(e, count, true, false, s);
 }
 
-// Device member table: a structural change (creation, new potential rows, adjoint
-// operands) re-uploads the whole table and waits for the copy; a change of only the
-// states and record rows of a run is written by a bind kernel in stream order.
+// Device member table: a structural change (creation, new potential rows) re-uploads the whole
+// table and waits for the copy; a change of only the states and record rows of a run is written by
+// a bind kernel in stream order (steps and adjoint sweeps take their states as arguments).
 int sync_table(wh_ensemble* e, bool changed, hipStream_t s) {
   if (changed || e->table_dirty) {
     WH_HIP(hipMemcpyAsync(e->mem_dev.p, e->mem.data(), sizeof(wh::Member) * e->mem.size(), hipMemcpyHostToDevice, s),

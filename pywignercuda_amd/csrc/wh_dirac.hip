@@ -167,7 +167,8 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
     }
   }
   // (one transform's, or one bin's, temporaries at a time: interleaved, and with a last pass spread
-  // over both sides of the branch below, they spilled 104 VGPRs at N = 512)
+  // over both sides of the branch below, they spilled 104 VGPRs at N = 512.  The step filter's form
+  // still spills 12 to 36 in FP64 arithmetic from N = 256 on and 9 to 18 in FP32 from 512 on.)
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     pin(v[q]);

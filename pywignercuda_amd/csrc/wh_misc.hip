@@ -217,7 +217,6 @@ __global__ void __launch_bounds__(256) scale_kernel(const Member* members, const
   }
 }
 
-__global__ void set_int_kernel(int* p, int v) { *p = v; }
 __global__ void bind_kernel(BindArgs a) {
   const int i = threadIdx.x;
   if (i < a.count) {
@@ -473,10 +472,6 @@ hipError_t launch_scale(int prec, const Member* members, const unsigned* work, i
     hipLaunchKernelGGL(scale_kernel<double>, dim3(nwork), dim3(256), 0, s, members, work);
   else
     hipLaunchKernelGGL(scale_kernel<float>, dim3(nwork), dim3(256), 0, s, members, work);
-  return hipGetLastError();
-}
-hipError_t launch_set_int(int* p, int v, hipStream_t s) {
-  hipLaunchKernelGGL(set_int_kernel, dim3(1), dim3(1), 0, s, p, v);
   return hipGetLastError();
 }
 hipError_t launch_bind(const BindArgs& a, hipStream_t s) {

@@ -287,8 +287,8 @@ __device__ __forceinline__ void odm_back_body(const SweepArgs& a, CMember& m, in
   for (int j = 0; j < R; ++j) put(W + j * TT, to_arith<S>(w0[j]));
 }
 
-// KIND: kOdmX, kOdmP, kOdmBack, kOdmJoin.  With kTileScale a kOdmX launch has the members' record
-// items at the end of its list (the partials are the last join's).
+// KIND: kOdmX, kOdmP, kOdmBack, kOdmJoin.  The list of kOdmX ends with the members' record items; a launch
+// that is not to record (no join's partials are there yet, or another channel's did) is cut before them.
 template <typename S, typename T, int KIND>
 __global__ void __launch_bounds__(kOdmBlock) odm_kernel(SweepArgs a, double weight, double sgn) {
   __shared__ cplx<T> lds[lds_elems<kOdmBlock, kOdmR>() + kTileRedBytes / sizeof(cplx<T>)];

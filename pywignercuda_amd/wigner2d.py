@@ -301,7 +301,7 @@ class _PlanBase:
         else:
             xv, pv, pcl = tuned_variants(self.precision, sizes_x, sizes_p, self.cl, batch)
             if self.gp:
-                xv = -1  # the x variant of a Gross-Pitaevskii plan is fixed at creation
+                xv = -1  # a Gross-Pitaevskii plan has chosen its x variant at creation
         if (xv, pv, pcl) != (-1, -1, -1):
             rc = _lib.lib().wh_ensemble_set_variants(ens_handle, xv, pv, pcl)
             if rc != 0:
