@@ -328,11 +328,12 @@ struct TwSlots {
   static constexpr int count = off(NP) > 0 ? off(NP) : 1;
 };
 
-template <typename T, int N, int R>
+// EXACT: transforms with them take the low part of sqrt(1/2) (ConstMul).
+template <typename T, int N, int R, bool EXACT = false>
 struct TwRegs;
-template <int N, int R>
-struct TwRegs<double, N, R> {
-  static constexpr bool kExact = false;
+template <int N, int R, bool EXACT>
+struct TwRegs<double, N, R, EXACT> {
+  static constexpr bool kExact = EXACT;
   cplx<double> hi[TwSlots<N, R>::count];
   template <int DIR>
   __device__ __forceinline__ cplx<double> mul(cplx<double> x, int slot, int) const {
@@ -340,9 +341,9 @@ struct TwRegs<double, N, R> {
   }
   __device__ __forceinline__ void set(int slot, const Twiddles<double>& tw, int idx) { hi[slot] = gload(gmem(tw.hi) + idx); }
 };
-template <int N, int R>
-struct TwRegs<float, N, R> {
-  static constexpr bool kExact = false;
+template <int N, int R, bool EXACT>
+struct TwRegs<float, N, R, EXACT> {
+  static constexpr bool kExact = EXACT;
   cplx<float> hi[TwSlots<N, R>::count], lo[TwSlots<N, R>::count];
   template <int DIR>
   __device__ __forceinline__ cplx<float> mul(cplx<float> x, int slot, int) const {
@@ -354,8 +355,7 @@ struct TwRegs<float, N, R> {
   }
 };
 
-// Table-backed source with the same interface (twiddle index idx, slot unused).  EXACT: transforms with
-// it take the low part of sqrt(1/2) (ConstMul).
+// Table-backed source with the same interface (twiddle index idx, slot unused).
 template <typename T, bool EXACT = false>
 struct TwMem {
   static constexpr bool kExact = EXACT;
@@ -367,8 +367,8 @@ struct TwMem {
 };
 
 // Fills the registers of team index t from the table.
-template <typename T, int N, int R, int P = 1>
-__device__ __forceinline__ void load_twiddles(TwRegs<T, N, R>& w, int t, const Twiddles<T>& tw) {
+template <typename T, int N, int R, int P = 1, bool EXACT = false>
+__device__ __forceinline__ void load_twiddles(TwRegs<T, N, R, EXACT>& w, int t, const Twiddles<T>& tw) {
   if constexpr (P < num_passes(N, R)) {
     constexpr int r = pass_radix(N, R, P), Ns = ipow(R, P);
     const int tstep = (t % Ns) * (N / (Ns * r));

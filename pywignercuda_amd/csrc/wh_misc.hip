@@ -241,6 +241,9 @@ __global__ void set_scale_kernel(const Member* members, double re, double im) {
 // A forward and an inverse pair over both axes with two clones, us, against radix 16, block barriers and
 // 256 lanes a block for every length: 2048^2 complex128 239 -> 147, complex64 205 -> 119; 1024^2
 // 65 -> 60 and 64 -> 44; 512 x 1024 47 -> 38; below, the calls' host time (38 us) covers the kernels.
+// Complex128 radix-8 teams carry sqrt(1/2) with its low part (ConstMul): <q^2> of a Gaussian after 72
+// forward and inverse transforms of 128..512 is 6e-16 to 4e-15 off, without it 8e-14 to 1.3e-13, with
+// radix 16 6e-15 to 1.7e-14; at most 0.2 us a call.
 // Wide form (large batches, the rules are in fft_rows_n and fft_cols_n): radix 16 in blocks of 256 lanes.
 // Its rows of columns are whole 128-byte lines (64 bytes at complex64 512) and it exchanges once less; a
 // narrow block's rows of 4 columns are 32 or 64 bytes, too short once the batch is beyond the L2s.
@@ -258,7 +261,7 @@ struct FftShape {
 template <bool REGS, typename T, int N, int R>
 __device__ __forceinline__ auto fft_twiddles(int t, const Twiddles<T>& tw) {
   if constexpr (REGS) {
-    TwRegs<T, N, R> r;
+    TwRegs<T, N, R, sizeof(T) == 8 && R == 8> r;
     load_twiddles<T, N, R>(r, t, tw);
     return r;
   } else {
