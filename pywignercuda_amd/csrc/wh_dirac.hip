@@ -66,6 +66,10 @@ __device__ __forceinline__ cplx<T> narrow(cplx<double> v) { return {T(v.x), T(v.
 // takes 22 us); whole steps 115 -> 88 us, at 1024^2 553 -> 430, 2048 x 512 525 -> 347 and with the
 // step filter at 512^2 229 -> 142 us.  At 2048 four groups would be 1024 lanes of 128 registers
 // each: one group per block there.
+// Complex128 states carry sqrt(1/2) with its low part (ConstMul), in this sweep and in the p sweep: W
+// against 80-bit steps, 40 steps at 128^2, 20 at 256^2 and 10 at 512^2, is 4.2e-15, 2.6e-15 and 1.6e-15
+// off, without it 9.0e-15, 5.2e-15 and 3.3e-15; it costs up to 2.6% (256^2 with friction 55.4 -> 56.8 us
+// a step, 512^2 63.4 -> 64.1).
 template <int N>
 struct DiracX {
   static constexpr int R = 8, TT = N / R;
@@ -134,7 +138,7 @@ __device__ __forceinline__ void dirac_xsweep_body(const DiracPlan& d, int block,
     const int r = (q >> 1) ? 3 - gr : gr, c = (q & 1) ? 3 - gc : gc;
     return 4 * r + c;
   };
-  TwRegs<T, N, R> twr;
+  TwRegs<T, N, R, sizeof(S) == 8> twr;
   load_twiddles<T, N, R>(twr, t, tw);
   cplx<T> v[4][R];
   // 32-bit byte offsets (16 planes of 2048^2 complex128 are 1 GiB), recomputed from an opaque
@@ -570,7 +574,7 @@ __device__ __forceinline__ void dirac_psweep_body(const DiracPlan& d, int tile, 
       tab[N + i] = T(gmem(d.theta_host)[i] * (1.0 / N));
     }
   }
-  TwRegs<T, N, R> twr;
+  TwRegs<T, N, R, sizeof(S) == 8> twr;
   load_twiddles<T, N, R>(twr, tc, tw);
 
   const unsigned jstride = unsigned(TT) * unsigned(X) * unsigned(sizeof(cplx<S>));
